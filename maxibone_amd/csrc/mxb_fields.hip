@@ -310,176 +310,6 @@ __global__ __launch_bounds__(kRowThreads) void k_field_histogram(const uint16_t 
     }
 }
 
-struct AxisHistArgs {
-    int64_t nz, ny, nx, z_offset, Nz, Nr, vb;
-    const int32_t *vlut;  // per uint16 value: bin or -1
-    int64_t cy, cx;
-};
-
-__device__ __forceinline__ int64_t isqrt64(int64_t s) {
-    int64_t r = (int64_t)sqrt((double)s);
-    while (r * r > s) --r;
-    while ((r + 1) * (r + 1) <= s) ++r;
-    return r;
-}
-
-// Axis histograms, y and z bins.  A block walks whole rows (grid-stride); the
-// voxels of a row share y and z, so their bin counts gather in LDS (one
-// histogram for the row's y, one for the current z plane) and reach y_bins /
-// z_bins as one atomic per nonzero bin: at the end of each row for y, when
-// the plane changes (rows of a block come in increasing order) for z.  x and
-// r vary along the row; k_axis_xr counts them.  LDS: 2 x vb uint32.
-__global__ __launch_bounds__(kRowThreads) void k_axis_histograms(const uint16_t *__restrict__ vox,
-                                                                 RowWalk w, AxisHistArgs a, int vec,
-                                                                 unsigned long long *__restrict__ yb,
-                                                                 unsigned long long *__restrict__ zb) {
-    extern __shared__ uint32_t hist[];  // [0, vb): row (y); [vb, 2 vb): plane (z)
-    uint32_t *hy = hist, *hz = hist + a.vb;
-    for (int64_t i = threadIdx.x; i < 2 * a.vb; i += kRowThreads) hist[i] = 0;
-    __syncthreads();
-    int64_t zcur = -1;  // plane whose counts hz holds (uniform)
-    auto flush = [&](uint32_t *h, unsigned long long *dst) {
-        for (int64_t i = threadIdx.x; i < a.vb; i += kRowThreads) {
-            const uint32_t c = h[i];
-            if (c != 0) {
-                atomicAdd(&dst[i], (unsigned long long)c);
-                h[i] = 0;
-            }
-        }
-    };
-    for (int64_t row = blockIdx.x; row < w.rows; row += gridDim.x) {
-        const int64_t y = row % a.ny, z = row / a.ny + a.z_offset;
-        if (z >= a.Nz) break;  // rows come in increasing order: the rest lie beyond Nz too
-        if (z != zcur) {
-            if (zcur >= 0) {
-                __syncthreads();
-                flush(hz, zb + zcur * a.vb);
-                __syncthreads();
-            }
-            zcur = z;
-        }
-        for (int64_t x0 = (int64_t)threadIdx.x * kPerThread; x0 < w.nx; x0 += kRowChunk) {
-            uint16_t v[8];
-            load8(vox + row * w.nx, x0, w.nx, vec != 0, v);
-#pragma unroll
-            for (int k = 0; k < 8; ++k) {
-                const int64_t x = x0 + k;
-                if (x >= w.nx) break;
-                const int32_t vi = a.vlut[v[k]];
-                if (vi < 0) continue;
-                atomicAdd(&hy[vi], 1u);
-                atomicAdd(&hz[vi], 1u);
-            }
-        }
-        __syncthreads();
-        flush(hy, yb + y * a.vb);
-        __syncthreads();
-    }
-    if (zcur >= 0) {
-        __syncthreads();
-        flush(hz, zb + zcur * a.vb);
-    }
-}
-
-// Lanes of a wave that hold the same key (among those with `valid`) are
-// combined: returns true on one lane per distinct key, with `count` the
-// number of lanes that hold it.  After kMaxGroups keys the remaining lanes
-// return true with count 1 (bounded work when the keys are mostly distinct:
-// on noisy CT data 0-4 groups cost the same, 16 cost 8 % more, 64 2.2x).
-// Call from wave-uniform control flow.
-constexpr int kMaxGroups = 4;
-__device__ __forceinline__ bool wave_group(uint32_t key, bool valid, uint32_t &count) {
-    const int lane = (int)__lane_id();
-    uint64_t pending = __ballot(valid);
-    bool leader = false;
-    count = 0;
-    for (int it = 0; it < kMaxGroups && pending != 0; ++it) {
-        const int l = __ffsll((unsigned long long)pending) - 1;
-        const uint32_t k = (uint32_t)__shfl((int)key, l);
-        const uint64_t same = __ballot(valid && key == k) & pending;
-        if (lane == l) {
-            leader = true;
-            count = (uint32_t)__popcll(same);
-        }
-        pending &= ~same;
-    }
-    if ((pending >> lane) & 1ull) {
-        leader = true;
-        count = 1;
-    }
-    return leader;
-}
-
-// Axis histograms, x and r bins.  Counted along rows, the lanes would hold
-// different x, so each voxel cost one global atomic for x and one for r
-// (45-52 ms each on 1024^3 with 4096 bins).  Here a block takes COLS columns
-// x0 .. x0+COLS-1 and kXrThreads consecutive z (one per lane) and walks y:
-// the lanes of a wave then share x, y and therefore r, and differ only in the
-// voxel bin.  x counts gather in LDS (COLS x vb uint32, at most kXrLds
-// bytes: 8 columns up to 4096 bins, 4 up to 8192) and reach x_bins once per
-// block; r counts are combined over the wave (one atomic per distinct voxel
-// bin) and added to r_bins.
-constexpr int kXrThreads = 256;
-constexpr int64_t kXrLds = 128 * 1024;
-
-// COLS (4 or 8) consecutive uint16 of a row starting at x0 (past nx read 0).
-template <int COLS>
-__device__ __forceinline__ void load_cols(const uint16_t *__restrict__ row, int64_t x0, int64_t nx, bool vec,
-                                          uint16_t v[8]) {
-    if constexpr (COLS == 8) {
-        load8(row, x0, nx, vec, v);
-    } else if (vec && x0 + 4 <= nx) {
-        const uint2 q = *reinterpret_cast<const uint2 *>(row + x0);
-        const uint32_t w[2] = {q.x, q.y};
-#pragma unroll
-        for (int k = 0; k < 4; ++k) v[k] = (uint16_t)(w[k >> 1] >> (16 * (k & 1)));
-    } else {
-#pragma unroll
-        for (int k = 0; k < 4; ++k) v[k] = x0 + k < nx ? row[x0 + k] : (uint16_t)0;
-    }
-}
-
-template <int COLS>
-__global__ __launch_bounds__(kXrThreads) void k_axis_xr(const uint16_t *__restrict__ vox, AxisHistArgs a,
-                                                        int vec, unsigned long long *__restrict__ xb,
-                                                        unsigned long long *__restrict__ rb) {
-    constexpr int kXrCols = COLS;
-    extern __shared__ uint32_t hx[];  // [COLS][vb]
-    for (int64_t i = threadIdx.x; i < kXrCols * a.vb; i += kXrThreads) hx[i] = 0;
-    __syncthreads();
-    const int64_t ncol = (a.nx + kXrCols - 1) / kXrCols;
-    const int64_t x0 = (blockIdx.x % ncol) * kXrCols;
-    const int64_t z = (blockIdx.x / ncol) * kXrThreads + threadIdx.x;
-    const bool zok = z < a.nz && z + a.z_offset < a.Nz;
-    const uint16_t *base = vox + (zok ? z : 0) * a.ny * a.nx;
-    uint16_t cur[8] = {0, 0, 0, 0, 0, 0, 0, 0}, nxt[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-    if (zok && a.ny > 0) load_cols<COLS>(base, x0, a.nx, vec != 0, cur);
-    for (int64_t y = 0; y < a.ny; ++y) {
-        if (zok && y + 1 < a.ny) load_cols<COLS>(base + (y + 1) * a.nx, x0, a.nx, vec != 0, nxt);
-        const int64_t dy2 = (y - a.cy) * (y - a.cy);
-#pragma unroll
-        for (int k = 0; k < kXrCols; ++k) {
-            const int64_t x = x0 + k;
-            if (x >= a.nx) break;  // uniform
-            const int32_t vi = a.vlut[cur[k]];
-            uint32_t cnt;
-            if (wave_group((uint32_t)vi, zok && vi >= 0, cnt)) {
-                atomicAdd(&hx[k * a.vb + vi], cnt);
-                const int64_t r = isqrt64((x - a.cx) * (x - a.cx) + dy2);
-                if (r < a.Nr) atomicAdd(&rb[r * a.vb + vi], (unsigned long long)cnt);
-            }
-        }
-#pragma unroll
-        for (int k = 0; k < COLS; ++k) cur[k] = nxt[k];
-    }
-    __syncthreads();
-    for (int64_t i = threadIdx.x; i < kXrCols * a.vb; i += kXrThreads) {
-        const uint32_t c = hx[i];
-        const int64_t x = x0 + i / a.vb;
-        if (c != 0 && x < a.nx) atomicAdd(&xb[x * a.vb + i % a.vb], (unsigned long long)c);
-    }
-}
-
 // Host-side bin tables: histograms.cc:61-62 (:278-279) and :292.
 static void voxel_lut(double vmin, double vmax, int64_t vb, int32_t *lut) {
     for (int64_t i = 0; i < 65536; ++i) {
@@ -640,45 +470,20 @@ static int device_field_histogram(const uint16_t *vox, int64_t nZ, int64_t nY, i
 static int device_axis_histograms(const uint16_t *vox, int64_t nz, int64_t ny, int64_t nx,
                                   int64_t z_offset, uint64_t *xb, uint64_t *yb, uint64_t *zb,
                                   uint64_t *rb, int64_t Nz, int64_t Nr, int64_t vb, uint64_t cy,
-                                  uint64_t cx, double vmin, double vmax, void *ws, hipStream_t s) {
+                                  uint64_t cx, double vmin, double vmax, hipStream_t s) {
     if (nz * ny * nx == 0) return OK;
     if (vb < 1 || z_offset < 0 || Nz < 0 || Nr < 0) {
         set_error("axis_histograms: invalid arguments");
         return EINVAL_;
     }
-    // every argument check precedes the copy of the lookup table
     const RowWalk w = row_walk(nz * ny, nx);
     if (int rc = check_grid(w)) return rc;
     if (vb > 8192) {
         set_error("axis_histograms: at most 8192 voxel bins");
         return EINVAL_;
     }
-    const int cols = 8 * vb * 4 <= kXrLds ? 8 : 4;  // vb <= 8192: 4 columns fit
-    const int64_t blocks = ((nx + cols - 1) / cols) * ((nz + kXrThreads - 1) / kXrThreads);
-    if (blocks > 0x7fffffffLL) {
-        set_error("axis_histograms: volume too large for one launch");
-        return EINVAL_;
-    }
-    const int smem = (int)(cols * vb * 4);
-    const void *fn = cols == 8 ? reinterpret_cast<const void *>(&k_axis_xr<8>)
-                               : reinterpret_cast<const void *>(&k_axis_xr<4>);
-    MXB_FHIP(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, smem));
-    std::vector<int32_t> host(65536);
-    voxel_lut(vmin, vmax, vb, host.data());
-    int32_t *d = (int32_t *)ws;
-    MXB_FHIP(hipMemcpyAsync(d, host.data(), host.size() * 4, hipMemcpyHostToDevice, s));
-    AxisHistArgs a{nz, ny, nx, z_offset, Nz, Nr, vb, d, (int64_t)cy, (int64_t)cx};
-    const unsigned grid = (unsigned)std::min<int64_t>(w.rows, 4096);
-    hipLaunchKernelGGL(k_axis_histograms, dim3(grid), dim3(kRowThreads), (unsigned)(2 * vb * 4), s, vox, w, a,
-                       vec_ok(vox, nx), (unsigned long long *)yb, (unsigned long long *)zb);
-    MXB_FHIP_AFTER_COPY(hipGetLastError(), s);
-    if (cols == 8)
-        hipLaunchKernelGGL(k_axis_xr<8>, dim3((unsigned)blocks), dim3(kXrThreads), (unsigned)smem, s, vox, a,
-                           vec_ok(vox, nx), (unsigned long long *)xb, (unsigned long long *)rb);
-    else
-        hipLaunchKernelGGL(k_axis_xr<4>, dim3((unsigned)blocks), dim3(kXrThreads), (unsigned)smem, s, vox, a,
-                           vec_ok(vox, nx), (unsigned long long *)xb, (unsigned long long *)rb);
-    MXB_FHIP_AFTER_COPY(hipGetLastError(), s);
+    MXB_FHIP(launch_axis_histograms(vox, nz, ny, nx, z_offset, xb, yb, zb, rb, Nz, Nr, vb, (int64_t)cy, (int64_t)cx,
+                                    vmin, vmax, s));
     MXB_FHIP(hipStreamSynchronize(s));
     return OK;
 }
@@ -808,8 +613,7 @@ int mxb_device_axis_histograms(const uint16_t *dev_voxels, int64_t nz, int64_t n
         return EINVAL_;
     }
     return device_axis_histograms(dev_voxels, nz, ny, nx, z_offset, dev_x_bins, dev_y_bins, dev_z_bins,
-                                  dev_r_bins, Nz, Nr, voxel_bins, cy, cx, vmin, vmax, dev_workspace,
-                                  (hipStream_t)stream);
+                                  dev_r_bins, Nz, Nr, voxel_bins, cy, cx, vmin, vmax, (hipStream_t)stream);
 }
 
 int mxb_axis_histograms(const uint16_t *voxels, int64_t nz, int64_t ny, int64_t nx,
@@ -824,11 +628,10 @@ int mxb_axis_histograms(const uint16_t *voxels, int64_t nz, int64_t ny, int64_t 
     }
     const int64_t n = nz * ny * nx;
     if (n == 0) return OK;
-    FBuf v, xb, yb, zb, rb, ws;
+    FBuf v, xb, yb, zb, rb;
     int rc;
     if ((rc = v.alloc(n * 2)) || (rc = xb.alloc(nx * voxel_bins * 8)) || (rc = yb.alloc(ny * voxel_bins * 8)) ||
-        (rc = zb.alloc(Nz * voxel_bins * 8)) || (rc = rb.alloc(Nr * voxel_bins * 8)) ||
-        (rc = ws.alloc(65536 * 4)))
+        (rc = zb.alloc(Nz * voxel_bins * 8)) || (rc = rb.alloc(Nr * voxel_bins * 8)))
         return rc;
     MXB_FHIP(staged_copy(v.p, voxels, n * 2, true, nullptr));
     MXB_FHIP(hipMemcpy(xb.p, x_bins, nx * voxel_bins * 8, hipMemcpyHostToDevice));
@@ -837,7 +640,7 @@ int mxb_axis_histograms(const uint16_t *voxels, int64_t nz, int64_t ny, int64_t 
     if (Nr > 0) MXB_FHIP(hipMemcpy(rb.p, r_bins, Nr * voxel_bins * 8, hipMemcpyHostToDevice));
     rc = device_axis_histograms((const uint16_t *)v.p, nz, ny, nx, z_offset, (uint64_t *)xb.p, (uint64_t *)yb.p,
                                 (uint64_t *)zb.p, (uint64_t *)rb.p, Nz, Nr, voxel_bins, cy, cx, vmin, vmax,
-                                ws.p, nullptr);
+                                nullptr);
     if (rc != OK) return rc;
     MXB_FHIP(hipMemcpy(x_bins, xb.p, nx * voxel_bins * 8, hipMemcpyDeviceToHost));
     MXB_FHIP(hipMemcpy(y_bins, yb.p, ny * voxel_bins * 8, hipMemcpyDeviceToHost));

@@ -1,0 +1,67 @@
+// Bins of uint16 values and 16-byte chunk loads, shared by the histogram kernels.
+#ifndef MXB_HIST_H
+#define MXB_HIST_H
+
+#include <hip/hip_runtime.h>
+
+#include <cstdint>
+
+namespace mxb {
+
+// bin(v) = floor(c * ((v - lo) / d)) in float64 (cpu/histograms.cc:62, :279,
+// :292), counted where vlo <= v <= vhi and 0 <= bin <= c.
+//
+// A table over the 65536 values would make every voxel a scattered read (up
+// to 64 cache lines per wave), so the kernels evaluate the expression.  The
+// division is done with the correctly rounded reciprocal rd = 1/d and one
+// residual: q0 = x rd, q = q0 + (x - q0 d) rd with FMAs, which is the
+// correctly rounded x / d whenever d's significand is not all ones (Markstein,
+// IBM J. Res. Dev. 34(1), 1990); `fast` says that this and the ranges hold,
+// else the kernels divide.
+struct BinMap {
+    double lo, d, rd, c;
+    uint32_t vlo, vhi;
+    int fast;
+};
+
+// mask_range: values outside [lo, hi] are not counted (the voxel axis);
+// otherwise every nonzero value with a bin in range is (the field axis).
+BinMap make_bin_map(double lo, double hi, int64_t nbins, bool mask_range);
+
+// The bin of v, or -1.
+template <bool FAST>
+__device__ __forceinline__ int bin_of(uint32_t v, const BinMap &m) {
+#pragma clang fp contract(off)
+    const double x = (double)v - m.lo;
+    double q;
+    if constexpr (FAST) {
+        q = x * m.rd;
+        q = __builtin_fma(__builtin_fma(-q, m.d, x), m.rd, q);
+    } else {
+        q = x / m.d;
+    }
+    const double t = m.c * q;
+    // t < c + 1 and t >= 0 exactly when floor(t) is a bin (false for NaN)
+    const bool ok = v - m.vlo <= m.vhi - m.vlo && t >= 0.0 && t < m.c + 1.0;
+    return ok ? (int)t : -1;
+}
+
+// Elements 8 c .. 8 c + 7 of `base` (16-byte aligned); those outside [b, e)
+// are not read and come back as 0.
+__device__ __forceinline__ void load_chunk(const uint16_t *__restrict__ base, int64_t c, int64_t b, int64_t e,
+                                           uint16_t q[8]) {
+    const int64_t e0 = c * 8;
+    if (e0 >= b && e0 + 8 <= e) {
+        const uint4 u = *reinterpret_cast<const uint4 *>(base + e0);
+        const uint32_t w[4] = {u.x, u.y, u.z, u.w};
+#pragma unroll
+        for (int k = 0; k < 8; ++k) q[k] = (uint16_t)(w[k >> 1] >> (16 * (k & 1)));
+    } else {
+#pragma unroll
+        for (int k = 0; k < 8; ++k) q[k] = e0 + k >= b && e0 + k < e ? base[e0 + k] : (uint16_t)0;
+    }
+}
+
+}  // namespace mxb
+
+#endif  // MXB_HIST_H

@@ -38,6 +38,12 @@ struct LineGeom {
 // and the device go through pinned chunks filled or drained by host threads.
 hipError_t staged_copy(void *dst, const void *src, size_t bytes, bool h2d, hipStream_t s);
 
+// Axis histograms (mxb_histograms.hip), enqueued on `s`: vb <= 8192, every
+// extent at least 1.
+hipError_t launch_axis_histograms(const uint16_t *vox, int64_t nz, int64_t ny, int64_t nx, int64_t z_offset,
+                                  uint64_t *xb, uint64_t *yb, uint64_t *zb, uint64_t *rb, int64_t Nz, int64_t Nr,
+                                  int64_t vb, int64_t cy, int64_t cx, double vmin, double vmax, hipStream_t s);
+
 // The mask packed to bits along x, words interleaved across y: bit (x mod 32)
 // of word [(z * words_per_row(nx) + x / 32) * ny + y] is (mask[z][y][x] != 0),
 // so one 32-position word of consecutive lines (y) is contiguous.  The

@@ -1,0 +1,60 @@
+"""Histogram kernels at the sizes where their shapes change: ragged rows,
+volumes that start off a 16-byte boundary, table widths from 1 to the most
+bins, radii around the annulus edges, centres off the volume, and value ranges
+whose bin edges fall on whole numbers.  Counts equal the oracle's."""
+import numpy as np
+import pytest
+
+from maxibone_amd import capi, hip
+from oracle import fields as F
+
+pytestmark = pytest.mark.gpu
+
+
+def _at(a, shift):
+    """A device copy of `a` that starts `shift` bytes after an aligned address."""
+    buf = hip.DeviceBuffer(a.nbytes + 64)
+    hip.check(hip.rt().hipMemcpy(buf.ptr + shift, np.ascontiguousarray(a).ctypes.data, a.nbytes, hip.H2D))
+    return buf
+
+
+AXIS = [  # shape, z_offset, Nz, Nr, bins, centre, range, byte shift, distinct values
+    ((3, 1, 1), 0, 3, 1, 1, (0, 0), (1.0, 65535.0), 0, None),
+    ((5, 7, 9), 0, 5, 40, 3, (30, -20), (0.0, 65535.0), 2, None),
+    ((70, 9, 130), 5, 60, 70, 256, (4, 65), (1.0, 40000.0), 0, None),
+    ((33, 40, 61), 0, 33, 50, 4096, (20, 30), (1.0, 40000.0), 6, None),
+    ((40, 64, 72), 0, 40, 16, 4096, (32, 36), (13333.0, 26666.0), 0, None),
+    ((40, 64, 72), 0, 40, 17, 4097, (31, 36), (0.1, 60000.7), 0, None),
+    ((9, 33, 264), 0, 9, 150, 8192, (16, 132), (65000.0, 1000.0), 0, None),
+    ((9, 33, 264), 0, 9, 150, 8192, (16, 132), (1.0, 65535.0), 8, None),
+    ((300, 30, 16), 0, 300, 20, 512, (15, 8), (1.0, 65535.0), 0, 2),
+    ((2, 1300, 24), 0, 2, 700, 64, (650, 12), (1.0, 65535.0), 0, None),
+    ((4, 40, 40), 0, 4, 30, 100, (20, 20), (500.0, 500.0), 0, None),
+]
+
+
+@pytest.mark.parametrize("case", range(len(AXIS)))
+def test_axis_histograms_at_edges(gpu, case):
+    shape, z_off, Nz, Nr, vb, centre, vrange, shift, distinct = AXIS[case]
+    print("axis histograms", AXIS[case], flush=True)
+    rng = np.random.default_rng(900 + case)
+    if distinct:
+        vox = (rng.integers(0, distinct, shape) * 30000).astype(np.uint16)
+    else:
+        vox = rng.integers(0, 65536, shape, dtype=np.uint16)
+        vox[rng.random(shape) < 0.1] = 13333
+    sizes = (shape[2], shape[1], Nz, Nr)
+    bins = [rng.integers(0, 3, (n, vb)).astype(np.uint64) for n in sizes]
+    with np.errstate(all="ignore"):
+        if vrange[0] < vrange[1]:
+            want = F.axis_histograms(vox, z_off, *[b.copy() for b in bins], centre, vrange)
+        else:
+            want = bins  # no value lies in the range, or the bin is 0/0
+    L = capi.lib()
+    dv = _at(vox, shift)
+    db = [hip.DeviceBuffer.from_array(b) for b in bins]
+    ws = hip.DeviceBuffer(L.mxb_histogram_workspace_bytes(*shape))
+    capi.check(L.mxb_device_axis_histograms(dv.ptr + shift, *shape, z_off, *(b.ptr for b in db), Nz, Nr, vb,
+                                            centre[0] % 2**64, centre[1] % 2**64, *vrange, ws.ptr, None))
+    for b, w, n in zip(db, want, sizes):
+        assert np.array_equal(b.to_array(np.uint64, (n, vb)), w)

@@ -56,3 +56,36 @@ def test_bf16_widens_to_fp16():
     normal = v >= 2.0 ** -14
     assert np.array_equal(h[normal], v[normal])
     assert np.abs(h[~normal] - v[~normal]).max() <= 2.0 ** -25
+
+
+def test_reciprocal_and_residual_divide_like_float64():
+    """The histogram bins divide with q0 = x r, q = q0 + (x - q0 d) r for the
+    correctly rounded r = 1/d (two FMAs): the correctly rounded quotient x / d
+    for every d whose significand is not all ones."""
+    from fractions import Fraction
+
+    def fma(a, b, c):
+        return float(Fraction(a) * Fraction(b) + Fraction(c))  # one rounding
+
+    rng = np.random.default_rng(9)
+    pairs = [(0.1, 60000.7), (1.0, 40000.0), (1.0, 65535.0), (13333.0, 26666.0), (0.0, 65535.0)]
+    pairs += [tuple(sorted(rng.uniform(0, 65535, 2))) for _ in range(10)]
+    for lo, hi in pairs:
+        d = hi - lo
+        r = 1.0 / d
+        for v in rng.integers(1, 65536, 300).astype(float):
+            x = v - lo
+            q0 = x * r
+            assert fma(fma(-q0, d, x), r, q0) == x / d
+
+
+def test_rings_hold_at_most_seven_pixels_per_radius():
+    """A ring floor(sqrt(dx^2 + dy^2)) = r holds at most 7 (r + 1) lattice
+    points: the bound that keeps the 16-bit radius counters from overflowing."""
+    R = 3000
+    x = np.arange(-R, R + 1, dtype=np.int64)
+    count = np.zeros(R + 1, np.int64)
+    for y in range(R + 1):
+        r = np.floor(np.sqrt((x * x + y * y).astype(np.float64))).astype(np.int64)
+        count += np.bincount(r[r <= R], minlength=R + 1) * (1 if y == 0 else 2)
+    assert (count <= 7 * (np.arange(R + 1) + 1)).all()
