@@ -15,11 +15,7 @@
 // script exactly: (1) max g, max e; (2) min/max of c overall and inside the
 // cylinder; (3) the output.
 //
-// Histograms (cpu/histograms.cc): the float64 bin expressions depend only on
-// the uint16 value, so the host evaluates them once per value into lookup
-// tables (-1 = not counted); field coordinates floor(Z*nz/nZ) etc. become
-// per-axis maps.  Kernels add with 64-bit global atomics (vector memory
-// atomics), after which the caller's bins hold the sums.
+// The histograms' kernels are in mxb_histograms.hip.
 #include <algorithm>
 #include <cmath>
 #include <cstring>
@@ -28,6 +24,7 @@
 
 #include "maxibone_diffusion.h"
 #include "maxibone_fields.h"
+#include "mxb_hist.h"  // launch_field_histogram
 #include "mxb_internal.h"
 
 namespace mxb {
@@ -213,121 +210,6 @@ __global__ __launch_bounds__(kRowThreads) void k_combine_out(const uint16_t *__r
     }
 }
 
-// ------------------------------------------------------------- histograms
-struct FieldHistArgs {
-    int64_t nZ, nY, nX, nz, ny, nx, vb, fb;
-    const int32_t *vlut, *flut;          // per uint16 value: bin or -1
-    const int32_t *zmap, *ymap, *xmap;   // voxel coordinate -> field coordinate
-};
-
-// Field histogram.  The volume is walked in bricks of kBrickZ x kBrickY x
-// kBrickX voxels; each block takes one contiguous range of bricks.  A brick
-// covers a small part of the (smooth) field, so few field bins, and its
-// (field bin, voxel bin) pairs repeat: they gather in an LDS hash table of
-// kHashSlots keys (linear probing) that also counts the distinct keys it
-// holds.  The table reaches the global bins, one atomic per distinct pair,
-// when it holds more than kFlushAt keys after a step of kRowChunk voxels, and
-// at the end of the range; a step adds at most kRowChunk keys, so the table
-// is never more than half full and a free slot or the key itself is always
-// found.  Global atomics are the cost here: walking whole rows, which cross
-// the whole field, took 127 ms on 1024^3 (4096 x 2048 bins), of which 20.7 ms
-// without the atomics.
-constexpr int kHashSlots = 8192;
-constexpr int kHashShift = 19;  // 32 - log2(kHashSlots)
-constexpr uint32_t kFlushAt = kHashSlots / 2 - kRowChunk;
-constexpr unsigned kFieldHistBlocks = 512;  // two 64 KB blocks per CU of a 256-CU device
-constexpr int kBrickX = 64, kBrickY = 32, kBrickZ = 32;
-constexpr int kBrickRowsPerStep = kRowChunk / kBrickX;  // 16 brick rows of 64 voxels per step
-constexpr uint32_t kEmpty = 0xffffffffu;
-static_assert(kHashSlots == (1 << (32 - kHashShift)), "hash table size");
-static_assert(kBrickX % kPerThread == 0 && (kBrickY * kBrickZ) % kBrickRowsPerStep == 0, "brick shape");
-
-__global__ __launch_bounds__(kRowThreads) void k_field_histogram(const uint16_t *__restrict__ vox, const uint16_t *__restrict__ field,
-                                                                 FieldHistArgs a, int vec,
-                                                                 unsigned long long *__restrict__ bins) {
-    __shared__ uint32_t keys[kHashSlots];
-    __shared__ uint32_t counts[kHashSlots];
-    __shared__ uint32_t n_keys;
-    for (int i = threadIdx.x; i < kHashSlots; i += kRowThreads) {
-        keys[i] = kEmpty;
-        counts[i] = 0;
-    }
-    if (threadIdx.x == 0) n_keys = 0;
-    __syncthreads();
-    const int64_t bx_n = (a.nX + kBrickX - 1) / kBrickX, by_n = (a.nY + kBrickY - 1) / kBrickY;
-    const int64_t bricks = bx_n * by_n * ((a.nZ + kBrickZ - 1) / kBrickZ);
-    const int64_t per = (bricks + gridDim.x - 1) / gridDim.x;
-    const int64_t b0 = (int64_t)blockIdx.x * per, b1 = b0 + per < bricks ? b0 + per : bricks;
-    const int xo = (threadIdx.x % (kBrickX / kPerThread)) * kPerThread;
-    const int ro = threadIdx.x / (kBrickX / kPerThread);
-    constexpr int kSteps = kBrickY * kBrickZ / kBrickRowsPerStep;
-    for (int64_t b = b0; b < b1; ++b) {
-        const int64_t bx = b % bx_n, by = (b / bx_n) % by_n, bz = b / (bx_n * by_n);
-        const int64_t x0 = bx * kBrickX + xo;
-        for (int step = 0; step < kSteps; ++step) {
-            const int r = step * kBrickRowsPerStep + ro;
-            const int64_t Y = by * kBrickY + r % kBrickY, Z = bz * kBrickZ + r / kBrickY;
-            if (x0 < a.nX && Y < a.nY && Z < a.nZ) {
-                uint16_t v[8];
-                load8(vox + (Z * a.nY + Y) * a.nX, x0, a.nX, vec != 0, v);
-                const uint16_t *frow = field + ((int64_t)a.zmap[Z] * a.ny + a.ymap[Y]) * a.nx;
-#pragma unroll
-                for (int k = 0; k < 8; ++k) {
-                    if (x0 + k >= a.nX) break;
-                    const int32_t vi = a.vlut[v[k]];
-                    if (vi < 0) continue;
-                    const int32_t fi = a.flut[frow[a.xmap[x0 + k]]];
-                    if (fi < 0) continue;
-                    const uint32_t key = (uint32_t)fi * (uint32_t)a.vb + (uint32_t)vi;
-                    uint32_t slot = (key * 2654435761u) >> kHashShift;
-                    while (true) {
-                        const uint32_t prev = atomicCAS(&keys[slot], kEmpty, key);
-                        if (prev == kEmpty || prev == key) {
-                            atomicAdd(&counts[slot], 1u);
-                            if (prev == kEmpty) atomicAdd(&n_keys, 1u);
-                            break;
-                        }
-                        slot = (slot + 1) & (kHashSlots - 1);
-                    }
-                }
-            }
-            __syncthreads();
-            const bool flush = n_keys > kFlushAt || (b + 1 == b1 && step + 1 == kSteps);  // uniform: between two barriers
-            __syncthreads();
-            if (flush) {
-                for (int i = threadIdx.x; i < kHashSlots; i += kRowThreads) {
-                    const uint32_t key = keys[i];
-                    if (key != kEmpty) {
-                        atomicAdd(&bins[key], (unsigned long long)counts[i]);
-                        keys[i] = kEmpty;
-                        counts[i] = 0;
-                    }
-                }
-                if (threadIdx.x == 0) n_keys = 0;
-                __syncthreads();
-            }
-        }
-    }
-}
-
-// Host-side bin tables: histograms.cc:61-62 (:278-279) and :292.
-static void voxel_lut(double vmin, double vmax, int64_t vb, int32_t *lut) {
-    for (int64_t i = 0; i < 65536; ++i) {
-        const uint16_t raw = (uint16_t)i;
-        const uint16_t voxel = (raw >= vmin && raw <= vmax) ? raw : (uint16_t)0;
-        const int64_t idx = (int64_t)std::floor(static_cast<double>(vb - 1) * ((voxel - vmin) / (vmax - vmin)));
-        lut[i] = (voxel != 0 && idx >= 0 && idx < vb) ? (int32_t)idx : -1;
-    }
-}
-
-static void field_lut(double fmin, double fmax, int64_t fb, int32_t *lut) {
-    for (int64_t i = 0; i < 65536; ++i) {
-        const uint16_t f = (uint16_t)i;
-        const int64_t idx = (int64_t)std::floor(static_cast<double>(fb - 1) * ((f - fmin) / (fmax - fmin)));
-        lut[i] = (f > 0 && idx >= 0 && idx < fb) ? (int32_t)idx : -1;
-    }
-}
-
 static int vec_ok(const void *p, int64_t nx) {
     return (nx % 8 == 0 && reinterpret_cast<uintptr_t>(p) % 16 == 0) ? 1 : 0;
 }
@@ -431,7 +313,7 @@ static int device_combine(const uint16_t *g, const uint16_t *e, int64_t nz, int6
 }
 
 static int64_t field_ws_bytes(int64_t nZ, int64_t nY, int64_t nX) {
-    return 2 * 65536 * 4 + (nZ + nY + nX) * 4 + 256;
+    return kFieldHistWorkspace + (nZ + nY + nX) * 4 + 256;
 }
 
 static int device_field_histogram(const uint16_t *vox, int64_t nZ, int64_t nY, int64_t nX,
@@ -443,26 +325,9 @@ static int device_field_histogram(const uint16_t *vox, int64_t nZ, int64_t nY, i
         set_error("field_histogram: invalid field shape or bin counts");
         return EINVAL_;
     }
-    std::vector<int32_t> host(2 * 65536 + nZ + nY + nX);
-    voxel_lut(vmin, vmax, vb, host.data());
-    field_lut(fmin, fmax, fb, host.data() + 65536);
-    // histograms.cc:246-249, :284-287
-    const double dz = (double)nz / (double)nZ, dy = (double)ny / (double)nY, dx = (double)nx / (double)nX;
-    int32_t *zm = host.data() + 2 * 65536, *ym = zm + nZ, *xm = ym + nY;
-    for (int64_t Z = 0; Z < nZ; ++Z) zm[Z] = (int32_t)std::min<int64_t>(nz - 1, (int64_t)std::floor((double)Z * dz));
-    for (int64_t Y = 0; Y < nY; ++Y) ym[Y] = (int32_t)std::min<int64_t>(ny - 1, (int64_t)std::floor((double)Y * dy));
-    for (int64_t X = 0; X < nX; ++X) xm[X] = (int32_t)std::min<int64_t>(nx - 1, (int64_t)std::floor((double)X * dx));
-    int32_t *d = (int32_t *)ws;
-    MXB_FHIP(hipMemcpyAsync(d, host.data(), host.size() * 4, hipMemcpyHostToDevice, s));
-    FieldHistArgs a{nZ, nY, nX, nz, ny, nx, vb, fb, d, d + 65536, d + 2 * 65536, d + 2 * 65536 + nZ,
-                    d + 2 * 65536 + nZ + nY};
-    const int64_t bricks = ((nX + kBrickX - 1) / kBrickX) * ((nY + kBrickY - 1) / kBrickY) *
-                           ((nZ + kBrickZ - 1) / kBrickZ);
-    const unsigned grid = (unsigned)std::min<int64_t>(bricks, kFieldHistBlocks);
-    hipLaunchKernelGGL(k_field_histogram, dim3(grid), dim3(kRowThreads), 0, s, vox, field, a, vec_ok(vox, nX),
-                       (unsigned long long *)bins);
-    MXB_FHIP_AFTER_COPY(hipGetLastError(), s);
-    // the host table must outlive the copy
+    std::vector<int32_t> words;  // host tables: outlive their copy
+    MXB_FHIP_AFTER_COPY(launch_field_histogram(vox, nZ, nY, nX, field, nz, ny, nx, bins, fb, vb, vmin, vmax, fmin, fmax,
+                                               ws, words, s), s);
     MXB_FHIP(hipStreamSynchronize(s));
     return OK;
 }

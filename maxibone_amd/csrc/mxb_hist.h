@@ -1,10 +1,11 @@
-// Bins of uint16 values and 16-byte chunk loads, shared by the histogram kernels.
+// Bins of uint16 values and 16-byte chunk loads of the histogram kernels.
 #ifndef MXB_HIST_H
 #define MXB_HIST_H
 
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <vector>
 
 namespace mxb {
 
@@ -61,6 +62,16 @@ __device__ __forceinline__ void load_chunk(const uint16_t *__restrict__ base, in
         for (int k = 0; k < 8; ++k) q[k] = e0 + k >= b && e0 + k < e ? base[e0 + k] : (uint16_t)0;
     }
 }
+
+// Bytes of a field histogram's workspace beside 4 per voxel coordinate of each axis.
+constexpr int64_t kFieldHistWorkspace = 2 * 65536 * 4;
+
+// Field histogram, enqueued on `s`.  `words` receives the host tables that are
+// copied to the start of `ws`: they must outlive the copy.
+hipError_t launch_field_histogram(const uint16_t *vox, int64_t nZ, int64_t nY, int64_t nX, const uint16_t *field,
+                                  int64_t nz, int64_t ny, int64_t nx, uint64_t *bins, int64_t fb, int64_t vb,
+                                  double vmin, double vmax, double fmin, double fmax, void *ws,
+                                  std::vector<int32_t> &words, hipStream_t s);
 
 }  // namespace mxb
 

@@ -1,5 +1,6 @@
 // 2D histograms of uint16 volumes (gfx950): the axis histograms of
-// src/lib/cpp/cpu/histograms.cc:14-78.  C entries in mxb_fields.hip.
+// src/lib/cpp/cpu/histograms.cc:14-78 and the field histogram of :231-306.
+// C entries in mxb_fields.hip.
 //
 // Every voxel adds one count to each histogram, so the work is counting, not
 // arithmetic.  A count that goes straight to the 64-bit bins in memory is a
@@ -12,6 +13,7 @@
 #include <algorithm>
 #include <cmath>
 #include <cstring>
+#include <type_traits>
 
 #include "mxb_hist.h"
 #include "mxb_internal.h"
@@ -477,6 +479,648 @@ hipError_t launch_axis_histograms(const uint16_t *vox, int64_t nz, int64_t ny, i
     if (r.zc > kU) r.zc -= r.zc % kU;
     if (m.fast) return wide ? launch_rings<true, true>(vox, r, m, vb, rb, st) : launch_rings<true, false>(vox, r, m, vb, rb, st);
     return wide ? launch_rings<false, true>(vox, r, m, vb, rb, st) : launch_rings<false, false>(vox, r, m, vb, rb, st);
+}
+
+// ------------------------------------------------------------- field histogram
+// Voxels against a field sampled at floor(Z nz / nZ) etc.
+// (cpu/histograms.cc:231-306): one count per voxel into bins[fb][vb], a table
+// far larger than LDS (64 MB at 2048 x 4096).  Noisy voxels over a smooth
+// field give nearly as many (field bin, voxel bin) pairs as voxels in any
+// compact piece of the volume, so gathering pieces in LDS saves little
+// (an LDS hash table per brick: 52 ms at 1024^3, nearly all of it global
+// atomics).  The field is what is smooth: the voxels of a few neighbouring
+// field bins lie in a shell, and their counts fit in LDS.  So:
+//   k_field_ranges: per brick of field values, the least and greatest nonzero
+//                   value;
+//   k_field_plan:   per group of G field bins (an interval of field values,
+//                   as bins are monotone in the value), how many bricks meet
+//                   it, and how many blocks serve it;
+//   k_field_groups: a block takes a group and a share of its bricks.  Its
+//                   waves test the bricks' field values, queue the matches,
+//                   and count the queued values' voxels in the block's
+//                   G x vb table, which reaches the bins once.
+// 1024^3 voxels, 512^3 field, 2048 x 4096 bins: 52.5 -> 4.8 ms; with a 1024^3
+// field 53.5 -> 15.7 (tests of field values against about ten groups each);
+// 240^3 with a 60^3 field 0.71 -> 0.15.  Bound by the latency of the scattered
+// reads (cache lines of a steep field are fetched by several groups' blocks)
+// with 16 waves per CU, which the table allows.
+// A field that is not smooth (noise) makes every brick meet every group; then,
+// and for tables or axes beyond the limits below, k_field_hash counts.
+namespace {
+
+constexpr int kGroupThreads = 1024, kGroupWaves = kGroupThreads / 64;
+constexpr int64_t kGroupCells = 32768;   // 32-bit counters of a block's table (128 KB)
+constexpr int64_t kMaxGroups = 2048;
+constexpr int64_t kMaxBricks = 49152;    // 192 KB of ranges in the workspace
+constexpr int kQueue = 368;              // field values queued per wave
+constexpr int kList = kGroupThreads * 3 / 2; // bricks a block lists at a time
+constexpr int64_t kMaxBox = 512;         // voxels per field value
+constexpr int kGroupBlocks = 1024;       // blocks wanted at most (one fits a CU at a time; 256 leave a long tail)
+constexpr int64_t kBlockVoxels = 2048;   // and one per so many voxels: each clears and flushes its table
+
+struct FieldGeom {
+    int64_t n[3], nf[3];   // voxel and field extents (z, y, x)
+    int32_t nb[3], lb[3];  // bricks, log2 of brick edges (x at least 16)
+    int32_t width[3];      // widest segment
+    int32_t lbox;          // every segment is as wide and a box holds 2^lbox <= 64 voxels; else -1
+    int32_t bricks, ng, G;
+    int32_t blocks_wanted;
+    int32_t pairs;         // layer pairs per unit of work: 4, or 1 where a value stands for many voxels
+    int64_t fb, vb;
+    uint32_t box, m_box, m_xy, m_x;  // voxels per value and magic reciprocals
+    const int32_t *starts[3];        // first voxel coordinate of every segment, and the extent
+    uint32_t *ranges;                // per brick: least << 16 | greatest nonzero value
+    uint32_t *start;                 // per group: first block; [ng]: blocks, [ng + 1]: brick visits
+    const uint32_t *bound;           // per group: least field value, [ng]: end
+    uint32_t visits_max;             // beyond, the hash form counts
+};
+
+// i / d for i < 2^20, d <= 512 by m = ceil(2^32 / d); d = 1: m = 0
+__device__ __forceinline__ uint32_t div_magic(uint32_t i, uint32_t m) { return m == 0 ? i : __umulhi(i, m); }
+
+__device__ __forceinline__ void wave_lds_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+__device__ __forceinline__ void brick_origin(const FieldGeom &g, uint32_t brick, int o[3]) {
+    const uint32_t bx = brick % (uint32_t)g.nb[2], r = brick / (uint32_t)g.nb[2];
+    o[2] = (int)(bx << g.lb[2]);
+    o[1] = (int)((r % (uint32_t)g.nb[1]) << g.lb[1]);
+    o[0] = (int)((r / (uint32_t)g.nb[1]) << g.lb[0]);
+}
+
+// One wave per brick; lanes 16 x by 4 y.  Reads the field once.
+__global__ __launch_bounds__(256) void k_field_ranges(const uint16_t *__restrict__ field, FieldGeom g) {
+    const int lane = threadIdx.x & 63;
+    const uint32_t brick = blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (brick >= (uint32_t)g.bricks) return;
+    int o[3];
+    brick_origin(g, brick, o);
+    uint32_t lo = 65535, hi = 0;
+    const int lx = lane & 15, ly = lane >> 4;
+    for (int z = 0; z < 1 << g.lb[0] && o[0] + z < g.nf[0]; ++z)
+        for (int y = ly; y < 1 << g.lb[1] && o[1] + y < g.nf[1]; y += 4)
+            for (int x = lx; x < 1 << g.lb[2] && o[2] + x < g.nf[2]; x += 16) {
+                const uint32_t f = field[((o[0] + z) * g.nf[1] + o[1] + y) * g.nf[2] + o[2] + x];
+                if (f != 0) {
+                    lo = min(lo, f);
+                    hi = max(hi, f);
+                }
+            }
+    for (int d = 32; d > 0; d >>= 1) {
+        lo = min(lo, (uint32_t)__shfl_xor((int)lo, d));
+        hi = max(hi, (uint32_t)__shfl_xor((int)hi, d));
+    }
+    if (lane == 0) g.ranges[brick] = lo << 16 | hi;
+}
+
+// Blocks per group, in proportion to its work; one block.
+__global__ __launch_bounds__(kGroupThreads) void k_field_plan(FieldGeom g) {
+    __shared__ uint32_t bound[kMaxGroups + 1];
+    __shared__ int32_t diff[kMaxGroups + 1];
+    __shared__ int32_t wsum[kGroupWaves];
+    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+    for (int i = tid; i <= g.ng; i += kGroupThreads) {
+        bound[i] = g.bound[i];
+        diff[i] = 0;
+    }
+    __syncthreads();
+    auto last_at = [&](uint32_t f) {  // the last group that starts at or before f, or -1
+        int lo = -1, hi = g.ng;
+        while (hi - lo > 1) {
+            const int mid = (lo + hi) >> 1;
+            if (bound[mid] <= f) lo = mid;
+            else hi = mid;
+        }
+        return lo;
+    };
+    int met = 0;  // brick visits
+    for (int i = tid; i < g.bricks; i += kGroupThreads) {
+        const uint32_t r = g.ranges[i], lo = r >> 16, hi = r & 0xffffu;
+        if (lo > hi || lo >= bound[g.ng] || hi < bound[0]) continue;
+        int a = last_at(lo), b = last_at(hi);
+        a = a < 0 ? 0 : a;
+        // a visit tests all of the brick's values and counts its share of their voxels
+        const int cost = 4 + 12 * (int)g.box / (b - a + 1);
+        atomicAdd(&diff[a], cost);
+        atomicAdd(&diff[b + 1], -cost);
+        met += b - a + 1;
+    }
+    __syncthreads();
+    // two groups per thread: inclusive scans of diff (work per group), then of
+    // the blocks per group; `before` is what lies before the thread's two
+    auto scan = [&](int a, int b, int &before, int &total) {
+        int incl = a + b;
+#pragma unroll
+        for (int d = 1; d < 64; d <<= 1) {
+            const int u = __shfl_up(incl, d, 64);
+            if (lane >= d) incl += u;
+        }
+        if (lane == 63) wsum[wv] = incl;
+        __syncthreads();
+        before = incl - a - b;
+        total = 0;
+        for (int w = 0; w < kGroupWaves; ++w) {
+            if (w < wv) before += wsum[w];
+            total += wsum[w];
+        }
+        __syncthreads();
+    };
+    const int i0 = 2 * tid, i1 = i0 + 1;
+    const int d0 = i0 < g.ng ? diff[i0] : 0, d1 = i1 < g.ng ? diff[i1] : 0;
+    int before, total, visits, work;
+    scan(met, 0, before, visits);
+    scan(d0, d1, before, total);
+    const int v0 = i0 < g.ng ? before + d0 : 0, v1 = i1 < g.ng ? before + d0 + d1 : 0;
+    scan(v0, v1, before, work);
+    const int64_t want = min(g.blocks_wanted, max(visits, 1));
+    auto blocks = [&](int v) { return v == 0 ? 0 : (int)((v * want + work - 1) / work); };
+    const int p0 = blocks(v0), p1 = blocks(v1);
+    scan(p0, p1, before, total);
+    if (i0 < g.ng) g.start[i0] = (uint32_t)before;
+    if (i1 < g.ng) g.start[i1] = (uint32_t)(before + p0);
+    if (tid == 0) {
+        g.start[g.ng] = (uint32_t)total;
+        g.start[g.ng + 1] = (uint32_t)visits;
+    }
+}
+
+// LDS: the table, the waves' queues and segment starts, the brick list.
+constexpr int kUnitStarts = 17 + 9 + 9;  // x, y, z starts of a unit
+constexpr int kGroupLds = kGroupCells * 4 + (kGroupWaves * (kQueue + kUnitStarts) + kList) * 4;
+static_assert(kGroupLds <= 160 * 1024 - 256, "one block per CU");
+
+__global__ __launch_bounds__(kGroupThreads) void k_field_groups(const uint16_t *__restrict__ vox,
+                                                                const uint16_t *__restrict__ field, FieldGeom g,
+                                                                BinMap vm, BinMap fm,
+                                                                unsigned long long *__restrict__ bins) {
+    extern __shared__ __attribute__((aligned(16))) uint32_t tab[];
+    uint32_t *const queue = tab + kGroupCells + (threadIdx.x >> 6) * kQueue;
+    int32_t *const starts = reinterpret_cast<int32_t *>(tab + kGroupCells + kGroupWaves * kQueue) + (threadIdx.x >> 6) * kUnitStarts;
+    uint32_t *const list = tab + kGroupCells + kGroupWaves * (kQueue + kUnitStarts);
+    __shared__ int32_t s_grp, s_part, s_parts, s_count, s_next;
+    const int tid = threadIdx.x, lane = tid & 63;
+    // neighbouring groups meet the same cache lines: each XCD (block x % 8) takes
+    // a contiguous range of the blocks
+    const uint32_t blocks = g.start[g.ng], each = (blocks + 7) / 8;
+    const uint32_t blk = blockIdx.x % 8 * each + blockIdx.x / 8;
+    if (blockIdx.x / 8 >= each || blk >= blocks || g.start[g.ng + 1] > g.visits_max) return;
+    for (int i = tid; i < g.ng; i += kGroupThreads) {
+        const uint32_t a = g.start[i], b = g.start[i + 1];
+        if (a <= blk && blk < b) {
+            s_grp = i;
+            s_part = (int)(blk - a);
+            s_parts = (int)(b - a);
+        }
+    }
+    if (tid == 0) s_count = 0;
+    clear_tables(tab, (int)(kGroupCells * 4));  // ends in a barrier
+    const int grp = s_grp;
+    const uint32_t part = (uint32_t)s_part, parts = (uint32_t)s_parts;
+    const uint32_t lo = g.bound[grp], hi = g.bound[grp + 1] - 1;
+    const int f0 = grp * g.G;
+    if (lo > hi) return;  // no value has these bins
+
+    // the voxels of the wave's queued field values: entry = local bin row << 10
+    // | z << 7 | y << 4 | x within the unit at o, whose starts are in LDS
+    const int64_t vplane = g.n[1] * g.n[2];
+    // even boxes of 1, 2, 4 .. 64 voxels: a lane keeps one place in the box
+    const int lw = lane & ((int)g.box - 1);
+    const int ldz = (int)div_magic(lw, g.m_xy), ldy = (int)div_magic(lw - ldz * g.width[1] * g.width[2], g.m_x);
+    const uint32_t place = (uint32_t)(ldz * vplane + ldy * g.n[2] + (lw - (ldz * g.width[1] + ldy) * g.width[2]));
+    const int per_step = 64 >> g.lbox, e_lane = lane >> g.lbox;
+    auto drain_even = [&](int n, const int o[3]) {
+        wave_lds_sync();
+        const uint16_t *const base = vox + ((int64_t)o[0] * g.width[0] * g.n[1] + (int64_t)o[1] * g.width[1]) * g.n[2] + (int64_t)o[2] * g.width[2];
+        const uint32_t sz = (uint32_t)(g.width[0] * vplane), sy = (uint32_t)(g.width[1] * g.n[2]), sx = (uint32_t)g.width[2];
+        auto step = [&](int e0, auto U) {
+            constexpr int kU = decltype(U)::value;
+            uint32_t v[kU], row[kU];
+#pragma unroll
+            for (int u = 0; u < kU; ++u) {
+                const int e = e0 + u * per_step;
+                v[u] = 0;
+                row[u] = 0;
+                if (e < n) {
+                    const uint32_t q = queue[e];
+                    v[u] = base[place + (q >> 7 & 7) * sz + (q >> 4 & 7) * sy + (q & 15) * sx];
+                    row[u] = (q >> 10) * (uint32_t)g.vb;
+                }
+            }
+#pragma unroll
+            for (int u = 0; u < kU; ++u) {
+                const int bin = bin_of<true>(v[u], vm);  // 0 has no bin
+                if (bin >= 0) atomicAdd(&tab[row[u] + (uint32_t)bin], 1u);
+            }
+        };
+        // whole steps of 8 loads per lane, then pairs
+        int e0 = 0;
+        for (; e0 + 6 * per_step < n; e0 += 8 * per_step) step(e0 + e_lane, std::integral_constant<int, 8>{});
+        for (; e0 < n; e0 += 2 * per_step) step(e0 + e_lane, std::integral_constant<int, 2>{});
+        wave_lds_sync();
+    };
+    auto drain = [&](int n, const int o[3]) {
+        if (g.lbox >= 0) {
+            drain_even(n, o);
+            return;
+        }
+        wave_lds_sync();
+        const uint32_t items = (uint32_t)n * g.box;
+        constexpr int kU = 4;
+        for (uint32_t i0 = lane; i0 < items; i0 += 64 * kU) {
+            uint32_t v[kU], row[kU];
+#pragma unroll
+            for (int u = 0; u < kU; ++u) {
+                const uint32_t i = i0 + 64 * u;
+                v[u] = 0;
+                row[u] = 0;
+                if (i < items) {
+                    const uint32_t e = div_magic(i, g.m_box), w = i - e * g.box;
+                    const uint32_t dz = div_magic(w, g.m_xy), w2 = w - dz * (uint32_t)(g.width[1] * g.width[2]);
+                    const uint32_t dy = div_magic(w2, g.m_x), dx = w2 - dy * (uint32_t)g.width[2];
+                    const uint32_t q = queue[e];
+                    const int sz = (int)(q >> 7 & 7), sy = (int)(q >> 4 & 7), sx = (int)(q & 15);
+                    const int z = starts[26 + sz] + (int)dz, y = starts[17 + sy] + (int)dy, x = starts[sx] + (int)dx;
+                    const bool in = z < starts[27 + sz] && y < starts[18 + sy] && x < starts[sx + 1];
+                    if (in) {
+                        v[u] = vox[((int64_t)z * g.n[1] + y) * g.n[2] + x];
+                        row[u] = (q >> 10) * (uint32_t)g.vb;
+                    }
+                }
+            }
+#pragma unroll
+            for (int u = 0; u < kU; ++u) {
+                const int bin = bin_of<true>(v[u], vm);  // 0 has no bin
+                if (bin >= 0) atomicAdd(&tab[row[u] + (uint32_t)bin], 1u);
+            }
+        }
+        wave_lds_sync();
+    };
+    // a unit: 16 x 8 x 8 field values of a brick; a lane tests four neighbours
+    // in x in each of four layer pairs
+    const int lx = (lane & 3) * 4, ly = (lane >> 2) & 7, lz = lane >> 5;
+    const int lux = g.lb[2] - 4, luy = g.lb[1] - 3, lp = g.pairs == 4 ? 0 : 2, lunits = lp + lux + luy + g.lb[0] - 3;
+    struct Unit {
+        int o[3];
+        uint2 f[4];
+    };
+    auto fetch = [&](uint32_t brick, int unit, Unit &un) {
+        int *const o = un.o;
+        const int pair0 = unit & ((1 << lp) - 1);
+        unit >>= lp;
+        o[2] = (int)(brick & 0x7ff) << g.lb[2] | (unit & ((1 << lux) - 1)) << 4;
+        o[1] = (int)(brick >> 11 & 0x3ff) << g.lb[1] | (unit >> lux & ((1 << luy) - 1)) << 3;
+        o[0] = (int)(brick >> 21) << g.lb[0] | unit >> (lux + luy) << 3;
+        const int left = (int)g.nf[2] - o[2] - lx;  // values of the row from the lane's first on
+        const bool rows = o[1] + ly < g.nf[1];
+        const int64_t plane = g.nf[1] * g.nf[2];
+        const uint16_t *const p = field + ((int64_t)(o[0] + lz) * g.nf[1] + o[1] + ly) * g.nf[2] + o[2] + lx;
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const bool mine = u >= pair0 && u < pair0 + g.pairs;
+            const bool in = mine && rows && o[0] + lz + 2 * u < g.nf[0];
+            const uint16_t *const q = p + 2 * u * plane;
+            uint2 w = make_uint2(0, 0);
+            if (in && left >= 4) {
+                __builtin_memcpy(&w, q, 8);  // rows start at any 2-byte address
+            } else if (in) {
+                w.x = left > 0 ? q[0] | (left > 1 ? (uint32_t)q[1] << 16 : 0u) : 0u;
+                w.y = left > 2 ? q[2] : 0u;
+            }
+            un.f[u] = w;
+        }
+    };
+    auto count = [&](const Unit &un) {
+        const int *const o = un.o;
+        if (g.lbox < 0 && lane < kUnitStarts) {
+            const int k = lane < 17 ? 2 : (lane < 26 ? 1 : 0), i = lane - (lane < 17 ? 0 : (lane < 26 ? 17 : 26));
+            starts[lane] = g.starts[k][min(o[k] + i, (int)g.nf[k])];
+        }
+        // which of the lane's 16 values belong to the group
+        uint32_t hits = 0;
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const uint32_t f[4] = {un.f[u].x & 0xffffu, un.f[u].x >> 16, un.f[u].y & 0xffffu, un.f[u].y >> 16};
+#pragma unroll
+            for (int k = 0; k < 4; ++k) hits |= f[k] - lo <= hi - lo ? 1u << (4 * u + k) : 0u;  // lo > 0: a zero does not hit
+        }
+        if (__ballot(hits != 0) == 0) return;
+        // queues the lane's values in h, layer pair by layer pair (neighbours in x
+        // stay neighbours); returns the wave's count, queueing none beyond kQueue
+        auto push = [&](uint32_t h) {
+            int at[4], n = 0;
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const uint32_t c = (uint32_t)__popc(h >> (4 * u) & 15u);
+                const uint64_t c0 = __ballot(c & 1), c1 = __ballot(c & 2), c2 = __ballot(c & 4);
+                auto below = [&](uint64_t m) { return (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0)); };
+                at[u] = n + below(c0) + 2 * below(c1) + 4 * below(c2);
+                n += __popcll(c0) + 2 * __popcll(c1) + 4 * __popcll(c2);
+            }
+            if (n > kQueue) return n;
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const uint32_t f[4] = {un.f[u].x & 0xffffu, un.f[u].x >> 16, un.f[u].y & 0xffffu, un.f[u].y >> 16};
+#pragma unroll
+                for (int k = 0; k < 4; ++k)
+                    if (h >> (4 * u + k) & 1) {
+                        const int fi = bin_of<true>(f[k], fm) - f0;
+                        queue[at[u]++] = (uint32_t)fi << 10 | (uint32_t)(lz + 2 * u) << 7 | (uint32_t)ly << 4 | (uint32_t)(lx + k);
+                    }
+            }
+            return n;
+        };
+        // all at once where the queue holds them, else one layer pair (256
+        // values at most) at a time
+        uint32_t left = hits, part = hits;
+#pragma unroll 1
+        for (int u = 0; __ballot(left != 0) != 0;) {
+            const int n = push(part);
+            if (n > kQueue) {
+                part = left & 15u;
+                u = 1;
+                continue;
+            }
+            if (n > 0) drain(n, o);
+            left &= ~part;
+            part = left & (15u << (4 * u));
+            ++u;
+        }
+    };
+
+    for (int b0 = 0; b0 < g.bricks; b0 += kGroupThreads) {
+        const int i = b0 + tid;
+        if (i < g.bricks) {
+            const uint32_t r = g.ranges[i], rlo = r >> 16, rhi = r & 0xffffu;
+            // bricks go to the group's blocks by a hash of their number
+            if (rlo <= hi && rhi >= lo && (((uint32_t)i * 2654435761u) >> 12) % parts == part)
+                {
+                const uint32_t y = (uint32_t)i / (uint32_t)g.nb[2];
+                list[atomicAdd(&s_count, 1)] = (uint32_t)i % (uint32_t)g.nb[2] | y % (uint32_t)g.nb[1] << 11 | y / (uint32_t)g.nb[1] << 21;
+            }
+        }
+        if (tid == 0) s_next = 0;
+        __syncthreads();
+        const int listed = s_count;
+        const bool take = listed > kList - kGroupThreads || b0 + kGroupThreads >= g.bricks;  // uniform
+        if (take) {
+            // the next unit's values are on their way while one is counted
+            auto next = [&](Unit &un) {
+                int e = 0;
+                if (lane == 0) e = atomicAdd(&s_next, 1);
+                e = __builtin_amdgcn_readfirstlane(e);
+                if (e >= listed << lunits) return false;
+                fetch((uint32_t)__builtin_amdgcn_readfirstlane((int)list[e >> lunits]), e & ((1 << lunits) - 1), un);
+                return true;
+            };
+            Unit a, b;
+            bool more = next(a);
+            while (more) {
+                more = next(b);
+                count(a);
+                a = b;
+            }
+        }
+        __syncthreads();
+        if (take && tid == 0) s_count = 0;
+        __syncthreads();
+    }
+    const int64_t rows = g.fb - f0 < g.G ? g.fb - f0 : g.G;
+    flush_tables<true>(tab, rows, g.vb, f0, f0 + rows, bins);
+}
+
+// The general form.  Bricks of 32 x 32 x 64 voxels, walked by blocks that each
+// take a contiguous range; pairs gather in an LDS hash table of kHashSlots
+// keys (linear probing) that also counts its distinct keys.  The table
+// reaches the bins, one atomic per distinct pair, when it holds more than
+// kFlushAt keys after a step of kStepVoxels voxels, and at the end of the
+// range; a step adds at most kStepVoxels keys, so the table is never more than
+// half full and a free slot or the key itself is always found.
+constexpr int kHashThreads = 128, kPerThread = 8;
+constexpr int kStepVoxels = kHashThreads * kPerThread;
+constexpr int kHashSlots = 8192;
+constexpr int kHashShift = 19;  // 32 - log2(kHashSlots)
+constexpr uint32_t kFlushAt = kHashSlots / 2 - kStepVoxels;
+constexpr unsigned kHashBlocks = 512;  // two 64 KB blocks per CU of a 256-CU device
+constexpr int kBrickX = 64, kBrickY = 32, kBrickZ = 32;
+constexpr int kBrickRowsPerStep = kStepVoxels / kBrickX;  // 16 brick rows of 64 voxels per step
+constexpr uint32_t kEmpty = 0xffffffffu;
+static_assert(kHashSlots == (1 << (32 - kHashShift)), "hash table size");
+static_assert(kBrickX % kPerThread == 0 && (kBrickY * kBrickZ) % kBrickRowsPerStep == 0, "brick shape");
+
+struct HashArgs {
+    int64_t nZ, nY, nX, nz, ny, nx, vb;
+    const int32_t *zmap, *ymap, *xmap;  // voxel coordinate -> field coordinate
+    const uint32_t *visits;             // of the grouped form, which counted unless they exceed visits_max; or null
+    uint32_t visits_max;
+};
+
+template <bool FAST>
+__global__ __launch_bounds__(kHashThreads) void k_field_hash(const uint16_t *__restrict__ vox, const uint16_t *__restrict__ field,
+                                                             HashArgs a, BinMap vm, BinMap fm,
+                                                             unsigned long long *__restrict__ bins) {
+    __shared__ uint32_t keys[kHashSlots];
+    __shared__ uint32_t counts[kHashSlots];
+    __shared__ uint32_t n_keys;
+    if (a.visits != nullptr && *a.visits <= a.visits_max) return;
+    for (int i = threadIdx.x; i < kHashSlots; i += kHashThreads) {
+        keys[i] = kEmpty;
+        counts[i] = 0;
+    }
+    if (threadIdx.x == 0) n_keys = 0;
+    __syncthreads();
+    const int64_t bx_n = (a.nX + kBrickX - 1) / kBrickX, by_n = (a.nY + kBrickY - 1) / kBrickY;
+    const int64_t bricks = bx_n * by_n * ((a.nZ + kBrickZ - 1) / kBrickZ);
+    const int64_t per = (bricks + gridDim.x - 1) / gridDim.x;
+    const int64_t b0 = (int64_t)blockIdx.x * per, b1 = b0 + per < bricks ? b0 + per : bricks;
+    const int xo = (threadIdx.x % (kBrickX / kPerThread)) * kPerThread;
+    const int ro = threadIdx.x / (kBrickX / kPerThread);
+    constexpr int kSteps = kBrickY * kBrickZ / kBrickRowsPerStep;
+    for (int64_t b = b0; b < b1; ++b) {
+        const int64_t bx = b % bx_n, by = (b / bx_n) % by_n, bz = b / (bx_n * by_n);
+        const int64_t x0 = bx * kBrickX + xo;
+        for (int step = 0; step < kSteps; ++step) {
+            const int r = step * kBrickRowsPerStep + ro;
+            const int64_t Y = by * kBrickY + r % kBrickY, Z = bz * kBrickZ + r / kBrickY;
+            if (x0 < a.nX && Y < a.nY && Z < a.nZ) {
+                const uint16_t *vrow = vox + (Z * a.nY + Y) * a.nX;
+                const uint16_t *frow = field + ((int64_t)a.zmap[Z] * a.ny + a.ymap[Y]) * a.nx;
+                uint16_t v[8];
+#pragma unroll
+                for (int k = 0; k < 8; ++k) v[k] = x0 + k < a.nX ? vrow[x0 + k] : (uint16_t)0;
+#pragma unroll
+                for (int k = 0; k < 8; ++k) {
+                    if (x0 + k >= a.nX) break;
+                    const int32_t vi = bin_of<FAST>(v[k], vm);
+                    if (vi < 0) continue;
+                    const int32_t fi = bin_of<FAST>(frow[a.xmap[x0 + k]], fm);
+                    if (fi < 0) continue;
+                    const uint32_t key = (uint32_t)fi * (uint32_t)a.vb + (uint32_t)vi;
+                    uint32_t slot = (key * 2654435761u) >> kHashShift;
+                    while (true) {
+                        const uint32_t prev = atomicCAS(&keys[slot], kEmpty, key);
+                        if (prev == kEmpty || prev == key) {
+                            atomicAdd(&counts[slot], 1u);
+                            if (prev == kEmpty) atomicAdd(&n_keys, 1u);
+                            break;
+                        }
+                        slot = (slot + 1) & (kHashSlots - 1);
+                    }
+                }
+            }
+            __syncthreads();
+            const bool flush = n_keys > kFlushAt || (b + 1 == b1 && step + 1 == kSteps);  // uniform: between two barriers
+            __syncthreads();
+            if (flush) {
+                for (int i = threadIdx.x; i < kHashSlots; i += kHashThreads) {
+                    const uint32_t key = keys[i];
+                    if (key != kEmpty) {
+                        atomicAdd(&bins[key], (unsigned long long)counts[i]);
+                        keys[i] = kEmpty;
+                        counts[i] = 0;
+                    }
+                }
+                if (threadIdx.x == 0) n_keys = 0;
+                __syncthreads();
+            }
+        }
+    }
+}
+
+// The least field value whose bin is at least b (65536: none).  Bins are
+// monotone in the value: subtraction, division by a positive number,
+// multiplication and floor all are, rounded or not.
+uint32_t least_value(const BinMap &m, int64_t b) {
+    uint32_t lo = 0, hi = 65536;  // the value 0 is not counted
+    while (hi - lo > 1) {
+        const uint32_t mid = (lo + hi) / 2;
+        if (std::floor(m.c * (((double)mid - m.lo) / m.d)) >= (double)b) hi = mid;
+        else lo = mid;
+    }
+    return hi;
+}
+
+}  // namespace
+
+// Axis tables: the field coordinate of every voxel coordinate (z, y, x axis
+// after axis), then the first voxel coordinate of every segment, and the
+// extent.  A segment is a run of voxel coordinates with one field coordinate.
+struct AxisTables {
+    int64_t ns[3] = {0, 0, 0}, width[3] = {0, 0, 0};  // segments, the widest
+};
+
+static AxisTables axis_tables(const int64_t n[3], const int64_t nf[3], std::vector<int32_t> &words) {
+    AxisTables t;
+    words.clear();
+    for (int k = 0; k < 3; ++k) {
+        const double d = (double)nf[k] / (double)n[k];  // histograms.cc:246-249, :284-287
+        for (int64_t i = 0; i < n[k]; ++i)
+            words.push_back((int32_t)std::min<int64_t>(nf[k] - 1, (int64_t)std::floor((double)i * d)));
+    }
+    int64_t at = 0;
+    for (int k = 0; k < 3; ++k) {
+        int64_t first = 0;
+        for (int64_t i = 0; i <= n[k]; ++i) {
+            if (i != 0 && i != n[k] && words[at + i] == words[at + i - 1]) continue;
+            if (i != 0) t.width[k] = std::max(t.width[k], i - first);
+            if (i != n[k]) ++t.ns[k];
+            first = i;
+            words.push_back((int32_t)i);
+        }
+        at += n[k];
+    }
+    return t;
+}
+
+hipError_t launch_field_histogram(const uint16_t *vox, int64_t nZ, int64_t nY, int64_t nX, const uint16_t *field,
+                                  int64_t nz, int64_t ny, int64_t nx, uint64_t *bins, int64_t fb, int64_t vb,
+                                  double vmin, double vmax, double fmin, double fmax, void *ws,
+                                  std::vector<int32_t> &words, hipStream_t s) {
+    const BinMap vm = make_bin_map(vmin, vmax, vb, true), fm = make_bin_map(fmin, fmax, fb, false);
+    if (vm.vlo > vm.vhi) return hipSuccess;  // no voxel is counted
+    const int64_t n[3] = {nZ, nY, nX}, nf[3] = {nz, ny, nx}, nmaps = nZ + nY + nX;
+    const AxisTables t = axis_tables(n, nf, words);
+    int32_t *const d = static_cast<int32_t *>(ws);
+    unsigned long long *const dst = reinterpret_cast<unsigned long long *>(bins);
+
+    // The grouped form: every field coordinate is sampled (the segments are the
+    // field's coordinates), the tables fit the workspace, a group holds at least one row
+    // of bins, and bins are monotone in the value.
+    FieldGeom g{};
+    g.G = (int32_t)std::min<int64_t>(2047, std::min(fb, kGroupCells / vb));
+    const int64_t box = t.width[0] * t.width[1] * t.width[2];
+    bool grouped = g.G >= 1 && (fb + g.G - 1) / g.G <= kMaxGroups && box <= kMaxBox && vm.fast && fm.fast &&
+                   nmaps <= 40000;
+    for (int k = 0; k < 3; ++k) grouped = grouped && t.ns[k] == nf[k] && nf[k] <= 8192;  // brick numbers of 11, 10 and 11 bits
+    // bricks: 16 x 8 x 8 field values, doubled along the shortest edge (in
+    // voxels) until the table of ranges fits
+    g.lb[0] = 3; g.lb[1] = 3; g.lb[2] = 4;
+    int64_t bricks = 0;
+    while (grouped) {
+        bricks = 1;
+        for (int k = 0; k < 3; ++k) {
+            g.nb[k] = (int32_t)((nf[k] + (int64_t(1) << g.lb[k]) - 1) >> g.lb[k]);
+            bricks *= g.nb[k];
+        }
+        if (bricks <= kMaxBricks) break;
+        int best = 0;
+        for (int k = 1; k < 3; ++k)
+            if ((t.width[k] << g.lb[k]) < (t.width[best] << g.lb[best])) best = k;
+        if (++g.lb[best] > 7) grouped = false;
+    }
+    if (grouped) {
+        g.bricks = (int32_t)bricks;
+        g.fb = fb;
+        g.vb = vb;
+        g.ng = (int32_t)((fb + g.G - 1) / g.G);
+        const int32_t *st = d + nmaps;
+        bool even = true;
+        for (int k = 0; k < 3; ++k) {
+            g.n[k] = n[k];
+            g.nf[k] = nf[k];
+            g.width[k] = (int32_t)t.width[k];
+            even = even && t.width[k] * nf[k] == n[k];
+            g.starts[k] = st;
+            st += t.ns[k] + 1;
+        }
+        auto magic = [](int64_t v) { return v <= 1 ? 0u : (uint32_t)(((uint64_t(1) << 32) + v - 1) / v); };
+        g.box = (uint32_t)box;
+        g.m_box = magic(box);
+        g.m_xy = magic(t.width[1] * t.width[2]);
+        g.m_x = magic(t.width[2]);
+        // testing a field value costs about 1/64 of hashing a voxel (0.7 against
+        // 50 ps at 1024^3), and a value stands for `box` voxels
+        g.visits_max = (uint32_t)std::min<int64_t>(0x7fffffff, 64 * box * bricks);
+        g.bound = reinterpret_cast<const uint32_t *>(d) + words.size();
+        for (int i = 0; i <= g.ng; ++i)
+            words.push_back((int32_t)least_value(fm, i < g.ng ? (int64_t)i * g.G : fb));
+        g.start = reinterpret_cast<uint32_t *>(d) + words.size();
+        g.ranges = g.start + g.ng + 2;
+        g.blocks_wanted = (int32_t)std::max<int64_t>(1, std::min<int64_t>(kGroupBlocks, nZ * nY * nX / kBlockVoxels));
+        g.pairs = box <= 8 ? 4 : 1;
+        // 32-bit offsets within a unit
+        even = even && box <= 64 && (box & (box - 1)) == 0 && 8 * t.width[0] * nY * nX < (int64_t(1) << 31);
+        g.lbox = -1;
+        for (int k = 0; even && k <= 6; ++k)
+            if (box == int64_t(1) << k) g.lbox = k;
+    }
+    hipError_t e = hipMemcpyAsync(ws, words.data(), words.size() * 4, hipMemcpyHostToDevice, s);
+    if (e != hipSuccess) return e;
+    if (grouped) {
+        auto *fn = &k_field_groups;
+        if ((e = allow_lds(fn, kGroupLds)) != hipSuccess) return e;
+        hipLaunchKernelGGL(k_field_ranges, dim3((unsigned)((bricks + 3) / 4)), dim3(256), 0, s, field, g);
+        hipLaunchKernelGGL(k_field_plan, dim3(1), dim3(kGroupThreads), 0, s, g);
+        hipLaunchKernelGGL(fn, dim3((unsigned)(g.blocks_wanted + g.ng + 7) / 8 * 8), dim3(kGroupThreads), kGroupLds, s, vox, field, g, vm, fm, dst);
+    }
+    HashArgs h{nZ, nY, nX, nz, ny, nx, vb, d, d + nZ, d + nZ + nY, grouped ? g.start + g.ng + 1 : nullptr, g.visits_max};
+    const int64_t hb = ((nX + kBrickX - 1) / kBrickX) * ((nY + kBrickY - 1) / kBrickY) * ((nZ + kBrickZ - 1) / kBrickZ);
+    const unsigned grid = (unsigned)std::min<int64_t>(hb, kHashBlocks);
+    if (vm.fast && fm.fast) hipLaunchKernelGGL(k_field_hash<true>, dim3(grid), dim3(kHashThreads), 0, s, vox, field, h, vm, fm, dst);
+    else hipLaunchKernelGGL(k_field_hash<false>, dim3(grid), dim3(kHashThreads), 0, s, vox, field, h, vm, fm, dst);
+    return hipGetLastError();
 }
 
 }  // namespace mxb

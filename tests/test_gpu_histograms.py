@@ -58,3 +58,49 @@ def test_axis_histograms_at_edges(gpu, case):
                                             centre[0] % 2**64, centre[1] % 2**64, *vrange, ws.ptr, None))
     for b, w, n in zip(db, want, sizes):
         assert np.array_equal(b.to_array(np.uint64, (n, vb)), w)
+
+
+def _smooth(shape, top=65535.0):
+    z, y, x = (np.linspace(-1, 1, n) if n > 1 else np.zeros(1) for n in shape)
+    r = np.sqrt(y[:, None] ** 2 + x[None, :] ** 2)
+    f = top * np.exp(-3 * r)[None] * (1 + 0.2 * z[:, None, None]) / 1.2
+    return np.clip(f, 0, 65535).astype(np.uint16)
+
+
+FIELD = [  # voxel shape, field shape, (field bins, voxel bins), voxel range, field range, noisy field
+    ((1, 1, 1), (1, 1, 1), (1, 1), (0.0, 65535.0), (0.0, 65535.0), False),
+    ((20, 40, 37), (20, 40, 37), (2048, 4096), (1.0, 40000.0), (1.0, 65535.0), False),
+    ((33, 50, 71), (17, 25, 36), (2048, 4096), (1.0, 40000.0), (1.0, 65535.0), False),
+    ((33, 50, 71), (22, 33, 47), (500, 5000), (0.1, 60000.7), (100.5, 30000.25), False),
+    ((40, 64, 96), (10, 16, 24), (1024, 256), (1.0, 65535.0), (1.0, 65535.0), False),
+    ((40, 64, 96), (5, 8, 12), (7, 3), (1.0, 65535.0), (20000.0, 50000.0), False),
+    ((36, 44, 52), (3, 4, 4), (300, 1000), (1.0, 65535.0), (1.0, 65535.0), False),     # boxes above the limit
+    ((24, 24, 24), (24, 24, 24), (60, 32768), (1.0, 65535.0), (1.0, 65535.0), False),  # one row per group
+    ((24, 24, 24), (24, 24, 24), (60, 32769), (1.0, 65535.0), (1.0, 65535.0), False),  # no row fits
+    ((24, 24, 24), (24, 24, 24), (2048, 32768), (1.0, 65535.0), (1.0, 65535.0), False),
+    ((24, 24, 24), (24, 24, 24), (2049, 32768), (1.0, 65535.0), (1.0, 65535.0), False),  # groups beyond the limit
+    ((40, 40, 40), (40, 40, 40), (2048, 4096), (1.0, 65535.0), (1.0, 65535.0), True),  # every brick meets most groups
+    ((40, 40, 40), (20, 20, 20), (2048, 4096), (1.0, 65535.0), (1.0, 65535.0), True),
+    ((10, 12, 14), (20, 12, 30), (64, 64), (1.0, 65535.0), (1.0, 65535.0), False),     # field finer than the voxels
+    ((24, 24, 24), (24, 24, 24), (64, 64), (1.0, 65535.0), (65535.0, 1.0), False),     # bins fall with the value
+    ((600, 9, 10), (600, 9, 10), (64, 4096), (30000.0, 30100.0), (60000.0, 60001.0), False),
+]
+
+
+@pytest.mark.parametrize("case", range(len(FIELD)))
+def test_field_histogram_at_edges(gpu, case):
+    vshape, fshape, nbins, vrange, frange, noisy = FIELD[case]
+    print("field histogram", FIELD[case], flush=True)
+    rng = np.random.default_rng(950 + case)
+    vox = np.clip(rng.normal(30000, 9000, vshape), 0, 65535).astype(np.uint16)
+    vox[rng.random(vshape) < 0.1] = 0
+    fld = rng.integers(0, 65536, fshape, dtype=np.uint16) if noisy else _smooth(fshape)
+    fld[rng.random(fshape) < 0.05] = 0
+    init = rng.integers(0, 5, nbins).astype(np.uint64)
+    want = F.field_histogram(vox, fld, init.copy(), vrange, frange)
+    L = capi.lib()
+    dv, df, db = hip.DeviceBuffer.from_array(vox), hip.DeviceBuffer.from_array(fld), hip.DeviceBuffer.from_array(init)
+    ws = hip.DeviceBuffer(L.mxb_histogram_workspace_bytes(*vshape))
+    capi.check(L.mxb_device_field_histogram(dv.ptr, *vshape, df.ptr, *fshape, db.ptr, *nbins, *vrange, *frange,
+                                            ws.ptr, None))
+    assert np.array_equal(db.to_array(np.uint64, nbins), want)
