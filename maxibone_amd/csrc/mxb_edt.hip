@@ -7,17 +7,17 @@
 //   pass x: g1[i] = min over sites j of the row of (i - j)^2
 //   pass y: g2[i] = min_j g1[j] + (i - j)^2 along y
 //   pass z: g3[i] = min_j g2[j] + (i - j)^2 along z
-// Pass x is a row scan (k_edt_rows: per 64-position chunk a ballot of the
-// sites, then the nearest site before and after each chunk by prefix max /
-// suffix min over the chunks).
+// Pass x is a row scan (k_edt_rows).
 //
 // Passes y and z are the lower envelope of the parabolas g[j] + (i - j)^2.
 // Since g[j] + (i - j)^2 = i^2 + (c_j - 2 i j) with c_j = g[j] + j^2, the
 // minimum over j is attained at a vertex of the lower convex hull of the
 // points (j, c_j), and the minimising vertex moves right as i grows.  With
 // at most 4096 voxels per axis, positions are below 2^12 and c below 2^27:
-// 32-bit values, with 64-bit cross products.  One wave per line (64 lanes,
-// a band of L positions per lane, 64 L >= n):
+// 32-bit values, with 64-bit cross products.  With lines enough, a lane walks
+// one line (k_edt_lines); short lines that are few scan outward (k_edt_scan,
+// along z); the rest have one wave per line (k_edt_pass: 64 lanes, a band of L
+// positions per lane, 64 L >= n):
 //   A. each lane builds the lower hull of its band (monotone chain; the
 //      band's values preloaded into registers, the stack in LDS);
 //   B. six rounds merge adjacent groups of bands: the lower bridge of two
@@ -48,6 +48,7 @@
 
 #include "maxibone_diffusion.h"
 #include "maxibone_edt.h"
+#include "mxb_hist.h"
 #include "mxb_internal.h"
 
 namespace mxb {
@@ -55,6 +56,30 @@ namespace mxb {
 namespace {
 
 constexpr uint32_t kNone = MXB_EDT_NONE;
+// The wave's min and max into mm[0], mm[1]: one atomic per value, only when
+// it improves the global one.
+__device__ __forceinline__ void fold_minmax(uint32_t lo, uint32_t hi, uint32_t *mm) {
+#pragma unroll
+    for (int d = 32; d >= 1; d >>= 1) {
+        lo = min(lo, (uint32_t)__shfl_xor((int)lo, d, 64));
+        hi = max(hi, (uint32_t)__shfl_xor((int)hi, d, 64));
+    }
+    if ((threadIdx.x & 63) == 0) {
+        if (lo < __hip_atomic_load(mm, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMin(mm, lo);
+        if (hi > __hip_atomic_load(mm + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(mm + 1, hi);
+    }
+}
+
+// The correctly rounded square root of a whole number below 2^26 (as float32):
+// the reciprocal square root and one residual, equal to sqrtf for every such
+// value (all of them compared), in a third of its instructions.
+__device__ __forceinline__ float root(uint32_t d2) {
+    const float x = (float)d2, y = __builtin_amdgcn_rsqf(x);
+    const float g = x * y;
+    return d2 == 0 ? 0.0f : __builtin_fmaf(__builtin_fmaf(-g, g, x), 0.5f * y, g);
+}
+
+enum EdtOut { kSquared, kDistance, kField };  // what the last pass writes
 constexpr int kMaxLines = 8;              // lines (= waves) per block
 constexpr int kMetaInts = 3 * 64;         // per wave: band lo, hi and spare
 constexpr int kBlockBudget = 80 * 1024;   // LDS bytes per block (two blocks per CU)
@@ -113,7 +138,7 @@ __device__ __forceinline__ int switch_pos(int x0, int c0, int x1, int c1, int n)
     return t > n ? n : t;
 }
 
-// Envelope pass along y or z: uint32 -> uint32, or (LAST) uint32 -> float
+// Envelope pass along y or z: uint32 -> uint32, or uint32 -> float
 // distance x cylinder with the block's min and max folded into P.minmax.
 // Lines per block that the LDS budget admits for a band length L (the host
 // clamps to it): a line needs 4 (pitch + 64 L + kMetaInts) bytes, over 25 KB
@@ -122,7 +147,7 @@ __device__ __forceinline__ int switch_pos(int x0, int c0, int x1, int c1, int n)
 // (64 values each at L = 64) in registers without spilling.
 constexpr int edt_max_lines(int L) { return L >= 64 ? 2 : (L >= 32 ? 4 : kMaxLines); }
 
-template <int L, bool LAST>
+template <int L, EdtOut OUT>
 __global__ __launch_bounds__(edt_max_lines(L) * 64) void k_edt_pass(EdtPass P) {
     extern __shared__ __attribute__((aligned(16))) uint32_t smem[];
     const int kThreads = P.lines * 64;  // one wave per line
@@ -173,7 +198,7 @@ __global__ __launch_bounds__(edt_max_lines(L) * 64) void k_edt_pass(EdtPass P) {
     for (int l = wv; l < nl; l += P.lines) {
         uint32_t *const g = tile + l * P.pitch;
         float cyl = 1.0f;
-        if (LAST && P.cyl != nullptr) cyl = P.cyl[inner0 + l] != 0 ? 1.0f : 0.0f;
+        if (OUT == kField && P.cyl != nullptr) cyl = P.cyl[inner0 + l] != 0 ? 1.0f : 0.0f;
         auto cval = [&](int x) -> int { return (int)g[tix(x)] + x * x; };
 
         // A. lower hull of the band's points (the band's values preloaded)
@@ -339,12 +364,14 @@ __global__ __launch_bounds__(edt_max_lines(L) * 64) void k_edt_pass(EdtPass P) {
         for (int t = 0; t < L; ++t) {
             const int i = b0 + t;
             if (i < n) {
-                if (LAST) {
+                if (OUT != kSquared) {
                     const float d = res[t] == kNone ? INFINITY : sqrtf((float)res[t]);
                     const float f = d * cyl;
-                    const uint32_t o = f2ord_d(f);
-                    omin = min(omin, o);
-                    omax = max(omax, o);
+                    if (OUT == kField) {
+                        const uint32_t o = f2ord_d(f);
+                        omin = min(omin, o);
+                        omax = max(omax, o);
+                    }
                     g[tix(i)] = __float_as_uint(f);
                 } else {
                     g[tix(i)] = res[t];
@@ -368,7 +395,7 @@ __global__ __launch_bounds__(edt_max_lines(L) * 64) void k_edt_pass(EdtPass P) {
             for (int p = tid; p < n; p += kThreads)
                 P.out[base + (int64_t)l * P.inner_stride + (int64_t)p * P.pos_stride] = tile[l * P.pitch + tix(p)];
     }
-    if (LAST) {
+    if (OUT == kField) {
         // block min / max (in the tile's first words, free after the store),
         // then one atomic per value, only when it improves the global one
 #pragma unroll
@@ -402,105 +429,391 @@ __global__ void k_edt_minmax_init(uint32_t *mm) {
     }
 }
 
-// Pass x: g1 = squared distance to the nearest site of the row (sites:
-// data == 0, or data != 0 when INVERT), kNone when the row has none.  One
-// wave per row: a ballot per 64-position chunk gives the chunk's site mask
-// (lane c keeps chunk c's), prefix max / suffix min over the chunks give the
-// nearest site before and after each chunk, and each position combines them
-// with its own chunk's mask.  Reads 1 byte and writes 4 per voxel, both
-// coalesced.
-template <bool INVERT>
-__global__ __launch_bounds__(256) void k_edt_rows(const uint8_t *__restrict__ data, int64_t rows, int nx,
-                                                  uint32_t *__restrict__ out) {
-    constexpr int kNoSite = 1 << 30;
-    const int lane = threadIdx.x & 63;
-    const int nch = (nx + 63) / 64;  // <= 64
-    const int64_t wstride = (int64_t)gridDim.x * (blockDim.x >> 6);
-    for (int64_t r = (int64_t)blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6); r < rows; r += wstride) {
-        const uint8_t *row = data + r * nx;
-        uint32_t *orow = out + r * nx;
-        uint32_t mlo = 0, mhi = 0;  // lane c: chunk c's site mask
-        for (int c = 0; c < nch; ++c) {
-            const int x = 64 * c + lane;
-            bool site = false;
-            if (x < nx) site = (row[x] == 0) != INVERT;
-            const uint64_t m = __ballot(site);
-            if (lane == c) {
-                mlo = (uint32_t)m;
-                mhi = (uint32_t)(m >> 32);
-            }
-        }
-        const uint64_t mine = ((uint64_t)mhi << 32) | mlo;
-        int last = lane < nch && mine != 0 ? 64 * lane + top_bit(mine) : -1;
-        int first = lane < nch && mine != 0 ? 64 * lane + low_bit(mine) : kNoSite;
+// Pass x: the distance to the nearest site of the row (sites: data == 0, or
+// data != 0 when INVERT), as uint16 (0xffff: none) for the lane-per-line pass
+// or squared as uint32 (kNone) for k_edt_pass.  `group` lanes (a power of two)
+// share a row, 16 C voxels each, read and written in 16-byte pieces at any
+// alignment; the nearest site in the lanes before and after comes from a
+// prefix max and a suffix min over the group.  1024^3: 2.15 -> 1.13 ms (2.8
+// TB/s) against one voxel per lane and chunk; half its time is the 20
+// instructions per voxel (four rows per lane with their loads together: the
+// same, and slower for small volumes).
+template <bool INVERT, int C, typename OUT>
+__global__ __launch_bounds__(256) void k_edt_rows(const uint8_t *__restrict__ data, int64_t rows, int nx, int group,
+                                                  OUT *__restrict__ out) {
+    constexpr int kSpan = 16 * C;
+    constexpr int kFar = 20000;  // beyond any distance, and a difference of two still fits 16 bits
+    const int lane = threadIdx.x & 63, gl = lane & (group - 1);
+    const int64_t r = ((int64_t)blockIdx.x * 256 + threadIdx.x) / group;
+    const int x0 = gl * kSpan;
+    const uint8_t *const p = data + r * nx + x0;
+    uint64_t m = 0;  // the lane's sites
+    const int left = r < rows ? nx - x0 : 0;
 #pragma unroll
-        for (int d = 1; d < 64; d <<= 1) {
-            const int a = __shfl_up(last, d, 64);
-            const int b = __shfl_down(first, d, 64);
-            if (lane >= d) last = max(last, a);
-            if (lane + d < 64) first = min(first, b);
+    for (int c = 0; c < C; ++c) {
+        uint32_t bits = 0;  // nonzero bytes of 16
+        if (left >= 16 * c + 16) {
+            uint32_t w[4];
+            __builtin_memcpy(w, p + 16 * c, 16);
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                const uint32_t t = (((w[k] & 0x7f7f7f7fu) + 0x7f7f7f7fu) | w[k]) & 0x80808080u;
+                bits |= ((t * 0x00204081u) >> 28) << (4 * k);  // bits 7, 15, 23, 31 to 28 .. 31
+            }
+            bits = INVERT ? bits : ~bits & 0xffffu;
+        } else {
+#pragma unroll
+            for (int k = 0; k < 16; ++k)
+                if (16 * c + k < left && ((p[16 * c + k] != 0) == INVERT)) bits |= 1u << k;
         }
-        int before = __shfl_up(last, 1, 64);  // nearest site before chunk `lane`
-        int after = __shfl_down(first, 1, 64);
-        if (lane == 0) before = -1;
-        if (lane == 63) after = kNoSite;
-        for (int c = 0; c < nch; ++c) {
-            const uint64_t m = ((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)mhi, c) << 32) |
-                               (uint32_t)__builtin_amdgcn_readlane((int)mlo, c);
-            const int bc = __builtin_amdgcn_readlane(before, c), ac = __builtin_amdgcn_readlane(after, c);
-            const int x = 64 * c + lane;
-            const uint64_t below = m & bits_below(lane + 1), above = m & ~bits_below(lane);
-            const int l = below != 0 ? 64 * c + top_bit(below) : bc;
-            const int nx_site = above != 0 ? 64 * c + low_bit(above) : ac;
-            int d = kNoSite;
-            if (l >= 0) d = x - l;
-            if (nx_site < kNoSite) d = min(d, nx_site - x);
-            if (x < nx) orow[x] = d < kNoSite ? (uint32_t)(d * d) : kNone;
+        m |= (uint64_t)bits << (16 * c);
+    }
+    int last = m != 0 ? x0 + top_bit(m) : -kFar, first = m != 0 ? x0 + low_bit(m) : kFar;
+    for (int d = 1; d < group; d <<= 1) {
+        const int a = __shfl_up(last, d, group), b = __shfl_down(first, d, group);
+        if (gl >= d) last = max(last, a);
+        if (gl + d < group) first = min(first, b);
+    }
+    int before = __shfl_up(last, 1, group), after = __shfl_down(first, 1, group);
+    if (gl == 0) before = -kFar;
+    if (gl == group - 1) after = kFar;
+    if (left <= 0) return;
+    uint16_t d[kSpan];
+#pragma unroll
+    for (int k = 0; k < kSpan; ++k) {
+        if (m >> k & 1) before = x0 + k;
+        d[k] = (uint16_t)(x0 + k - before);
+    }
+#pragma unroll
+    for (int k = kSpan - 1; k >= 0; --k) {
+        if (m >> k & 1) after = x0 + k;
+        const int e = min((int)d[k], after - x0 - k);
+        d[k] = e > 4095 ? (uint16_t)0xffffu : (uint16_t)e;
+    }
+    OUT *const o = out + r * nx + x0;
+    constexpr int kPer = 16 / (int)sizeof(OUT);
+#pragma unroll
+    for (int k = 0; k < kSpan; k += kPer) {
+        OUT v[kPer];
+#pragma unroll
+        for (int t = 0; t < kPer; ++t) {
+            if constexpr (sizeof(OUT) == 2) v[t] = d[k + t];
+            else v[t] = d[k + t] == 0xffffu ? kNone : (uint32_t)d[k + t] * d[k + t];
+        }
+        if (left >= k + kPer) {
+            __builtin_memcpy(o + k, v, 16);
+        } else {
+#pragma unroll
+            for (int t = 0; t < kPer; ++t)
+                if (k + t < left) o[k + t] = v[t];
         }
     }
 }
 
+// ---- one lane per line
+// With lines enough to fill the device, a lane walks one line serially: the
+// lower hull by a stack (each point is pushed once and popped at most once),
+// then the answers from the far end, the stack shrinking as earlier vertices
+// take over.  64 neighbouring lines are consecutive in memory, so all loads
+// and stores are whole cache lines, and neighbours' stacks move alike.  The
+// two uppermost entries live in registers, the next kRing in an LDS ring, and
+// deeper ones in memory (`stack`), reached by evictions and by refills that
+// the whole wave makes together; each is one 32-bit word:
+//   Y: input uint16 distances; memory entries hold the position as uint16 in
+//      the half of the workspace that the input leaves free, the value is
+//      read again from the input;
+//   Z: input uint32 squared distances; entries hold position << gbits | value
+//      and are stored over the input (entry m <= positions read so far).
+// The turn test is done in float64, where products below 2^39 are exact.
+// 1024^3 implant field: y 10.1 -> 2.05 ms, z 14.8 -> 4.0 ms against one wave
+// per line (k_edt_pass: 7100 instructions per 1024-voxel line and one min/max
+// atomic per block); about 125 instructions per 64 voxels, half the VALU rate.
+struct EdtLines {
+    const void *in;
+    void *stack;
+    uint32_t *out;
+    int n;                       // positions per line
+    int64_t pos_stride;          // elements between positions
+    int64_t lines, inner;        // lines; consecutive ones
+    int64_t outer_stride;        // elements between runs of `inner` lines
+    int gbits;                   // Z: bits of a value
+    const uint8_t *cyl;          // kField: cylinder mask per line, or null
+    uint32_t *minmax;            // kField: ordered-encoded min and max
+};
+
+constexpr int kLineThreads = 256;
+constexpr int kRing = 16;    // entries per line in LDS (16 KB per block: eight blocks per CU)
+constexpr int kRefill = 8;
+
+template <bool Y, EdtOut OUT>
+__global__ __launch_bounds__(kLineThreads) void k_edt_lines(EdtLines P) {
+    __shared__ uint32_t ring[kRing][kLineThreads];
+    const int tid = threadIdx.x;
+    const int64_t line = (int64_t)blockIdx.x * kLineThreads + tid;
+    const bool live = line < P.lines;
+    const int64_t run = live ? line / P.inner : 0;
+    const int64_t base = live ? run * P.outer_stride + (line - run * P.inner) : 0;
+    const int64_t ps = P.pos_stride;
+    const int n = P.n;
+    const uint16_t *const in16 = static_cast<const uint16_t *>(P.in) + base;
+    const uint32_t *const in32 = static_cast<const uint32_t *>(P.in) + base;
+    uint16_t *const st16 = static_cast<uint16_t *>(P.stack) + base;
+    uint32_t *const st32 = static_cast<uint32_t *>(P.stack) + base;
+    const int gbits = P.gbits;
+    const uint32_t gmask = (1u << gbits) - 1;
+
+    auto load = [&](int j) -> uint32_t {
+        if constexpr (Y) return in16[j * ps];
+        else return in32[j * ps];
+    };
+    auto none = [&](uint32_t g) { return Y ? g == 0xffffu : g == kNone; };
+    auto entry = [&](int j, uint32_t g) { return Y ? (uint32_t)j << 16 | g : (uint32_t)j << gbits | g; };
+    auto pos_of = [&](uint32_t e) { return (int)(Y ? e >> 16 : e >> gbits); };
+    auto val_of = [&](uint32_t e) { return (int)(Y ? (e & 0xffffu) * (e & 0xffffu) : e & gmask); };
+
+    // entries [0, vlo) are in memory, [vlo, h - 2) in the ring, h - 2 and
+    // h - 1 (the top) in registers
+    int h = 0, vlo = 0;
+    auto evict = [&]() {  // the ring's lowest entry to memory
+        const uint32_t e = ring[vlo & (kRing - 1)][tid];
+        if constexpr (Y) st16[vlo * ps] = (uint16_t)(e >> 16);
+        else st32[vlo * ps] = e;
+        ++vlo;
+    };
+    auto refill = [&]() {  // up to kRefill entries from memory, below the ring's
+        const int c = vlo < kRefill ? vlo : kRefill;
+        uint32_t e[kRefill];
+#pragma unroll
+        for (int k = 0; k < kRefill; ++k) {
+            e[k] = 0;
+            if (k < c) e[k] = Y ? (uint32_t)st16[(vlo - 1 - k) * ps] : st32[(vlo - 1 - k) * ps];
+        }
+        if constexpr (Y) {
+#pragma unroll
+            for (int k = 0; k < kRefill; ++k)
+                if (k < c) e[k] = e[k] << 16 | in16[e[k] * ps];
+        }
+#pragma unroll
+        for (int k = 0; k < kRefill; ++k)
+            if (k < c) ring[(vlo - 1 - k) & (kRing - 1)][tid] = e[k];
+        vlo -= c;
+    };
+
+    // forward: the hull
+    uint32_t pa = 0, pb = 0;                     // second and top entry
+    double xa = 0, ca = 0, xb = 0, cb = 0;       // their points (j, g + j^2)
+    auto open = [&](uint32_t e, double &x, double &c) {
+        const int j = pos_of(e);
+        x = (double)j;
+        c = (double)(val_of(e) + __mul24(j, j));
+    };
+    constexpr int kAhead = 8;
+    uint32_t cur[kAhead], nxt[kAhead];
+    const uint32_t nothing = Y ? 0xffffu : kNone;
+#pragma unroll
+    for (int k = 0; k < kAhead; ++k) cur[k] = live && k < n ? load(k) : nothing;
+    for (int j0 = 0; j0 < n; j0 += kAhead) {
+#pragma unroll
+        for (int k = 0; k < kAhead; ++k) nxt[k] = live && j0 + kAhead + k < n ? load(j0 + kAhead + k) : nothing;
+#pragma unroll
+        for (int k = 0; k < kAhead; ++k) {
+            const int j = j0 + k;
+            if (!none(cur[k])) {
+                const uint32_t e = entry(j, cur[k]);
+                const double x = (double)j;
+                const double c = (double)((int)(Y ? cur[k] * cur[k] : cur[k]) + j * j);
+                while (h >= 2 && __builtin_fma(xb - xa, c - ca, -((cb - ca) * (x - xa))) <= 0.0) {
+                    --h;  // the top is on or above the segment between its neighbours
+                    pb = pa; xb = xa; cb = ca;
+                    if (h >= 2) {
+                        if (h - 2 < vlo) refill();
+                        pa = ring[(h - 2) & (kRing - 1)][tid];
+                        open(pa, xa, ca);
+                    }
+                }
+                if (h >= 2) {  // the second goes to the ring
+                    if (h - 2 - vlo == kRing) evict();
+                    ring[(h - 2) & (kRing - 1)][tid] = pa;
+                }
+                pa = pb; xa = xb; ca = cb;
+                pb = e; xb = x; cb = c;
+                ++h;
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < kAhead; ++k) cur[k] = nxt[k];
+    }
+
+    // backward: position i belongs to the top until the vertex below ties or wins
+    uint32_t *const out = P.out + base;
+    uint32_t lo = 0xffffffffu, hi = 0;
+    int xt = pos_of(pb), gt = val_of(pb), xs = pos_of(pa), gs = val_of(pa);
+    for (int i = n - 1; i >= 0; --i) {
+        // keep four entries at hand: all lanes with room refill together
+        if (__ballot(vlo > 0 && h - 2 - vlo < 4) != 0 && vlo > 0 && h - 2 - vlo <= kRing - kRefill) refill();
+        while (h >= 2 && gs + __mul24(i - xs, i - xs) <= gt + __mul24(i - xt, i - xt)) {
+            --h;
+            xt = xs; gt = gs;
+            if (h >= 2) {
+                if (h - 2 < vlo) refill();
+                const uint32_t e = ring[(h - 2) & (kRing - 1)][tid];
+                xs = pos_of(e);
+                gs = val_of(e);
+            }
+        }
+        const uint32_t d2 = h > 0 ? (uint32_t)(gt + __mul24(i - xt, i - xt)) : kNone;
+        if (live) {
+            if constexpr (OUT == kSquared) {
+                out[i * ps] = d2;
+            } else {
+                float cyl = 1.0f;
+                if (OUT == kField && P.cyl != nullptr) cyl = P.cyl[line] != 0 ? 1.0f : 0.0f;
+                const float f = (d2 == kNone ? INFINITY : root(d2)) * cyl;
+                out[i * ps] = __float_as_uint(f);
+                if constexpr (OUT == kField) {
+                    const uint32_t o = f2ord_d(f);
+                    lo = min(lo, o);
+                    hi = max(hi, o);
+                }
+            }
+        }
+    }
+    if constexpr (OUT == kField) fold_minmax(lo, hi, P.minmax);
+}
+
+// ---- outward scan
+// With too few lines for a lane each, and short ones, every position looks
+// outward for its minimum: g[j] + (i - j)^2 cannot win once (i - j)^2 reaches
+// the best value found.  A block holds 64 neighbouring lines in LDS (a lane's
+// line in its own bank); a thread answers 8 consecutive positions of a line
+// together, so a value read serves 8 of them with an addition and a minimum
+// each, the squares being uniform: from the left, at distance t from the
+// first position, g + t^2 + 2 t k + k^2 for position k, and mirrored from the
+// right.
+constexpr int kScanLines = 64, kScanMax = 256;  // 64 KB of LDS at most
+
+template <EdtOut OUT>
+__global__ __launch_bounds__(512) void k_edt_scan(EdtLines P) {
+    extern __shared__ int32_t vals[];  // [n][kScanLines]
+    constexpr int kFarValue = 1 << 29;
+    const int n = P.n, lane = threadIdx.x & 63, waves = blockDim.x >> 6;
+    const int64_t line = (int64_t)blockIdx.x * kScanLines + lane;
+    const bool live = line < P.lines;
+    const int64_t run = live ? line / P.inner : 0;
+    const int64_t base = live ? run * P.outer_stride + (line - run * P.inner) : 0;
+    const uint32_t *const in = static_cast<const uint32_t *>(P.in) + base;
+    for (int j = threadIdx.x >> 6; j < n; j += waves) {
+        const uint32_t g = live ? in[j * P.pos_stride] : kNone;
+        vals[j * kScanLines + lane] = g == kNone ? kFarValue : (int)g;
+    }
+    __syncthreads();
+    float cyl = 1.0f;
+    if (OUT == kField && P.cyl != nullptr && live) cyl = P.cyl[line] != 0 ? 1.0f : 0.0f;
+    uint32_t lo = 0xffffffffu, hi = 0;
+    for (int i0 = 8 * (threadIdx.x >> 6); i0 < n; i0 += 8 * waves) {
+        // l[k]: best from the left and within, less k^2; r[k]: from the right, less (7 - k)^2
+        int l[8], r[8];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) l[k] = r[k] = kFarValue;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const int g = i0 + j < n ? vals[(i0 + j) * kScanLines + lane] : kFarValue;
+#pragma unroll
+            for (int k = 0; k < 8; ++k) l[k] = min(l[k], g + (j - k) * (j - k) - k * k);
+        }
+        const int reach = max(i0, n - 8 - i0);
+        for (int t0 = 1; t0 <= reach; t0 += 4) {
+            int worst = 0;
+#pragma unroll
+            for (int k = 0; k < 8; ++k)
+                if (i0 + k < n) worst = max(worst, min(l[k] + k * k, r[k] + (7 - k) * (7 - k)));
+            if (__ballot(worst > t0 * t0) == 0) break;
+            int a[4], b[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const int t = t0 + u, jl = i0 - t, jr = i0 + 7 + t;
+                a[u] = jl >= 0 ? vals[jl * kScanLines + lane] : kFarValue;
+                b[u] = jr < n ? vals[jr * kScanLines + lane] : kFarValue;
+            }
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const int t = t0 + u, ca = a[u] + t * t, cb = b[u] + t * t;
+#pragma unroll
+                for (int k = 0; k < 8; ++k) {
+                    l[k] = min(l[k], ca + 2 * t * k);
+                    r[k] = min(r[k], cb + 2 * t * (7 - k));
+                }
+            }
+        }
+        if (live) {
+#pragma unroll
+            for (int k = 0; k < 8; ++k) {
+                if (i0 + k >= n) break;
+                const int best = min(l[k] + k * k, r[k] + (7 - k) * (7 - k));
+                const uint32_t d2 = best < kFarValue / 2 ? (uint32_t)best : kNone;
+                uint32_t *const o = P.out + base + (i0 + k) * P.pos_stride;
+                if constexpr (OUT == kSquared) {
+                    *o = d2;
+                } else {
+                    const float f = (d2 == kNone ? INFINITY : root(d2)) * cyl;
+                    *o = __float_as_uint(f);
+                    if constexpr (OUT == kField) {
+                        lo = min(lo, f2ord_d(f));
+                        hi = max(hi, f2ord_d(f));
+                    }
+                }
+            }
+        }
+    }
+    if constexpr (OUT == kField) fold_minmax(lo, hi, P.minmax);
+}
+
 // general.hh:96-118 on the float field: (uint16)((f - vmin) / (vmax - vmin) *
-// 65535) with vmax starting at FLT_MIN (general.hh:78), then x cylinder.
-// Rows of nx voxels, 4 per thread (one 16-byte load where nx % 4 == 0).
-__global__ __launch_bounds__(256) void k_edt_to_u16(const float *__restrict__ f, int64_t rows, int64_t ny,
-                                                    int64_t nx, const uint8_t *__restrict__ cyl,
+// 65535) with vmax starting at FLT_MIN (general.hh:78), then x cylinder.  A
+// thread takes 8 neighbours of a plane (the cylinder mask is one plane), at
+// any alignment.  The division is by a value all threads share, done with its
+// reciprocal and a residual (Div in mxb_hist.h); 1024^3: 1.8 -> 1.2 ms, where
+// rows, a 64-bit division per item and IEEE division sequences held the loads
+// back.
+__global__ __launch_bounds__(256) void k_edt_to_u16(const float *__restrict__ f, int64_t nz, int64_t plane,
+                                                    const uint8_t *__restrict__ cyl,
                                                     const uint32_t *__restrict__ mm,
                                                     uint16_t *__restrict__ out) {
     const float vmin = ord2f_d(mm[0]);
     const float vmax = fmaxf(ord2f_d(mm[1]), FLT_MIN);
-    const float span = vmax - vmin;
-    const int64_t per_row = (nx + 1023) / 1024;
-    const int64_t items = rows * per_row;
-    const bool vec = nx % 4 == 0;
-    for (int64_t it = blockIdx.x; it < items; it += gridDim.x) {
-        const int64_t r = it / per_row;
-        const int64_t x0 = (it % per_row) * 1024 + 4 * threadIdx.x;
-        if (x0 >= nx) continue;
-        const float *fr = f + r * nx;
-        const uint8_t *cr = cyl != nullptr ? cyl + (r % ny) * nx : nullptr;
-        uint16_t *orow = out + r * nx;
-        float v[4];
-        if (vec) {
-            const float4 q = *reinterpret_cast<const float4 *>(fr + x0);
-            v[0] = q.x; v[1] = q.y; v[2] = q.z; v[3] = q.w;
-        } else {
+    const SharedDiv div(vmax - vmin);
+    const int64_t e0 = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 8;
+    if (e0 >= plane) return;
+    const int left = plane - e0 < 8 ? (int)(plane - e0) : 8;
+    uint8_t c[8];
 #pragma unroll
-            for (int k = 0; k < 4; ++k) v[k] = x0 + k < nx ? fr[x0 + k] : 0.0f;
-        }
-        uint16_t o[4];
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            o[k] = (uint16_t)((v[k] - vmin) / span * 65535.0f);
-            if (cr != nullptr && x0 + k < nx && cr[x0 + k] == 0) o[k] = 0;
-        }
-        if (vec) {
-            *reinterpret_cast<uint2 *>(orow + x0) =
-                make_uint2((uint32_t)o[0] | ((uint32_t)o[1] << 16), (uint32_t)o[2] | ((uint32_t)o[3] << 16));
-        } else {
-            for (int k = 0; k < 4 && x0 + k < nx; ++k) orow[x0 + k] = o[k];
-        }
+    for (int k = 0; k < 8; ++k) c[k] = 1;
+    if (cyl != nullptr) {
+        if (left == 8) __builtin_memcpy(c, cyl + e0, 8);
+        else
+            for (int k = 0; k < left; ++k) c[k] = cyl[e0 + k];
     }
+    auto convert = [&](auto by) {
+        for (int64_t z = blockIdx.y; z < nz; z += gridDim.y) {
+            const float *const src = f + z * plane + e0;
+            uint16_t *const dst = out + z * plane + e0;
+            float v[8];
+            if (left == 8) __builtin_memcpy(v, src, 32);
+            else
+                for (int k = 0; k < 8; ++k) v[k] = k < left ? src[k] : 0.0f;
+            uint16_t o[8];
+#pragma unroll
+            for (int k = 0; k < 8; ++k) {
+                o[k] = (uint16_t)(by(v[k] - vmin) * 65535.0f);
+                if (c[k] == 0) o[k] = 0;
+            }
+            if (left == 8) __builtin_memcpy(dst, o, 16);
+            else
+                for (int k = 0; k < left; ++k) dst[k] = o[k];
+        }
+    };
+    if (div.exact) convert([&](float x) { return div.quick(x); });
+    else convert([&](float x) { return x / div.d; });
 }
 
 // Band length per lane: the least power of two with 64 L >= n.
@@ -515,28 +828,28 @@ size_t pass_smem(const EdtPass &P) {
     return (size_t)4 * P.lines * ((size_t)P.pitch + (size_t)(64 * L) + kMetaInts);
 }
 
-template <int L, bool LAST>
+template <int L, EdtOut OUT>
 hipError_t launch_l(const EdtPass &P, hipStream_t s) {
     if (P.lines > edt_max_lines(L)) return hipErrorInvalidValue;  // beyond the launch bound
     const size_t smem = pass_smem(P);
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(&k_edt_pass<L, LAST>),
+    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(&k_edt_pass<L, OUT>),
                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
     if (e != hipSuccess) return e;
     const int64_t blocks = ((P.n_inner + P.lines - 1) / P.lines) * P.n_outer;
-    hipLaunchKernelGGL((k_edt_pass<L, LAST>), dim3((unsigned)blocks), dim3(P.lines * 64), smem, s, P);
+    hipLaunchKernelGGL((k_edt_pass<L, OUT>), dim3((unsigned)blocks), dim3(P.lines * 64), smem, s, P);
     return hipGetLastError();
 }
 
-template <bool LAST>
+template <EdtOut OUT>
 hipError_t launch_mode(const EdtPass &P, hipStream_t s) {
     const int64_t need = (P.n + 63) / 64;
-    if (need <= 1) return launch_l<1, LAST>(P, s);
-    if (need <= 2) return launch_l<2, LAST>(P, s);
-    if (need <= 4) return launch_l<4, LAST>(P, s);
-    if (need <= 8) return launch_l<8, LAST>(P, s);
-    if (need <= 16) return launch_l<16, LAST>(P, s);
-    if (need <= 32) return launch_l<32, LAST>(P, s);
-    return launch_l<64, LAST>(P, s);
+    if (need <= 1) return launch_l<1, OUT>(P, s);
+    if (need <= 2) return launch_l<2, OUT>(P, s);
+    if (need <= 4) return launch_l<4, OUT>(P, s);
+    if (need <= 8) return launch_l<8, OUT>(P, s);
+    if (need <= 16) return launch_l<16, OUT>(P, s);
+    if (need <= 32) return launch_l<32, OUT>(P, s);
+    return launch_l<64, OUT>(P, s);
 }
 
 // Geometry of the pass along axis a (0 z, 1 y, 2 x) of an (nz, ny, nx) volume.
@@ -561,19 +874,62 @@ EdtPass pass_geom(int a, int64_t nz, int64_t ny, int64_t nx) {
     return P;
 }
 
-hipError_t run_pass(bool last, EdtPass P, hipStream_t s) {
+hipError_t run_pass(EdtOut mode, EdtPass P, hipStream_t s) {
     if (P.n_inner * P.n_outer == 0 || P.n == 0) return hipSuccess;
-    return last ? launch_mode<true>(P, s) : launch_mode<false>(P, s);
+    if (mode == kSquared) return launch_mode<kSquared>(P, s);
+    return mode == kDistance ? launch_mode<kDistance>(P, s) : launch_mode<kField>(P, s);
 }
 
-hipError_t run_rows(const uint8_t *data, bool invert, int64_t rows, int64_t nx, uint32_t *out, hipStream_t s) {
+template <bool INVERT, typename OUT>
+hipError_t launch_rows(const uint8_t *data, int64_t rows, int64_t nx, OUT *out, hipStream_t s) {
+    const int c = (int)((nx + 1023) / 1024);  // 1 .. 4 (at most 4096 voxels)
+    int group = 1;
+    while (group < 64 && group * 16 * c < nx) group <<= 1;
+    const unsigned blocks = (unsigned)((rows * group + 255) / 256);
+    if (c == 1) hipLaunchKernelGGL((k_edt_rows<INVERT, 1, OUT>), dim3(blocks), dim3(256), 0, s, data, rows, (int)nx, group, out);
+    else if (c == 2) hipLaunchKernelGGL((k_edt_rows<INVERT, 2, OUT>), dim3(blocks), dim3(256), 0, s, data, rows, (int)nx, group, out);
+    else hipLaunchKernelGGL((k_edt_rows<INVERT, 4, OUT>), dim3(blocks), dim3(256), 0, s, data, rows, (int)nx, group, out);
+    return hipGetLastError();
+}
+
+template <typename OUT>
+hipError_t run_rows(const uint8_t *data, bool invert, int64_t rows, int64_t nx, OUT *out, hipStream_t s) {
     if (rows == 0 || nx == 0) return hipSuccess;
-    int64_t blocks = (rows + 3) / 4;
-    if (blocks > 65536) blocks = 65536;
-    if (invert)
-        hipLaunchKernelGGL(k_edt_rows<true>, dim3((unsigned)blocks), dim3(256), 0, s, data, rows, (int)nx, out);
-    else
-        hipLaunchKernelGGL(k_edt_rows<false>, dim3((unsigned)blocks), dim3(256), 0, s, data, rows, (int)nx, out);
+    return invert ? launch_rows<true>(data, rows, nx, out, s) : launch_rows<false>(data, rows, nx, out, s);
+}
+
+template <EdtOut OUT>
+hipError_t launch_scan(const EdtLines &P, hipStream_t s) {
+    const size_t smem = (size_t)P.n * kScanLines * 4;
+    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(&k_edt_scan<OUT>),
+                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
+    if (e != hipSuccess) return e;
+    const unsigned waves = P.n > 128 ? 8 : 4;
+    hipLaunchKernelGGL(k_edt_scan<OUT>, dim3((unsigned)((P.lines + kScanLines - 1) / kScanLines)), dim3(64 * waves), smem, s, P);
+    return hipGetLastError();
+}
+
+hipError_t run_scan(const EdtLines &P, EdtOut mode, hipStream_t s) {
+    if (mode == kSquared) return launch_scan<kSquared>(P, s);
+    return mode == kDistance ? launch_scan<kDistance>(P, s) : launch_scan<kField>(P, s);
+}
+
+int bits_of(int64_t v) {
+    int b = 0;
+    while (v >> b) ++b;
+    return b;
+}
+
+template <bool Y>
+hipError_t run_lines(const EdtLines &P, EdtOut mode, hipStream_t s) {
+    const dim3 grid((unsigned)((P.lines + kLineThreads - 1) / kLineThreads)), block(kLineThreads);
+    if constexpr (Y) {
+        hipLaunchKernelGGL((k_edt_lines<true, kSquared>), grid, block, 0, s, P);
+    } else {
+        if (mode == kSquared) hipLaunchKernelGGL((k_edt_lines<false, kSquared>), grid, block, 0, s, P);
+        else if (mode == kDistance) hipLaunchKernelGGL((k_edt_lines<false, kDistance>), grid, block, 0, s, P);
+        else hipLaunchKernelGGL((k_edt_lines<false, kField>), grid, block, 0, s, P);
+    }
     return hipGetLastError();
 }
 
@@ -601,21 +957,52 @@ int check_extents(const char *who, int64_t nz, int64_t ny, int64_t nx) {
 }
 
 // The three passes; the first reads `data` (sites: data == 0, or != 0 when
-// `invert`), the last writes `last_out` in `last_mode` (2: squared, 3: float
-// x cylinder + min/max into mm).
+// `invert`), the last writes `last_out` in `mode` (kField: x cylinder, and
+// min/max into mm).
 int device_edt_core(const uint8_t *data, int64_t nz, int64_t ny, int64_t nx, bool invert, uint32_t *a,
-                    uint32_t *b, uint32_t *last_out, int last_mode, const uint8_t *cyl, uint32_t *mm,
+                    uint32_t *b, uint32_t *last_out, EdtOut mode, const uint8_t *cyl, uint32_t *mm,
                     hipStream_t s) {
-    EdtPass py = pass_geom(1, nz, ny, nx), pz = pass_geom(0, nz, ny, nx);
-    py.in = a; py.out = b;
-    pz.in = b; pz.out = last_out; pz.cyl = cyl; pz.minmax = mm;
-    if (last_mode == 3) {
+    if (mode == kField) {
         hipLaunchKernelGGL(k_edt_minmax_init, dim3(1), dim3(64), 0, s, mm);
         MXB_EHIP(hipGetLastError());
     }
-    MXB_EHIP(run_rows(data, invert, nz * ny, nx, a, s));
-    MXB_EHIP(run_pass(false, py, s));
-    MXB_EHIP(run_pass(last_mode == 3, pz, s));
+    // A lane per line needs lines enough for the device, and is bound by the
+    // latency of its serial steps below that (129x300x257: along y, 33 K lines,
+    // 140 us against 95 for k_edt_pass; 400x333x417, 139 K lines along z, 920
+    // us for the whole field against 1458 scanning outward).  Along z, where
+    // after the y pass every plane with a site has values throughout, short
+    // lines that are not plenty scan outward (200^3: 104 us, k_edt_pass 240;
+    // 256^3: 378 us for the field, lanes 503; 500x250x250: 1002, k_edt_pass 689).
+    constexpr int64_t kLinesWanted = 65536, kLinesPlenty = 131072;
+    if (nz * nx >= kLinesWanted) {
+        // distances in the first half of `a`, the stacks in the second
+        uint16_t *const d = reinterpret_cast<uint16_t *>(a);
+        MXB_EHIP(run_rows(data, invert, nz * ny, nx, d, s));
+        const EdtLines P{d, d + nz * ny * nx, b, (int)ny, nx, nz * nx, nx, ny * nx, 0, nullptr, nullptr};
+        MXB_EHIP(run_lines<true>(P, kSquared, s));
+    } else {
+        EdtPass py = pass_geom(1, nz, ny, nx);
+        py.in = a; py.out = b;
+        MXB_EHIP(run_rows(data, invert, nz * ny, nx, a, s));
+        MXB_EHIP(run_pass(kSquared, py, s));
+    }
+    // a value and a position share 32 bits up to 1024-voxel axes
+    const int gbits = bits_of((nx - 1) * (nx - 1) + (ny - 1) * (ny - 1));
+#ifndef SZL
+#define SZL 100000
+#endif
+    const bool scan = nz <= kScanMax && ny * nx < kLinesPlenty;
+    if (!scan && ny * nx >= kLinesWanted && gbits + bits_of(nz - 1) <= 32) {
+        const EdtLines P{b, b, last_out, (int)nz, ny * nx, ny * nx, ny * nx, 0, gbits, cyl, mm};
+        MXB_EHIP(run_lines<false>(P, mode, s));
+    } else if (scan) {
+        const EdtLines P{b, nullptr, last_out, (int)nz, ny * nx, ny * nx, ny * nx, 0, 0, cyl, mm};
+        MXB_EHIP(run_scan(P, mode, s));
+    } else {
+        EdtPass pz = pass_geom(0, nz, ny, nx);
+        pz.in = b; pz.out = last_out; pz.cyl = cyl; pz.minmax = mm;
+        MXB_EHIP(run_pass(mode, pz, s));
+    }
     return OK;
 }
 
@@ -661,10 +1048,10 @@ int mxb_device_edt(const uint8_t *dev_data, int64_t nz, int64_t ny, int64_t nx, 
     uint32_t *a = (uint32_t *)dev_workspace;
     uint32_t *b = (uint32_t *)((char *)dev_workspace + vol_words_bytes(n));
     uint32_t *mm = (uint32_t *)((char *)dev_workspace + 2 * vol_words_bytes(n));
-    if (dev_sq_out != nullptr && (rc = device_edt_core(dev_data, nz, ny, nx, false, a, b, dev_sq_out, 2,
+    if (dev_sq_out != nullptr && (rc = device_edt_core(dev_data, nz, ny, nx, false, a, b, dev_sq_out, kSquared,
                                                        nullptr, mm, s)) != OK)
         return rc;
-    if (dev_out != nullptr && (rc = device_edt_core(dev_data, nz, ny, nx, false, a, b, (uint32_t *)dev_out, 3,
+    if (dev_out != nullptr && (rc = device_edt_core(dev_data, nz, ny, nx, false, a, b, (uint32_t *)dev_out, kDistance,
                                                     nullptr, mm, s)) != OK)
         return rc;
     return OK;
@@ -685,12 +1072,10 @@ int mxb_device_edt_field(const uint8_t *dev_implant_solid, int64_t nz, int64_t n
     uint32_t *b = (uint32_t *)((char *)dev_workspace + vol_words_bytes(n));
     uint32_t *mm = (uint32_t *)((char *)dev_workspace + 2 * vol_words_bytes(n));
     // 0950:41 negates the implant mask: the sites are the implant voxels
-    if ((rc = device_edt_core(dev_implant_solid, nz, ny, nx, true, a, b, a, 3, dev_cylinder, mm, s)) != OK)
+    if ((rc = device_edt_core(dev_implant_solid, nz, ny, nx, true, a, b, a, kField, dev_cylinder, mm, s)) != OK)
         return rc;
-    int64_t blocks = nz * ny * ((nx + 1023) / 1024);
-    if (blocks > 16384) blocks = 16384;
-    hipLaunchKernelGGL(k_edt_to_u16, dim3((unsigned)blocks), dim3(256), 0, s, (const float *)a, nz * ny, ny, nx,
-                       dev_cylinder, mm, dev_out);
+    const dim3 grid((unsigned)((ny * nx + 2047) / 2048), (unsigned)std::min<int64_t>(nz, 65535));
+    hipLaunchKernelGGL(k_edt_to_u16, grid, dim3(256), 0, s, (const float *)a, nz, ny * nx, dev_cylinder, mm, dev_out);
     MXB_EHIP(hipGetLastError());
     return OK;
 }

@@ -1,4 +1,5 @@
-// Bins of uint16 values and 16-byte chunk loads of the histogram kernels.
+// Arithmetic shared by the field consumers: bins of uint16 values, division by
+// a shared divisor, 16-byte chunk loads.
 #ifndef MXB_HIST_H
 #define MXB_HIST_H
 
@@ -46,6 +47,23 @@ __device__ __forceinline__ int bin_of(uint32_t v, const BinMap &m) {
     const bool ok = v - m.vlo <= m.vhi - m.vlo && t >= 0.0 && t < m.c + 1.0;
     return ok ? (int)t : -1;
 }
+
+// Float32 division of many values by one: the correctly rounded quotient from
+// the correctly rounded reciprocal and one residual (Markstein, as above),
+// where d is far from under- and overflow and its significand is not all
+// ones (`exact`); the dividends must be 0 or within 2^40 of d.
+struct SharedDiv {
+    float d, r;
+    bool exact;
+    __device__ __forceinline__ explicit SharedDiv(float divisor) : d(divisor), r(1.0f / divisor) {
+        const uint32_t b = __float_as_uint(d);
+        exact = d > 0x1p-40f && d < 0x1p40f && (b & 0x7fffffu) != 0x7fffffu;
+    }
+    __device__ __forceinline__ float quick(float x) const {
+        const float q = x * r;
+        return __builtin_fmaf(__builtin_fmaf(-q, d, x), r, q);
+    }
+};
 
 // Elements 8 c .. 8 c + 7 of `base` (16-byte aligned); those outside [b, e)
 // are not read and come back as 0.

@@ -137,3 +137,42 @@ def test_edt_field_large_host_copies(gpu):
     assert np.array_equal(host, dq.to_array(np.uint16, shape))
     for b in (dm, dc, dq, ws):
         b.free()
+
+
+# Enough lines for the lane-per-line passes (65536 along y, along z, or both),
+# ragged rows, one to four 1024-voxel pieces per row, value and position bits
+# that do and do not share a word.
+WIDE = [(300, 5, 257), (5, 300, 257), (270, 265, 250), (70, 9, 1030), (33, 40, 2500), (17, 23, 4096), (64, 1025, 65),
+        (1200, 70, 1000)]
+
+
+@pytest.mark.parametrize("case", range(len(WIDE)))
+@pytest.mark.parametrize("kind", ["sparse", "dense", "planes", "late"])
+def test_edt_many_lines(gpu, case, kind):
+    """Few and many sites, equal parabolas all along y and z (the stack holds
+    the whole line), and a near site after a long rise (it pops all of it)."""
+    shape = WIDE[case]
+    rng = np.random.default_rng(1100 + case)
+    data = np.ones(shape, bool)
+    if kind == "sparse":
+        data[rng.random(shape) < 2e-5] = False
+    elif kind == "dense":
+        data[rng.random(shape) < 0.05] = False
+    elif kind == "planes":
+        data[:, :, shape[2] // 3] = False
+    else:
+        y, z = np.meshgrid(np.arange(shape[1]), np.arange(shape[0]))
+        x = np.clip(shape[2] // 2 - (y + z) // 2, 0, shape[2] - 1)  # sites move off as y and z grow
+        data[z, y, x] = False
+        data[-1, -1, :] = False
+    data.flat[rng.integers(data.size)] = False
+    _say("edt many lines", shape, kind)
+    assert np.array_equal(edt.edt_sq(data).astype(np.uint64), E.edt_sq(data))
+    if kind == "sparse" and data.size < 20_000_000:
+        cyl = generate_cylinder_mask(shape[1], shape[2])
+        assert np.array_equal(edt.edt(data), E.edt(data))
+        assert np.array_equal(edt.generate_edt_field(~data, cyl), E.edt_field(~data, cyl))
+
+
+def test_edt_many_lines_without_sites(gpu):
+    assert np.all(edt.edt_sq(np.ones((260, 258, 256), bool)) == edt.EDT_NONE)
