@@ -683,18 +683,19 @@ __global__ __launch_bounds__(kLineThreads) void k_edt_lines(EdtLines P) {
 
 // ---- outward scan
 // With too few lines for a lane each, and short ones, every position looks
-// outward for its minimum: g[j] + (i - j)^2 cannot win once (i - j)^2 reaches
-// the best value found.  A block holds 64 neighbouring lines in LDS (a lane's
+// outward for its minimum: g[j] + (i - j)^2 cannot win once (i - j)^2 and the
+// line's least g reach the best value found.  A block holds 64 neighbouring lines in LDS (a lane's
 // line in its own bank); a thread answers 8 consecutive positions of a line
 // together, so a value read serves 8 of them with an addition and a minimum
 // each, the squares being uniform: from the left, at distance t from the
 // first position, g + t^2 + 2 t k + k^2 for position k, and mirrored from the
 // right.
-constexpr int kScanLines = 64, kScanMax = 256;  // 64 KB of LDS at most
+constexpr int kScanLines = 64, kScanMax = 512;  // 128 KB of LDS at most
 
 template <EdtOut OUT>
 __global__ __launch_bounds__(512) void k_edt_scan(EdtLines P) {
     extern __shared__ int32_t vals[];  // [n][kScanLines]
+    __shared__ int32_t least[kScanLines];
     constexpr int kFarValue = 1 << 29;
     const int n = P.n, lane = threadIdx.x & 63, waves = blockDim.x >> 6;
     const int64_t line = (int64_t)blockIdx.x * kScanLines + lane;
@@ -702,11 +703,18 @@ __global__ __launch_bounds__(512) void k_edt_scan(EdtLines P) {
     const int64_t run = live ? line / P.inner : 0;
     const int64_t base = live ? run * P.outer_stride + (line - run * P.inner) : 0;
     const uint32_t *const in = static_cast<const uint32_t *>(P.in) + base;
+    if (threadIdx.x < kScanLines) least[lane] = kFarValue;
+    __syncthreads();
+    int gmin = kFarValue;
     for (int j = threadIdx.x >> 6; j < n; j += waves) {
         const uint32_t g = live ? in[j * P.pos_stride] : kNone;
-        vals[j * kScanLines + lane] = g == kNone ? kFarValue : (int)g;
+        const int v = g == kNone ? kFarValue : (int)g;
+        vals[j * kScanLines + lane] = v;
+        gmin = min(gmin, v);
     }
+    atomicMin(&least[lane], gmin);
     __syncthreads();
+    gmin = least[lane];
     float cyl = 1.0f;
     if (OUT == kField && P.cyl != nullptr && live) cyl = P.cyl[line] != 0 ? 1.0f : 0.0f;
     uint32_t lo = 0xffffffffu, hi = 0;
@@ -727,7 +735,7 @@ __global__ __launch_bounds__(512) void k_edt_scan(EdtLines P) {
 #pragma unroll
             for (int k = 0; k < 8; ++k)
                 if (i0 + k < n) worst = max(worst, min(l[k] + k * k, r[k] + (7 - k) * (7 - k)));
-            if (__ballot(worst > t0 * t0) == 0) break;
+            if (__ballot(worst > gmin + t0 * t0) == 0) break;
             int a[4], b[4];
 #pragma unroll
             for (int u = 0; u < 4; ++u) {
@@ -971,8 +979,9 @@ int device_edt_core(const uint8_t *data, int64_t nz, int64_t ny, int64_t nx, boo
     // 140 us against 95 for k_edt_pass; 400x333x417, 139 K lines along z, 920
     // us for the whole field against 1458 scanning outward).  Along z, where
     // after the y pass every plane with a site has values throughout, short
-    // lines that are not plenty scan outward (200^3: 104 us, k_edt_pass 240;
-    // 256^3: 378 us for the field, lanes 503; 500x250x250: 1002, k_edt_pass 689).
+    // lines that are not plenty scan outward (200^3: 95 us, k_edt_pass 240;
+    // 256^3: 349 us for the field, lanes 503; 500x250x250: 599, k_edt_pass 690);
+    // along y, where most values are none, scanning is no faster.
     constexpr int64_t kLinesWanted = 65536, kLinesPlenty = 131072;
     if (nz * nx >= kLinesWanted) {
         // distances in the first half of `a`, the stacks in the second
