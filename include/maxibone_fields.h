@@ -33,9 +33,9 @@ int mxb_combine_fields(const uint16_t *gauss, const uint16_t *edt, int64_t nz, i
                        int64_t nx, const uint8_t *cylinder, uint16_t *out, int verbose);
 
 /* Device form: bytes of the workspace it needs (a few KB).  The passes are
- * enqueued on `stream`, and the call synchronises it twice (the host derives
- * each pass's parameters from the previous reductions); it returns with the
- * output written. */
+ * enqueued on `stream`, each reading the previous one's reductions from the
+ * workspace, and the call synchronises it at the end (a zero maximum is
+ * reported); it returns with the output written. */
 int64_t mxb_combine_workspace_bytes(void);
 int mxb_device_combine_fields(const uint16_t *dev_gauss, const uint16_t *dev_edt, int64_t nz,
                               int64_t ny, int64_t nx, const uint8_t *dev_cylinder,

@@ -1,7 +1,7 @@
-"""Histogram kernels at the sizes where their shapes change: ragged rows,
+"""Histogram and combination kernels at the sizes where their shapes change: ragged rows,
 volumes that start off a 16-byte boundary, table widths from 1 to the most
 bins, radii around the annulus edges, centres off the volume, and value ranges
-whose bin edges fall on whole numbers.  Counts equal the oracle's."""
+whose bin edges fall on whole numbers.  Counts and combined fields equal the oracle's."""
 import numpy as np
 import pytest
 
@@ -104,3 +104,30 @@ def test_field_histogram_at_edges(gpu, case):
     capi.check(L.mxb_device_field_histogram(dv.ptr, *vshape, df.ptr, *fshape, db.ptr, *nbins, *vrange, *frange,
                                             ws.ptr, None))
     assert np.array_equal(db.to_array(np.uint64, nbins), want)
+
+
+COMBINE = [  # shape, byte shift of the fields, cylinder: None, "all", "none", "disc", "random"
+    ((1, 1, 2), 0, None), ((3, 5, 7), 2, "random"), ((70, 9, 11), 0, "disc"), ((2, 33, 64), 6, "none"),
+    ((5, 40, 64), 0, "all"), ((4, 200, 211), 2, "disc"), ((300, 16, 128), 0, "random"),
+]
+
+
+@pytest.mark.parametrize("case", range(len(COMBINE)))
+def test_combine_at_edges(gpu, case):
+    shape, shift, kind = COMBINE[case]
+    print("combine", COMBINE[case], flush=True)
+    rng = np.random.default_rng(980 + case)
+    g = rng.integers(0, 60000, shape, dtype=np.uint16)
+    e = rng.integers(0, 65536, shape, dtype=np.uint16)
+    g.flat[0], e.flat[0], g.flat[-1], e.flat[-1] = 59999, 0, 0, 65535
+    cyl = {None: None, "all": np.ones(shape[1:], bool), "none": np.zeros(shape[1:], bool),
+           "disc": (np.add.outer((np.arange(shape[1]) - shape[1] / 2) ** 2, (np.arange(shape[2]) - shape[2] / 2) ** 2)
+                    < (min(shape[1:]) / 2) ** 2), "random": rng.random(shape[1:]) > 0.5}[kind]
+    want = F.combine_fields(g, e, np.ones(shape[1:], bool) if cyl is None else cyl)
+    L = capi.lib()
+    dg, de, out = _at(g, shift), _at(e, shift), hip.DeviceBuffer(g.nbytes + 64)
+    dc = None if cyl is None else hip.DeviceBuffer.from_array(cyl.astype(np.uint8))
+    ws = hip.DeviceBuffer(L.mxb_combine_workspace_bytes())
+    capi.check(L.mxb_device_combine_fields(dg.ptr + shift, de.ptr + shift, *shape, None if dc is None else dc.ptr,
+                                           out.ptr, ws.ptr, None))
+    assert np.array_equal(out.to_array(np.uint16, shape), want)
