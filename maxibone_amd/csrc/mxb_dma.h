@@ -78,6 +78,17 @@ __device__ __forceinline__ void store16(float *p, v4f32 v) {
         *q = v;
 }
 
+// The same for an address aligned to its elements only (one store
+// instruction all the same: global accesses need no more).
+typedef v4u32 __attribute__((aligned(2))) v4u32_a2;
+typedef v4f32 __attribute__((aligned(4))) v4f32_a4;
+__device__ __forceinline__ void store16_any(uint16_t *p, uint4 v) {
+    *(__attribute__((address_space(1))) v4u32_a2 *)p = v4u32{v.x, v.y, v.z, v.w};
+}
+__device__ __forceinline__ void store16_any(float *p, v4f32 v) {
+    *(__attribute__((address_space(1))) v4f32_a4 *)p = v;
+}
+
 // LDS byte address of a __shared__ object.
 __device__ __forceinline__ uint32_t lds_addr(const void *p) {
     return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) void *)p;

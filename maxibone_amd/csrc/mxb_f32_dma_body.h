@@ -47,6 +47,31 @@ constexpr int kF32StagePitchV = 36;      // floats per line row (position-contig
 // row groups one MFMA result writes (4 kg + r) in distinct 16-bank groups
 constexpr int kF32StagePitchZ = 68;
 
+// ANY: rows of any 4-byte alignment and any number of lines from 64 on.  The
+// last group then starts at n_lane - 64, so that every group is whole: the
+// lines it shares with the group before are computed twice, to the same bits.
+// FP32, sigma 4, 10 repetitions: 257x331x403 5.73 -> 2.55 ms (the register-ring
+// form's 64-byte pieces: 175 us per pass), 257x331x404 3.30 -> 2.41 (the
+// VGPR-staged form), against 2.01 for 257x328x400 with 16-byte loads.
+template <bool ANY>
+__device__ __forceinline__ int64_t f32_first_line(int64_t lb, int64_t n_lane) {
+    const int64_t l = lb * 64;
+    return ANY && l + 64 > n_lane ? n_lane - 64 : l;
+}
+
+// ANY: a wave's four rows of a slot, positions p0 .. p0 + 3, in four loads of
+// 4 bytes per lane (a 16-byte load needs a 16-byte-aligned address): lane i
+// of row r fetches the line that the rotated row holds at column i.
+__device__ __forceinline__ void f32_dma_rows(const float *__restrict__ lines, int64_t in_ax_b, int64_t p0,
+                                             int64_t n_ax, bool wanted, int lane, uint32_t lds) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        const char *const src = reinterpret_cast<const char *>(lines + ((lane - 16 * r) & 63)) + (p0 + r) * in_ax_b;
+        const bool ok = wanted && p0 + r >= 0 && p0 + r < n_ax;
+        dma4(lds + 256u * (uint32_t)r, ok ? static_cast<const void *>(src) : static_cast<const void *>(g_dma_zero));
+    }
+}
+
 // Shared-memory layout of one block of the one-tile pass (bytes):
 // [ring | stage | tap table].
 template <int RT, int D, bool MASK, bool ZSTAGE>
@@ -63,7 +88,7 @@ struct F32DmaSmem {
 // `outer`, positions of segment `seg_id`; `taps` holds the 2RT+1 centred taps
 // (any address space).  Returns with the wave's loads and stores drained and
 // every thread past a final barrier, so the caller may reuse `smem` at once.
-template <int RT, int D, bool MASK, bool OUTF, bool OUTU, bool ZSTAGE, typename TapSrc>
+template <int RT, int D, bool MASK, bool OUTF, bool OUTU, bool ZSTAGE, bool ANY = false, typename TapSrc>
 __device__ __forceinline__ void f32_dma_body(const float *__restrict__ in, const LineGeom &g,
                                              const Epilogue &e, int64_t outer, int64_t lb,
                                              int64_t seg_id, const TapSrc &taps,
@@ -77,6 +102,7 @@ __device__ __forceinline__ void f32_dma_body(const float *__restrict__ in, const
     static_assert(!MASK, "the illuminating pass runs on f32_dma_body2 (mask bits)");
     static_assert(!ZSTAGE || (OUTF && !OUTU && !MASK), "line-contiguous epilogue writes floats only");
     static_assert(ST >= 1, "at least one output");
+    constexpr int GL = ANY ? 4 : 1;  // loads per slot and wave
     using M = F32DmaSmem<RT, D, MASK, ZSTAGE>;
     constexpr int TAPS = M::TAPS / 4;
     float *const ring = reinterpret_cast<float *>(smem);
@@ -87,7 +113,7 @@ __device__ __forceinline__ void f32_dma_body(const float *__restrict__ in, const
     const int lane = tid & 63;
     const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int col = lane & 15, kg = lane >> 4;
-    const int64_t line0 = lb * 64;
+    const int64_t line0 = f32_first_line<ANY>(lb, g.n_lane);
     const int64_t a0 = seg_id * g.seg;
     const int64_t a1 = a0 + g.seg < g.n_ax ? a0 + g.seg : g.n_ax;
     const int64_t n_ax = g.n_ax;
@@ -108,6 +134,11 @@ __device__ __forceinline__ void f32_dma_body(const float *__restrict__ in, const
     const int64_t pos_first = a0 - RT;
     const uint32_t ring_lds = lds_addr(ring) + 1024u * (uint32_t)wv;
     auto issue_data = [&](int slot) {
+        if constexpr (ANY) {
+            f32_dma_rows(in + outer * g.in_outer + line0, in_ax_b, pos_first + 16 * (int64_t)slot + 4 * wv, n_ax,
+                         slot < nslots, lane, ring_lds + (uint32_t)((slot % NSL) * kF32Slot * 4));
+            return;
+        }
         const int64_t p = pos_first + 16 * (int64_t)slot + dr;
         const bool ok = dl_ok && slot < nslots && p >= 0 && p < n_ax;
         const void *src = ok ? static_cast<const void *>(dsrc + p * in_ax_b)
@@ -135,9 +166,9 @@ __device__ __forceinline__ void f32_dma_body(const float *__restrict__ in, const
 
     for (int j = 0; j < ntiles; ++j) {
         if (j >= D)
-            vm_wait<(D - 1) + (ZSTAGE ? D : D / 2) * ST>();
+            vm_wait<GL * (D - 1) + (ZSTAGE ? D : D / 2) * ST>();
         else
-            vm_wait<D - 1>();
+            vm_wait<GL * (D - 1)>();
         __syncthreads();
         issue_group(j + D);
         int sb[W];
@@ -161,12 +192,14 @@ __device__ __forceinline__ void f32_dma_body(const float *__restrict__ in, const
             const int64_t p = tpos + zr;
             float *op = e.out_f32 + outer * g.out_outer + p * g.out_ax + line0 + 4 * zq;
             if (full) {
-                if (nt_rows_ok(e.out_f32, 4 * g.out_outer))
+                if (ANY)
+                    store16_any(op, v);
+                else if (nt_rows_ok(e.out_f32, 4 * g.out_outer))
                     store16<true>(zq_ok ? op : sinkf, v);
                 else
                     store16<false>(zq_ok ? op : sinkf, v);
             } else if (zq_ok && p < a1) {
-                store16<false>(op, v);
+                store16_any(op, v);
             }
         } else {
             const int half = j & 1;
@@ -184,8 +217,8 @@ __device__ __forceinline__ void f32_dma_body(const float *__restrict__ in, const
                 if (pfull && half == 1) {
                     if (OUTF) {
                         float *dst = sl_ok ? e.out_f32 + off : sinkf;
-                        store16<false>(dst, v[0]);
-                        store16<false>(dst + (sl_ok ? 4 : 0), v[1]);
+                        store16_any(dst, v[0]);
+                        store16_any(dst + (sl_ok ? 4 : 0), v[1]);
                     }
                     if (OUTU) {
                         uint32_t w[4];
@@ -194,7 +227,7 @@ __device__ __forceinline__ void f32_dma_body(const float *__restrict__ in, const
                             w[2 * h] = (uint32_t)quantise_u16_l(v[h][0]) | ((uint32_t)quantise_u16_l(v[h][1]) << 16);
                             w[2 * h + 1] = (uint32_t)quantise_u16_l(v[h][2]) | ((uint32_t)quantise_u16_l(v[h][3]) << 16);
                         }
-                        store16<false>(sl_ok ? e.out_u16 + off : sinku, make_uint4(w[0], w[1], w[2], w[3]));
+                        store16_any(sl_ok ? e.out_u16 + off : sinku, make_uint4(w[0], w[1], w[2], w[3]));
                     }
                 } else if (sl_ok) {
                     // a segment's last (partial or unpaired) tiles
@@ -246,7 +279,7 @@ struct F32Dma2Smem {
     static constexpr int BYTES = RING + MRING + STAGE + TAPS;
 };
 
-template <int RT, int D, bool MASK, bool OUTF, bool OUTU, bool ZSTAGE, typename TapSrc>
+template <int RT, int D, bool MASK, bool OUTF, bool OUTU, bool ZSTAGE, bool ANY = false, typename TapSrc>
 __device__ __forceinline__ void f32_dma_body2(const float *__restrict__ in, const LineGeom &g,
                                               const Epilogue &e, int64_t outer, int64_t lb,
                                               int64_t seg_id, const TapSrc &taps,
@@ -255,7 +288,8 @@ __device__ __forceinline__ void f32_dma_body2(const float *__restrict__ in, cons
     constexpr int C = S::C, W = S::W, NSL = S::NSL;
     // loads issued in D - 1 groups: 2 data slots each, and (with (D - 1) % 4
     // == 0) exactly (D - 1) / 4 mask loads (one per 4 pairs)
-    constexpr int GW = 2 * (D - 1) + (MASK ? (D - 1) / 4 : 0);
+    constexpr int GL = ANY ? 4 : 1;  // loads per slot and wave
+    constexpr int GW = 2 * GL * (D - 1) + (MASK ? (D - 1) / 4 : 0);
     static_assert(!MASK || (D - 1) % 4 == 0, "a fixed count of mask loads per D - 1 groups");
     constexpr int NM4 = F32Dma2Smem<RT, D, MASK, ZSTAGE>::NM4;
     constexpr int ST = ZSTAGE ? 2 : (OUTF ? 2 : 0) + (OUTU ? 1 : 0);
@@ -272,7 +306,7 @@ __device__ __forceinline__ void f32_dma_body2(const float *__restrict__ in, cons
     const int lane = tid & 63;
     const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int col = lane & 15, kg = lane >> 4;
-    const int64_t line0 = lb * 64;
+    const int64_t line0 = f32_first_line<ANY>(lb, g.n_lane);
     const int64_t a0 = seg_id * g.seg;
     const int64_t a1 = a0 + g.seg < g.n_ax ? a0 + g.seg : g.n_ax;
     const int64_t n_ax = g.n_ax;
@@ -293,6 +327,11 @@ __device__ __forceinline__ void f32_dma_body2(const float *__restrict__ in, cons
     const int64_t pos_first = a0 - RT;
     const uint32_t ring_lds = lds_addr(ring) + 1024u * (uint32_t)wv;
     auto issue_data = [&](int slot) {
+        if constexpr (ANY) {
+            f32_dma_rows(in + outer * g.in_outer + line0, in_ax_b, pos_first + 16 * (int64_t)slot + 4 * wv, n_ax,
+                         slot < nslots, lane, ring_lds + (uint32_t)((slot % NSL) * kF32Slot * 4));
+            return;
+        }
         const int64_t p = pos_first + 16 * (int64_t)slot + dr;
         const bool ok = dl_ok && slot < nslots && p >= 0 && p < n_ax;
         const void *src = ok ? static_cast<const void *>(dsrc + p * in_ax_b)
@@ -373,12 +412,14 @@ __device__ __forceinline__ void f32_dma_body2(const float *__restrict__ in, cons
                 const int64_t p = ppos + row;
                 float *op = e.out_f32 + outer * g.out_outer + p * g.out_ax + line0 + 4 * zq;
                 if (full) {
-                    if (nt_rows_ok(e.out_f32, 4 * g.out_outer))
+                    if (ANY)
+                        store16_any(op, v);
+                    else if (nt_rows_ok(e.out_f32, 4 * g.out_outer))
                         store16<true>(zq_ok ? op : sinkf, v);
                     else
                         store16<false>(zq_ok ? op : sinkf, v);
                 } else if (zq_ok && p < a1) {
-                    store16<false>(op, v);
+                    store16_any(op, v);
                 }
             }
         } else {
@@ -404,8 +445,8 @@ __device__ __forceinline__ void f32_dma_body2(const float *__restrict__ in, cons
                 }
                 if (OUTF) {
                     float *dst = sl_ok ? e.out_f32 + off : sinkf;
-                    store16<false>(dst, v[0]);
-                    store16<false>(dst + (sl_ok ? 4 : 0), v[1]);
+                    store16_any(dst, v[0]);
+                    store16_any(dst + (sl_ok ? 4 : 0), v[1]);
                 }
                 if (OUTU) {
                     uint32_t w[4];
@@ -414,7 +455,7 @@ __device__ __forceinline__ void f32_dma_body2(const float *__restrict__ in, cons
                         w[2 * h] = (uint32_t)quantise_u16_l(v[h][0]) | ((uint32_t)quantise_u16_l(v[h][1]) << 16);
                         w[2 * h + 1] = (uint32_t)quantise_u16_l(v[h][2]) | ((uint32_t)quantise_u16_l(v[h][3]) << 16);
                     }
-                    store16<false>(sl_ok ? e.out_u16 + off : sinku, make_uint4(w[0], w[1], w[2], w[3]));
+                    store16_any(sl_ok ? e.out_u16 + off : sinku, make_uint4(w[0], w[1], w[2], w[3]));
                 }
             } else if (sl_ok) {
 #pragma unroll
@@ -447,15 +488,15 @@ struct F32DmaForm {
     static constexpr int BYTES = bytes();
 };
 
-template <int RT, int D, bool MASK, bool OUTF, bool OUTU, bool ZSTAGE, typename TapSrc>
+template <int RT, int D, bool MASK, bool OUTF, bool OUTU, bool ZSTAGE, bool ANY = false, typename TapSrc>
 __device__ __forceinline__ void f32_dma_pass(const float *__restrict__ in, const LineGeom &g,
                                              const Epilogue &e, int64_t outer, int64_t lb,
                                              int64_t seg_id, const TapSrc &taps, unsigned char *smem) {
     if constexpr (ZSTAGE)
-        f32_dma_body<RT, D, MASK, OUTF, OUTU, ZSTAGE>(in, g, e, outer, lb, seg_id, taps, smem);
+        f32_dma_body<RT, D, MASK, OUTF, OUTU, ZSTAGE, ANY>(in, g, e, outer, lb, seg_id, taps, smem);
     else
-        f32_dma_body2<RT, MASK ? MXB_F32_DEPTH_X : MXB_F32_DEPTH_Y, MASK, OUTF, OUTU, ZSTAGE>(in, g, e, outer, lb,
-                                                                                           seg_id, taps, smem);
+        f32_dma_body2<RT, MASK ? MXB_F32_DEPTH_X : MXB_F32_DEPTH_Y, MASK, OUTF, OUTU, ZSTAGE, ANY>(
+            in, g, e, outer, lb, seg_id, taps, smem);
 }
 
 }  // namespace mxb

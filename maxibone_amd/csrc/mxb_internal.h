@@ -96,8 +96,8 @@ hipError_t launch_quantise(const float *u, uint16_t *q, float *f, int64_t n, hip
 hipError_t launch_mask_from_state(const float *u, uint8_t *m, int64_t n, hipStream_t s);
 
 // LDS-staged FP32 MFMA pass (mxb_kernels_f32_lds.hip): 16-byte loads of whole
-// rows; needs 16-byte-aligned input rows.
-bool lds_pass_supported(const float *in, const LineGeom &g, int R);
+// rows where they are 16-byte aligned, else 4-byte ones (64 lines or more).
+bool lds_pass_supported(const float *in, const LineGeom &g, const Epilogue &e, int R);
 hipError_t launch_line_pass_f32_lds(const float *in, const LineGeom &g, const Epilogue &e,
                                     const float *taps, int R, hipStream_t s);
 

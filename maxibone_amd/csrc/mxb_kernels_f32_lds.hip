@@ -18,7 +18,7 @@ __global__ __launch_bounds__(256) void k_line_mfma_lds(const float *__restrict__
     lds_line_body<RT>(in, g, e, outer, lb, seg_id, smem);
 }
 
-template <int RT, int D, bool MASK, bool OUTF, bool OUTU, bool ZSTAGE>
+template <int RT, int D, bool MASK, bool OUTF, bool OUTU, bool ZSTAGE, bool ANY>
 __global__ __launch_bounds__(256) void k_line_f32_dma(const float *__restrict__ in, LineGeom g,
                                                       Epilogue e, TapsF<2 * RT + 1> taps) {
     __shared__ __attribute__((aligned(16))) unsigned char smem[F32DmaForm<RT, D, MASK, ZSTAGE>::BYTES];
@@ -28,12 +28,21 @@ __global__ __launch_bounds__(256) void k_line_f32_dma(const float *__restrict__ 
     const int64_t nlb = (g.n_lane + 63) >> 6;
     const int64_t lb = bid % nlb;
     const int64_t outer = bid / nlb;
-    f32_dma_pass<RT, D, MASK, OUTF, OUTU, ZSTAGE>(in, g, e, outer, lb, seg_id, taps.k, smem);
+    f32_dma_pass<RT, D, MASK, OUTF, OUTU, ZSTAGE, ANY>(in, g, e, outer, lb, seg_id, taps.k, smem);
 }
 
-// Which direct-load epilogue serves (g, e): 0 none (use the VGPR-staged
-// form), else a code for the template below.
-static int f32_dma_form(const LineGeom &g, const Epilogue &e) {
+// Which direct-load epilogue serves (g, e): 0 none, else a code for the
+// template below.  `any`: the form with 4-byte loads, which takes any rows and
+// any number of lines from 64 on; else 16-byte loads and stores.
+static int f32_dma_form(const float *in, const LineGeom &g, const Epilogue &e, bool any) {
+    if (any) {
+        const bool f = e.out_f32 != nullptr, u = e.out_u16 != nullptr, m = e.mask != nullptr;
+        if (g.n_lane < 64) return 0;
+        if (g.out_lane == 1 && !m && !u && f) return 1;
+        if (g.out_ax != 1 || (m && e.bits.w == nullptr)) return 0;
+        return 2 + (m ? 4 : 0) + (f ? 1 : 0) + (u ? 2 : 0);
+    }
+    if (g.in_outer % 4 != 0 || g.in_ax % 4 != 0 || reinterpret_cast<uintptr_t>(in) % 16 != 0) return 0;
     if (g.n_lane % 4 != 0) return 0;
     const bool f = e.out_f32 != nullptr, u = e.out_u16 != nullptr, m = e.mask != nullptr;
     if (f && reinterpret_cast<uintptr_t>(e.out_f32) % 16 != 0) return 0;
@@ -44,22 +53,26 @@ static int f32_dma_form(const LineGeom &g, const Epilogue &e) {
     return 2 + (m ? 4 : 0) + (f ? 1 : 0) + (u ? 2 : 0);
 }
 
-template <int RT>
+template <int RT, bool ANY>
 static hipError_t launch_f32_dma_rt(int form, const float *in, LineGeom g, const Epilogue &e,
                                     const TapsF<2 * RT + 1> &t, hipStream_t s) {
     constexpr int D = MXB_F32_DMA_DEPTH;
     const dim3 grid((unsigned)(g.nseg * ((g.n_lane + 63) / 64) * g.n_outer)), block(256);
     switch (form) {
-    case 1: hipLaunchKernelGGL((k_line_f32_dma<RT, D, false, true, false, true>), grid, block, 0, s, in, g, e, t); break;
-    case 3: hipLaunchKernelGGL((k_line_f32_dma<RT, D, false, true, false, false>), grid, block, 0, s, in, g, e, t); break;
-    case 4: hipLaunchKernelGGL((k_line_f32_dma<RT, D, false, false, true, false>), grid, block, 0, s, in, g, e, t); break;
-    case 5: hipLaunchKernelGGL((k_line_f32_dma<RT, D, false, true, true, false>), grid, block, 0, s, in, g, e, t); break;
-    case 7: hipLaunchKernelGGL((k_line_f32_dma<RT, D, true, true, false, false>), grid, block, 0, s, in, g, e, t); break;
-    case 8: hipLaunchKernelGGL((k_line_f32_dma<RT, D, true, false, true, false>), grid, block, 0, s, in, g, e, t); break;
-    case 9: hipLaunchKernelGGL((k_line_f32_dma<RT, D, true, true, true, false>), grid, block, 0, s, in, g, e, t); break;
+    case 1: hipLaunchKernelGGL((k_line_f32_dma<RT, D, false, true, false, true, ANY>), grid, block, 0, s, in, g, e, t); break;
+    case 3: hipLaunchKernelGGL((k_line_f32_dma<RT, D, false, true, false, false, ANY>), grid, block, 0, s, in, g, e, t); break;
+    case 4: hipLaunchKernelGGL((k_line_f32_dma<RT, D, false, false, true, false, ANY>), grid, block, 0, s, in, g, e, t); break;
+    case 5: hipLaunchKernelGGL((k_line_f32_dma<RT, D, false, true, true, false, ANY>), grid, block, 0, s, in, g, e, t); break;
+    case 7: hipLaunchKernelGGL((k_line_f32_dma<RT, D, true, true, false, false, ANY>), grid, block, 0, s, in, g, e, t); break;
+    case 8: hipLaunchKernelGGL((k_line_f32_dma<RT, D, true, false, true, false, ANY>), grid, block, 0, s, in, g, e, t); break;
+    case 9: hipLaunchKernelGGL((k_line_f32_dma<RT, D, true, true, true, false, ANY>), grid, block, 0, s, in, g, e, t); break;
     default: return hipErrorInvalidValue;
     }
     return hipGetLastError();
+}
+
+static bool rows_aligned(const float *in, const LineGeom &g) {
+    return g.in_outer % 4 == 0 && g.in_ax % 4 == 0 && reinterpret_cast<uintptr_t>(in) % 16 == 0;
 }
 
 template <int RT>
@@ -97,17 +110,19 @@ static hipError_t launch_lds_rt(const float *in, LineGeom g, const Epilogue &e, 
     const int64_t blocks = g.nseg * groups;
     if (blocks == 0) return hipSuccess;
     const TapsF<2 * RT + 1> t = centred_taps_l<RT>(k, R);
-    const int form = force_vgpr_staging() ? 0 : f32_dma_form(g, e);
-    if (form != 0) return launch_f32_dma_rt<RT>(form, in, g, e, t, s);
+    if (!force_vgpr_staging()) {
+        if (const int form = f32_dma_form(in, g, e, false)) return launch_f32_dma_rt<RT, false>(form, in, g, e, t, s);
+        if (const int form = f32_dma_form(in, g, e, true)) return launch_f32_dma_rt<RT, true>(form, in, g, e, t, s);
+    }
+    if (!rows_aligned(in, g)) return hipErrorNotSupported;
     hipLaunchKernelGGL((k_line_mfma_lds<RT>), dim3((unsigned)blocks), dim3(256), 0, s, in, g, e, t);
     return hipGetLastError();
 }
 
-// Usable when every input row is 16-byte aligned (in_outer, in_ax multiples of
-// 4 floats) and the radius is compiled.
-bool lds_pass_supported(const float *in, const LineGeom &g, int R) {
-    return R <= 64 && g.in_outer % 4 == 0 && g.in_ax % 4 == 0 &&
-           reinterpret_cast<uintptr_t>(in) % 16 == 0;
+// Usable when the radius is compiled and either every input row is 16-byte
+// aligned or the direct-load form with 4-byte loads serves.
+bool lds_pass_supported(const float *in, const LineGeom &g, const Epilogue &e, int R) {
+    return R <= 64 && (rows_aligned(in, g) || (!force_vgpr_staging() && f32_dma_form(in, g, e, true) != 0));
 }
 
 hipError_t launch_line_pass_f32_lds(const float *in, const LineGeom &g, const Epilogue &e,
