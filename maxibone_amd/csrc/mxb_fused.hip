@@ -8,8 +8,14 @@
 // reference's z, y, x (src/lib/cpp/cpu/diffusion.cc:314-320), with its own
 // rounding; illumination (cpu:295-302) follows the last pass, as there.
 //
+// Two kernels: k_xy_pair marches along y in steps of 32 rows and serves every
+// radius bucket up to 48 on planes that 32-bit offsets span; k_xy_fused marches
+// in steps of 16 rows and serves the rest (bucket 64, whose staging of 32 rows
+// does not fit the LDS, and planes or rows beyond the offsets).  Both produce
+// the same values bit for bit.
+//
 // Block = 512 threads (8 waves) on plane z, output columns [x0, x0 + TX) and
-// output rows [ya, yb).  It marches along y in steps of 16 rows:
+// output rows [ya, yb).  k_xy_fused's steps:
 //   1. direct loads bring input rows ya - RT + 16 j .. +15, columns
 //      [x0 - HALO, x0 + TX + HALO), into a staging buffer (D + 1 buffers:
 //      steps j + 1 .. j + D load while step j computes); pieces outside the
@@ -619,6 +625,391 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(SPLIT ? 1 :
     vm_wait<0>();
 }
 
+// ---------------------------------------------------------------- 32-row steps
+// The same pass in steps of 32 rows (a whole ring slot).
+//
+// Bound: neither memory (4.1 TB/s of the copy's 5.6 at 1024^3, R = 40) nor one
+// unit: MFMA 0.5 ms, vector instructions 0.55 ms and LDS 0.75 ms of 2.1, one
+// after the other within a wave, with the waves of a block in phase.  So the
+// step count and the chains inside a step are what is cut here:
+// * a pair costs two block barriers instead of three, and each wave's x-pass
+//   runs two column tiles whose MFMA chains overlap and share C + 1 operand
+//   reads;
+// * the y-pass takes the data as the first MFMA operand, so a lane ends with
+//   four columns of one row and stages them in one 8-byte write (16-byte for
+//   FP32) instead of four;
+// * loads and stores are buffer operations on the plane: offsets are 32 bits
+//   and advance by one addition per step, and what falls outside the plane
+//   (rows before or after it wrap to, or pass, the end; pieces beyond a row or
+//   the radius are sent there) reads zeros or is not stored, without selects
+//   and zero or sink pointers.
+// One step is prefetched.  The epilogue is the wave epilogue, staged in the
+// staging buffer its own step has consumed (every wave is past the y-pass
+// barrier, and the buffer is refilled after the next step's first barrier).
+//
+// Measured, 16-row steps -> 32-row steps: split form 1024^3 sigma 10 2.40 ->
+// 2.13 ms a pass, 128^3 225 -> 200 us for ten repetitions, 512^3 sigma 3 3155 ->
+// 2911 us for six; BF16 512^3 sigma 3 1805 -> 1693, 128^3 191 -> 157 us.
+template <int RT, int TX, bool SPLIT, int FIN>
+struct XYPair {
+    static constexpr int NW = kXYWaves;
+    static constexpr int P = SPLIT ? 2 : 1;
+    static constexpr int C = LowpChunks<RT>::C;
+    static constexpr int W = C + 1;
+    static constexpr int HALO = 64;
+    static constexpr int ROWH = TX + 2 * HALO;
+    static constexpr int PR = ROWH / 8;
+    static constexpr int HB = 16 * ROWH * 2;          // staging bytes per plane and 16 rows
+    static constexpr int SB = 2 * HB;                 // per plane and step
+    static constexpr int NI = 32 * PR / (64 * NW);    // direct loads per wave, plane and step
+    static constexpr int NSUB = TX / 64;
+    static constexpr int SLOT = NSUB * kSlotBytes;
+    static constexpr int MW = TX / 32;
+    static constexpr int MHALF = MW * 64 > 256 ? MW * 64 : 256;
+    static constexpr int MLOADS = (MW + 3) / 4;       // waves loading mask words per 16 rows
+    static constexpr int MSLOT = 2 * MHALF;
+    static constexpr int PLO = (HALO - (RT + 7) / 8 * 8) / 8;
+    static constexpr int STAGE = 2 * P * SB;
+    static constexpr int RING = W * P * SLOT;
+    static constexpr int WP16 = 48, WPF = 80;         // wave stage pitches, 16-bit and FP32 (bytes)
+    static constexpr int WEST = 32 * (FIN != 0 ? WPF : P * WP16);
+    static constexpr int MRING = 2 * MSLOT;
+    static constexpr int TAPS = 2 * LowpChunks<RT>::TW * 2;
+    static constexpr int BYTES = STAGE + RING + MRING + TAPS;
+    static constexpr int ST = FIN != 0 ? ((FIN & 1) ? 2 : 0) + ((FIN & 2) ? 1 : 0) : P;  // stores per lane and pair
+    static_assert(TX == 16 * NW && MLOADS * 2 <= NW && (32 * PR) % (64 * NW) == 0, "one column tile per wave");
+    static_assert(NW * WEST <= P * SB, "the wave stages fit the consumed staging buffer");
+    // the last tile's last chunk stays inside the staged row
+    static constexpr bool FITS = RT <= HALO && HALO - RT + TX + 32 * C - 16 <= ROWH && BYTES <= 160 * 1024 - 512;
+};
+
+typedef uint32_t v4u __attribute__((ext_vector_type(4)));
+
+// Buffer over [p, p + bytes): raw 32-bit byte offsets, those at or beyond
+// `bytes` read zeros and store nothing.  Uniform.
+__device__ __forceinline__ v4u raw_buffer(const void *p, uint32_t bytes) {
+    const uint64_t a = reinterpret_cast<uint64_t>(p);
+    return v4u{(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)a),
+               (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(a >> 32)) & 0xffffu,
+               (uint32_t)__builtin_amdgcn_readfirstlane((int)bytes), 0x00020000u};
+}
+
+// dma16 / dma4 from a buffer.
+__device__ __forceinline__ void dma16_buf(uint32_t lds_wave_base, v4u buf, uint32_t off) {
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"
+                 :
+                 : "s"(lds_wave_base), "v"(off), "s"(buf)
+                 : "memory", "m0");
+#pragma clang diagnostic pop
+}
+__device__ __forceinline__ void dma4_buf(uint32_t lds_wave_base, v4u buf, uint32_t off) {
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dword %1, %2, 0 offen lds"
+                 :
+                 : "s"(lds_wave_base), "v"(off), "s"(buf)
+                 : "memory", "m0");
+#pragma clang diagnostic pop
+}
+__device__ __forceinline__ void store16_buf(void *plane, uint32_t bytes, uint32_t off, v4u v) {
+    __builtin_amdgcn_raw_buffer_store_b128(v, __builtin_amdgcn_make_buffer_rsrc(plane, 0, (int)bytes, 0x00020000),
+                                           (int)off, 0, 0);
+}
+
+template <int RT, int TX, bool BF, bool SPLIT, int FIN>
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(SPLIT ? 1 : 4))) void k_xy_pair(
+    const uint16_t *__restrict__ in, uint16_t *__restrict__ out, const uint32_t *__restrict__ bits, XYGeom g,
+    TapsL<2 * RT + 1> taps, SplitIO io) {
+    using S = XYPair<RT, TX, SPLIT, FIN>;
+    using L = Lowp<BF>;
+    constexpr int C = S::C, W = S::W, PR = S::PR, SB = S::SB, HB = S::HB, NI = S::NI, NW = S::NW;
+    constexpr int SLOT = S::SLOT, MSLOT = S::MSLOT, MHALF = S::MHALF, P = S::P;
+    constexpr int TW = LowpChunks<RT>::TW;
+    static_assert(!SPLIT || !BF, "the split form runs on FP16 MFMAs");
+    static_assert(S::FITS, "shape fits the LDS");
+    __shared__ __attribute__((aligned(16))) unsigned char smem[S::BYTES];
+    unsigned char *const staging = smem;
+    unsigned char *const ring = smem + S::STAGE;
+    unsigned char *const mring = ring + S::RING;
+    uint16_t *const thi = reinterpret_cast<uint16_t *>(mring + S::MRING);
+    uint16_t *const tlo = thi + TW;
+
+    const int tid = threadIdx.x;
+    const int lane = tid & 63;
+    const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int col = lane & 15, kg = lane >> 4;
+
+    int64_t tile = xcd_tile(blockIdx.x, gridDim.x);
+    const int64_t strip = tile % g.nstrip;
+    tile /= g.nstrip;
+    const int seg = (int)(tile % g.nseg);
+    const int64_t z = tile / g.nseg;
+    const int ny = (int)g.ny, nx = (int)g.nx;  // a plane is below 2^28 voxels
+    const int x0 = (int)strip * TX;
+    const int ya = seg * (int)g.seg;
+    const int yb = ya + (int)g.seg < ny ? ya + (int)g.seg : ny;
+    const int npairs = (yb - ya + 31) / 32;
+    const int nsteps = npairs + W - 1;
+    const int64_t plane = g.ny * g.nx;
+    const uint32_t pbytes = 2u * (uint32_t)plane;
+    constexpr uint32_t kOutside = 0x80000000u;  // beyond any plane, also after every step's advance
+
+    lowp_fill_taps<RT>(thi, tlo, taps);
+
+    // ---- step loads: lane slot (n NW + wv) 64 + lane of a plane's staging is
+    // row lq / PR, LDS piece lq % PR, which holds the global piece
+    // (lq % PR) ^ (row & kXYSwz) of that row
+    const v4u in_hi = raw_buffer(in + z * plane, pbytes);
+    const v4u in_lo = raw_buffer(in + z * plane + (SPLIT ? io.in_lo : 0), pbytes);
+    const uint32_t stage_lds = lds_addr(staging) + 1024u * (uint32_t)wv;
+    uint32_t loff[NI];
+#pragma unroll
+    for (int n = 0; n < NI; ++n) {
+        const int lq = (n * NW + wv) * 64 + lane;
+        const int row = lq / PR, pc = (lq % PR) ^ (row & kXYSwz);
+        const int c = x0 - S::HALO + 8 * pc;
+        const bool ok = pc >= S::PLO && pc < PR - S::PLO && c >= 0 && c < nx;
+        loff[n] = ok ? 2u * (uint32_t)((ya - RT + row) * nx + c) : kOutside;
+    }
+    // mask words: wave 2 i + h loads word columns 4 i + lane / 16 of rows
+    // 16 h + lane % 16; words of rows or columns beyond the volume belong to
+    // outputs that are not stored
+    const uint32_t mwords = (uint32_t)(g.wpr * g.ny);
+    const v4u mbuf = raw_buffer(bits + z * g.wpr * g.ny, 4u * mwords);
+    const bool mwave = wv < 2 * S::MLOADS;
+    const uint32_t mring_lds = lds_addr(mring) + (uint32_t)((wv & 1) * MHALF + (wv >> 1) * 256);
+    uint32_t moff = 4u * (uint32_t)((x0 / 32 + 4 * (wv >> 1) + (lane >> 4)) * ny + ya + 16 * (wv & 1) + (lane & 15));
+    const uint32_t row_step = 64u * (uint32_t)nx;  // bytes of 32 rows
+    auto issue_step = [&](int j) {
+        const uint32_t dst = stage_lds + (uint32_t)((j & 1) * P * SB);
+#pragma unroll
+        for (int n = 0; n < NI; ++n) {
+            dma16_buf(dst + (uint32_t)(n * NW * 1024), in_hi, loff[n]);
+            if constexpr (SPLIT) dma16_buf(dst + (uint32_t)(SB + n * NW * 1024), in_lo, loff[n]);
+            loff[n] += row_step;
+        }
+        if (mwave && j >= W - 1) {
+            dma4_buf(mring_lds + (uint32_t)((j & 1) * MSLOT), mbuf, moff);
+            moff += 128;
+        }
+    };
+
+    issue_step(0);
+    __syncthreads();  // tap tables
+    v8s ahi[C], alo[C];
+    lowp_read_taps<RT>(thi, tlo, col, kg, ahi, alo);
+
+    // y-pass: wave wv takes quad wv % 4 of sub-ring wv / 4; lane (kg, col)
+    // reads rows rl and rl + 4 of a slot, rl = 16 u + 8 kg + col / 4, lines
+    // 4 (col & 3) .. +3 of its quad; for u = 1 the lanes kg >= 2 are in the
+    // next slot
+    const int quad = wv & 3;
+    int roff[2][2];
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+#pragma unroll
+        for (int hh = 0; hh < 2; ++hh) {
+            const int rr = (16 * u + 8 * kg + (col >> 2) + 4 * hh) & 31;
+            roff[u][hh] = (wv >> 2) * kSlotBytes + rr * 128 + ((quad ^ row_swizzle(rr)) << 5) + 8 * (col & 3);
+        }
+    // epilogue: lane l of a wave stores row l / 2 of its 32 x 16 tile, columns
+    // 8 (l % 2) .. +7
+    const int rw = lane >> 1, hf = lane & 1;
+    const int pc = 8 * (wv >> 2) + 2 * quad + hf;  // 8-column piece of the strip
+    uint32_t eoff = (uint32_t)((ya + rw) * nx + x0 + 8 * pc);  // elements
+    const bool ecol = x0 + 8 * pc < nx;
+    const uint32_t estep = 32u * (uint32_t)nx;
+
+    // x-pass: waves 0-3 take rows 0-15, waves 4-7 rows 16-31
+    const int ux = wv >> 2, t0 = (wv & 1) + 4 * ((wv >> 1) & 1);
+    const int xrow = ux * HB + col * PR * 16;
+    int wslot = 0;  // j % W
+    for (int j = 0; j < nsteps; ++j) {
+        // step j's loads are followed only by the epilogue of step j - 1
+        if (j >= W) vm_wait<S::ST>();
+        else vm_wait<0>();
+        __syncthreads();
+        if (j + 1 < nsteps) issue_step(j + 1);
+        unsigned char *const stg = staging + (j & 1) * P * SB;
+
+        // ---- x-pass: the wave's row tile (rows 16 ux + col) and column tiles
+        // t0 and t0 + 2; tile t0 + 2 starts one 32-position chunk after tile
+        // t0, so C + 1 operand reads feed both MFMA chains
+        unsigned char *const slot = ring + wslot * SLOT;
+        {
+            constexpr int NR = C + 1;
+            v4f acc[2];
+            v8s xs[NR], xls[NR];
+            const unsigned char *const rowp = stg + xrow;
+#pragma unroll
+            for (int q = 0; q < NR; ++q) {
+                const int o = S::HALO - RT + 16 * t0 + 32 * q + 8 * kg;  // halves [o, o + 8)
+                if constexpr (RT % 8 == 0) {
+                    const int boff = ((o >> 3) ^ (col & kXYSwz)) << 4;
+                    xs[q] = *reinterpret_cast<const v8s *>(rowp + boff);
+                    if constexpr (SPLIT) xls[q] = *reinterpret_cast<const v8s *>(rowp + SB + boff);
+                } else {
+                    uint2 part[2], plo[2];
+#pragma unroll
+                    for (int hh = 0; hh < 2; ++hh) {
+                        const int oh = o + 4 * hh;
+                        const int boff = (((oh >> 3) ^ (col & kXYSwz)) << 4) + ((oh & 7) << 1);
+                        part[hh] = *reinterpret_cast<const uint2 *>(rowp + boff);
+                        if constexpr (SPLIT) plo[hh] = *reinterpret_cast<const uint2 *>(rowp + SB + boff);
+                    }
+                    xs[q] = __builtin_bit_cast(v8s, make_uint4(part[0].x, part[0].y, part[1].x, part[1].y));
+                    if constexpr (SPLIT) xls[q] = __builtin_bit_cast(v8s, make_uint4(plo[0].x, plo[0].y, plo[1].x, plo[1].y));
+                }
+            }
+            __builtin_amdgcn_sched_barrier(0);  // keeps the reads ahead of the products
+#pragma unroll
+            for (int i = 0; i < 2; ++i) acc[i] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+            for (int q = 0; q < C; ++q) {
+#pragma unroll
+                for (int i = 0; i < 2; ++i) acc[i] = L::mfma(ahi[q], xs[q + i], acc[i]);
+#pragma unroll
+                for (int i = 0; i < 2; ++i) acc[i] = L::mfma(alo[q], xs[q + i], acc[i]);
+                if constexpr (SPLIT)
+#pragma unroll
+                    for (int i = 0; i < 2; ++i) acc[i] = L::mfma(ahi[q], xls[q + i], acc[i]);
+            }
+            // lane holds its row, columns 16 t + 4 kg .. +3: one 8-byte piece
+            const int rs = 16 * ux + col;
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                const int xc = 16 * (t0 + 2 * i) + 4 * kg, sub = xc >> 6, ln = xc & 63;
+                const int boff = sub * kSlotBytes + rs * 128 + (((ln >> 4) ^ row_swizzle(rs)) << 5) + ((ln & 15) << 1);
+                if constexpr (SPLIT) {
+                    uint16_t hv[4], lv[4];
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) split_f16_scaled(acc[i][e], io.scale, hv[e], lv[e]);
+                    *reinterpret_cast<uint2 *>(slot + boff) = make_uint2(pack2(hv[0], hv[1]), pack2(hv[2], hv[3]));
+                    *reinterpret_cast<uint2 *>(slot + W * SLOT + boff) =
+                        make_uint2(pack2(lv[0], lv[1]), pack2(lv[2], lv[3]));
+                } else {
+                    *reinterpret_cast<uint2 *>(slot + boff) =
+                        make_uint2(pack2(L::from_f32(acc[i][0]), L::from_f32(acc[i][1])),
+                                   pack2(L::from_f32(acc[i][2]), L::from_f32(acc[i][3])));
+                }
+            }
+        }
+        wslot = wslot + 1 == W ? 0 : wslot + 1;
+        if (j < W - 1) continue;
+        __syncthreads();
+
+        // ---- y-pass of the pair whose first slot is wslot (the oldest)
+        v4f acc[2];
+        v8s yx[C][2], yxl[C][2];
+        typedef __attribute__((address_space(3))) v4s lds_v4s;
+        int sb[C + 1];
+#pragma unroll
+        for (int c = 0; c <= C; ++c) {
+            int si = wslot + c;
+            si = si >= W ? si - W : si;
+            sb[c] = si * SLOT;
+        }
+#pragma unroll
+        for (int c = 0; c < C; ++c)
+#pragma unroll
+            for (int u = 0; u < 2; ++u) {
+                const int base = u == 0 ? sb[c] : (kg >= 2 ? sb[c + 1] : sb[c]);
+                v4s part[2], plo[2];
+#pragma unroll
+                for (int hh = 0; hh < 2; ++hh) {
+                    const unsigned char *a = ring + base + roff[u][hh];
+                    part[hh] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s *)a);
+                    if constexpr (SPLIT) plo[hh] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s *)(a + W * SLOT));
+                }
+                yx[c][u] = v8s{part[0][0], part[0][1], part[0][2], part[0][3], part[1][0], part[1][1], part[1][2], part[1][3]};
+                if constexpr (SPLIT)
+                    yxl[c][u] = v8s{plo[0][0], plo[0][1], plo[0][2], plo[0][3], plo[1][0], plo[1][1], plo[1][2], plo[1][3]};
+            }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int u = 0; u < 2; ++u) acc[u] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int c = 0; c < C; ++c) {
+            // the data as the first operand: a lane then holds four columns of one row
+#pragma unroll
+            for (int u = 0; u < 2; ++u) acc[u] = L::mfma(yx[c][u], ahi[c], acc[u]);
+#pragma unroll
+            for (int u = 0; u < 2; ++u) acc[u] = L::mfma(yx[c][u], alo[c], acc[u]);
+            if constexpr (SPLIT)
+#pragma unroll
+                for (int u = 0; u < 2; ++u) acc[u] = L::mfma(yxl[c][u], ahi[c], acc[u]);
+        }
+
+        // ---- epilogue: the wave stages its tile as [row][column] in its part
+        // of the consumed staging buffer and stores whole 16-byte pieces
+        const unsigned char *const msl = mring + (j & 1) * MSLOT;
+        const uint32_t m =
+            *reinterpret_cast<const uint32_t *>(msl + (rw >> 4) * MHALF + (pc >> 2) * 64 + (rw & 15) * 4) >> (8 * (pc & 3));
+        unsigned char *const west = stg + wv * S::WEST;
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            const int row = 16 * u + col;  // columns 4 kg .. +3
+            if constexpr (FIN != 0) {
+                *reinterpret_cast<v4f *>(west + row * S::WPF + 16 * kg) =
+                    v4f{acc[u][0] * io.scale, acc[u][1] * io.scale, acc[u][2] * io.scale, acc[u][3] * io.scale};
+            } else if constexpr (SPLIT) {
+                uint16_t hv[4], lv[4];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) split_f16_scaled(acc[u][e], io.scale, hv[e], lv[e]);
+                *reinterpret_cast<uint2 *>(west + row * S::WP16 + 8 * kg) = make_uint2(pack2(hv[0], hv[1]), pack2(hv[2], hv[3]));
+                *reinterpret_cast<uint2 *>(west + 32 * S::WP16 + row * S::WP16 + 8 * kg) =
+                    make_uint2(pack2(lv[0], lv[1]), pack2(lv[2], lv[3]));
+            } else {
+                *reinterpret_cast<uint2 *>(west + row * S::WP16 + 8 * kg) =
+                    make_uint2(pack2(L::from_f32(acc[u][0]), L::from_f32(acc[u][1])),
+                               pack2(L::from_f32(acc[u][2]), L::from_f32(acc[u][3])));
+            }
+        }
+        wave_lds_sync();
+        if constexpr (FIN != 0) {
+            v4f v[2];
+#pragma unroll
+            for (int hh = 0; hh < 2; ++hh) {
+                v[hh] = *reinterpret_cast<const v4f *>(west + rw * S::WPF + 32 * hf + 16 * hh);
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    if ((m >> (4 * hh + e)) & 1u) v[hh][e] = 1.0f;
+            }
+            if constexpr ((FIN & 1) != 0) {
+#pragma unroll
+                for (int hh = 0; hh < 2; ++hh)
+                    store16_buf(io.fin_f32 + z * plane, 2 * pbytes, ecol ? 4 * eoff + 16u * hh : kOutside,
+                                __builtin_bit_cast(v4u, v[hh]));
+            }
+            if constexpr ((FIN & 2) != 0) {
+                v4u w;
+#pragma unroll
+                for (int hh = 0; hh < 2; ++hh) {
+                    w[2 * hh] = (uint32_t)quantise_u16_s(v[hh][0]) | ((uint32_t)quantise_u16_s(v[hh][1]) << 16);
+                    w[2 * hh + 1] = (uint32_t)quantise_u16_s(v[hh][2]) | ((uint32_t)quantise_u16_s(v[hh][3]) << 16);
+                }
+                store16_buf(io.fin_u16 + z * plane, pbytes, ecol ? 2 * eoff : kOutside, w);
+            }
+        } else {
+            const uint32_t one2 = L::from_f32(1.0f) * 0x10001u;  // 1.0 in both halves
+            v4u w = *reinterpret_cast<const v4u *>(west + rw * S::WP16 + 16 * hf), wl;
+            if constexpr (SPLIT) wl = *reinterpret_cast<const v4u *>(west + 32 * S::WP16 + rw * S::WP16 + 16 * hf);
+#pragma unroll
+            for (int e2 = 0; e2 < 4; ++e2) {
+                const uint32_t sel = ((m >> (2 * e2)) & 1u) * 0xffffu | ((m >> (2 * e2 + 1)) & 1u) * 0xffff0000u;
+                w[e2] = (w[e2] & ~sel) | (one2 & sel);
+                if constexpr (SPLIT) wl[e2] &= ~sel;
+            }
+            store16_buf(out + z * plane, pbytes, ecol ? 2 * eoff : kOutside, w);
+            if constexpr (SPLIT) store16_buf(out + io.out_lo + z * plane, pbytes, ecol ? 2 * eoff : kOutside, wl);
+        }
+        eoff += estep;
+    }
+    vm_wait<0>();
+}
+
 // ---------------------------------------------------------------- host side
 // Strip width and prefetch depth per form (measured on 1024^3, R=40).
 #ifndef MXB_XY_TX16
@@ -634,7 +1025,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(SPLIT ? 1 :
 #define MXB_XY_DS 3
 #endif
 
-// Strip width and prefetch depth of a form and radius bucket: the deepest
+// Strip width and 16-row-step prefetch depth of a form and radius bucket: the deepest
 // prefetch up to the form's default whose shape fits the LDS.  FITS: the
 // fused pass serves the bucket.  The 16-bit forms take it where two blocks
 // share a CU (80 KB of LDS each): with one block per CU it was slower than
@@ -718,6 +1109,24 @@ static hipError_t launch_xy_rt(const uint16_t *in, uint16_t *out, const MaskBits
     const int fin = (io.fin_f32 != nullptr ? 1 : 0) + (io.fin_u16 != nullptr ? 2 : 0);
     const dim3 grid((unsigned)blocks), block(64 * kXYWaves);
     const uint32_t *w = bits.w;
+    if constexpr (XYPair<RT, TX, SPLIT, 0>::FITS && XYPair<RT, TX, SPLIT, SPLIT ? 3 : 0>::FITS) {
+        // byte offsets of the FP32 outputs, and of rows up to 512 before or
+        // after the plane, stay below the offset that means "outside"
+        if ((ny + 512) * nx < (int64_t(1) << 28)) {
+            if constexpr (SPLIT) {
+                switch (fin) {
+                case 0: hipLaunchKernelGGL((k_xy_pair<RT, TX, false, true, 0>), grid, block, 0, s, in, out, w, g, t, io); break;
+                case 1: hipLaunchKernelGGL((k_xy_pair<RT, TX, false, true, 1>), grid, block, 0, s, in, out, w, g, t, io); break;
+                case 2: hipLaunchKernelGGL((k_xy_pair<RT, TX, false, true, 2>), grid, block, 0, s, in, out, w, g, t, io); break;
+                default: hipLaunchKernelGGL((k_xy_pair<RT, TX, false, true, 3>), grid, block, 0, s, in, out, w, g, t, io); break;
+                }
+            } else {
+                if (fin != 0) return hipErrorInvalidValue;
+                hipLaunchKernelGGL((k_xy_pair<RT, TX, BF, false, 0>), grid, block, 0, s, in, out, w, g, t, io);
+            }
+            return hipGetLastError();
+        }
+    }
     if constexpr (!XYForm<RT, SPLIT>::FITS) {
         return hipErrorInvalidValue;
     } else if constexpr (SPLIT) {

@@ -32,3 +32,43 @@ def test_rows_of_any_alignment(gpu, monkeypatch, case, sigma):
     assert np.array_equal(got[1][0], want[1][0])
     u, _ = oracle.diffusion_f32(mask, k, 3)
     assert np.abs(got[0][1] - u).max() <= 1e-5
+
+
+@pytest.mark.parametrize("sigma", [0.9, 1.9, 2.9, 3.9, 5.9, 7.9, 9.9, 11.9])
+@pytest.mark.parametrize("prec", ["fp32_split", "bf16", "fp16"])
+def test_fused_pass_steps_of_16_and_32_rows(gpu, prec, sigma):
+    """The fused x -> y pass steps by 32 rows where a plane is small enough for
+    32-bit offsets, else by 16.  A few columns of mask at the edge of a very
+    wide volume (16 rows a step) and of a narrow one (32) give the same values,
+    bit for bit, in the columns that the other columns cannot reach; one
+    radius of each compiled size."""
+    ny, wide, narrow, reps = 41, 1 << 19, 968, 3
+    k = gauss_kernel(sigma).astype(np.float32)
+    keep = narrow - reps * (len(k) // 2)
+    rng = np.random.default_rng(31)
+    m = np.zeros((2, ny, wide), np.uint8)
+    m[:, :, :keep] = rng.random((2, ny, keep)) > 0.95
+    print("fused steps", prec, sigma, flush=True)
+    a = capi.diffusion(m, k, reps, precision=prec, u16=True, f32=True)
+    b = capi.diffusion(np.ascontiguousarray(m[:, :, :narrow]), k, reps, precision=prec, u16=True, f32=True)
+    keep -= len(k) // 2
+    assert np.array_equal(a[0][:, :, :keep], b[0][:, :, :keep])
+    assert np.array_equal(a[1][:, :, :keep], b[1][:, :, :keep])
+
+
+@pytest.mark.parametrize("prec, bar", [("fp32_split", 1e-5), ("bf16", 2e-3), ("fp16", 2e-3)])
+@pytest.mark.parametrize("shape", [(1, 31, 8), (2, 32, 120), (1, 65, 136), (1, 700, 264), (3, 1, 1024)])
+def test_fused_pass_edges(gpu, prec, bar, shape):
+    """Rows about one step, strips with a last piece of 8 columns, planes cut
+    into several segments, each with the outputs of the last repetition alone
+    and together."""
+    rng = np.random.default_rng(77)
+    m = (rng.random(shape) > 0.95).astype(np.uint8)
+    for sigma in (1.2, 4.0, 11.0):
+        k = gauss_kernel(sigma).astype(np.float32)
+        print("fused edges", prec, shape, sigma, flush=True)
+        q, u = capi.diffusion(m, k, 3, precision=prec, u16=True, f32=True)
+        ref = oracle.diffusion_f64(m, k.astype(np.float64), 3)
+        assert np.abs(u - ref).max() <= bar and np.all(u[m > 0] == 1.0)
+        assert np.array_equal(q, capi.diffusion(m, k, 3, precision=prec, u16=True, f32=False)[0])
+        assert np.array_equal(u, capi.diffusion(m, k, 3, precision=prec, u16=False, f32=True)[1])
