@@ -1091,7 +1091,11 @@ static hipError_t launch_xy_rt(const uint16_t *in, uint16_t *out, const MaskBits
     // whole columns per block unless the grid would be too small to fill the chip
     const int64_t cols = nz * g.nstrip;
     int64_t nseg = (256 * 2 + cols - 1) / cols;
-    const int64_t max_seg = (ny + 63) / 64;
+    // segments of at least 64 rows, or of one pair where that gives every
+    // block a CU of its own (64^3 split, sigma 3 / 10, ten repetitions: 126 ->
+    // 111 / 144 -> 130 us, BF16 106 -> 97; at 128^3, two blocks a CU, 200 -> 235)
+    const int64_t max_pairs = (ny + 31) / 32;
+    const int64_t max_seg = cols * max_pairs <= 256 ? max_pairs : (ny + 63) / 64;
     if (nseg > max_seg) nseg = max_seg;
     if (nseg < 1) nseg = 1;
     g.seg = ((ny + nseg - 1) / nseg + 31) / 32 * 32;

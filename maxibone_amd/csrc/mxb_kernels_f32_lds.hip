@@ -92,11 +92,17 @@ static hipError_t launch_lds_rt(const float *in, LineGeom g, const Epilogue &e, 
     const int64_t groups = ((g.n_lane + 63) / 64) * g.n_outer;
     const int64_t target = 256LL * 6;
     int64_t nseg = groups > 0 ? (target + groups - 1) / groups : 1;
-    const int64_t max_seg = (g.n_ax + 63) / 64;
+    const int64_t q = e.mask != nullptr ? 32 : 16;  // the illuminating pass: whole mask-bit words
+    // Segments of at least 64 positions, whose halo costs little; where single
+    // tiles leave fewer than four blocks a CU a pass is its blocks' own
+    // latency, and the shortest segments win (64^3, sigma 3 / 10, ten
+    // repetitions: 140 -> 125 / 176 -> 130 us, 96^3 sigma 3 186 -> 176; at
+    // 128^3, four blocks a CU, 244 -> 246).
+    const int64_t max_tiles = (g.n_ax + q - 1) / q;
+    const int64_t max_seg = groups * max_tiles < 256 * 4 ? max_tiles : (g.n_ax + 63) / 64;
     if (nseg > max_seg) nseg = max_seg;
     if (nseg < 1) nseg = 1;
     int64_t seg = (g.n_ax + nseg - 1) / nseg;
-    const int64_t q = e.mask != nullptr ? 32 : 16;  // the illuminating pass: whole mask-bit words
     seg = ((seg + q - 1) / q) * q;
     g.seg = seg;
     g.nseg = (g.n_ax + seg - 1) / seg;

@@ -312,7 +312,10 @@ static hipError_t launch_lowp_dma_rt(int form, const uint16_t *in, uint16_t *out
     const int64_t groups = ((g.n_lane + 63) / 64) * g.n_outer;
     const int64_t target = 256LL * 6;
     int64_t nseg = groups > 0 ? (target + groups - 1) / groups : 1;
-    const int64_t max_seg = (g.n_ax + 63) / 64;
+    // one pair a segment where every block has a CU of its own, as in the
+    // split form (64^3 BF16, sigma 3, ten repetitions: 106 -> 102 us)
+    const int64_t max_pairs = (g.n_ax + 31) / 32;
+    const int64_t max_seg = groups * max_pairs <= 256 ? max_pairs : (g.n_ax + 63) / 64;
     if (nseg > max_seg) nseg = max_seg;
     if (nseg < 1) nseg = 1;
     int64_t seg = (g.n_ax + nseg - 1) / nseg;
@@ -414,7 +417,11 @@ static hipError_t launch_split_rt(int form, const uint16_t *in, uint16_t *out, c
     const int64_t groups = ((g.n_lane + 63) / 64) * g.n_outer;
     const int64_t target = 256LL * 6;
     int64_t nseg = groups > 0 ? (target + groups - 1) / groups : 1;
-    const int64_t max_seg = (g.n_ax + 63) / 64;
+    // segments of at least 64 positions, or of one pair where that gives every
+    // block a CU of its own (64^3, sigma 3, ten repetitions: 126 -> 120 us; at
+    // 128^3, four blocks a CU, 200 -> 219)
+    const int64_t max_pairs = (g.n_ax + 31) / 32;
+    const int64_t max_seg = groups * max_pairs <= 256 ? max_pairs : (g.n_ax + 63) / 64;
     if (nseg > max_seg) nseg = max_seg;
     if (nseg < 1) nseg = 1;
     int64_t seg = (g.n_ax + nseg - 1) / nseg;
