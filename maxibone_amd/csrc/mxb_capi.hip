@@ -6,6 +6,7 @@
 #include <unistd.h>
 
 #include <algorithm>
+#include <atomic>
 #include <cerrno>
 #include <cmath>
 #include <cstdio>
@@ -13,6 +14,7 @@
 #include <cstring>
 #include <mutex>
 #include <string>
+#include <system_error>
 #include <thread>
 #include <vector>
 
@@ -622,48 +624,49 @@ static int chunked_host(const uint8_t *mask, int64_t nz, int64_t ny, int64_t nx,
 }
 
 // ---------------------------------------------------------------- staged copies
-// Copies between pageable host memory and the device through two pinned
-// 64 MB chunks: host threads fill (or drain) one chunk while the DMA engine
-// moves the other.  A pageable hipMemcpy runs at ~10 GB/s on the MI355X
-// boxes; the staged form moves several times that.  The pinned chunks are
-// allocated at the first large copy and kept until the process ends; one
-// staged copy runs at a time (a mutex).  Small copies, or a failed pinned
-// allocation, take the plain path.
+// Copies between pageable host memory and the device through a ring of pinned
+// units: host threads fill (or drain) a unit in pieces while the DMA engine
+// moves others.  A pageable hipMemcpy runs at ~10 GB/s, one thread's memcpy;
+// the staged form is bound by the DMA engine (45 GB/s) and by the 40 to 80 us
+// between two copies, hence units of 8 MB.  Whole calls on host arrays (one
+// FP32 repetition, uint16 output), pageable copies below 128 MB -> staged from
+// 8 MB: 200^3 2.0 -> 1.2 ms, 256^3 3.3 -> 2.2, 400^3 15.9 -> 5.6; 512^3 and
+// 640^3, staged in 64 MB chunks before, 12.6 -> 10.5 and 20.1 -> 19.2.
+// The pinned ring (64 MB) is allocated at the first large copy and kept until
+// the process ends; one staged copy runs at a time (a mutex).  Copies of fewer
+// than kStageMin bytes, where starting the threads costs more than it saves,
+// or a failed pinned allocation, take the plain path.
 namespace {
-constexpr size_t kStageChunk = size_t(64) << 20;
+constexpr size_t kStagePiece = size_t(2) << 20, kStagePieces = 4;  // a thread's share; pieces per unit
+constexpr size_t kStageUnit = kStagePiece * kStagePieces;
+constexpr size_t kStageMin = kStageUnit;
+constexpr int kStageThreads = 16, kStageSlots = 8;  // slots: units in the ring
 std::mutex g_stage_mu;
-void *g_stage[2] = {nullptr, nullptr};
-hipEvent_t g_stage_ev[2] = {nullptr, nullptr};
+char *g_stage = nullptr;
+hipEvent_t g_stage_ev[kStageSlots];
+int g_stage_dev = -1;  // the events' device
 
-void parallel_memcpy(void *dst, const void *src, size_t bytes) {
-    unsigned nt = std::thread::hardware_concurrency();
-    nt = nt == 0 ? 4 : std::min(nt, 16u);
-    const size_t part = (bytes + nt - 1) / nt;
-    std::vector<std::thread> th;
-    for (unsigned i = 0; i < nt; ++i) {
-        const size_t b = i * part;
-        if (b >= bytes) break;
-        const size_t len = std::min(part, bytes - b);
-        th.emplace_back([=] { std::memcpy(static_cast<char *>(dst) + b, static_cast<const char *>(src) + b, len); });
-    }
-    for (auto &t : th) t.join();
-}
-
-bool stage_ready() {
-    if (g_stage[0] != nullptr) return true;
-    for (int i = 0; i < 2; ++i) {
-        if (hipHostMalloc(&g_stage[i], kStageChunk, hipHostMallocDefault) != hipSuccess ||
-            hipEventCreateWithFlags(&g_stage_ev[i], hipEventDisableTiming) != hipSuccess) {
+// The pinned chunks (usable from every device) and events of the current device.
+bool stage_ready(int dev) {
+    if (g_stage == nullptr) {
+        void *p = nullptr;
+        if (hipHostMalloc(&p, kStageSlots * kStageUnit, hipHostMallocPortable) != hipSuccess) {
             (void)hipGetLastError();
-            for (int j = 0; j <= i; ++j) {
-                if (g_stage[j]) (void)hipHostFree(g_stage[j]);
-                if (g_stage_ev[j]) (void)hipEventDestroy(g_stage_ev[j]);
-                g_stage[j] = nullptr;
-                g_stage_ev[j] = nullptr;
-            }
+            return false;
+        }
+        g_stage = static_cast<char *>(p);
+    }
+    if (g_stage_dev == dev) return true;
+    for (int i = 0; i < kStageSlots && g_stage_dev >= 0; ++i) (void)hipEventDestroy(g_stage_ev[i]);
+    g_stage_dev = -1;
+    for (int made = 0; made < kStageSlots; ++made) {
+        if (hipEventCreateWithFlags(&g_stage_ev[made], hipEventDisableTiming) != hipSuccess) {
+            (void)hipGetLastError();
+            while (made > 0) (void)hipEventDestroy(g_stage_ev[--made]);
             return false;
         }
     }
+    g_stage_dev = dev;
     return true;
 }
 }  // namespace
@@ -671,41 +674,113 @@ bool stage_ready() {
 // Host -> device (h2d) or device -> host copy of `bytes`, ordered on `s`
 // after the work already queued there; returns with the copy complete.
 hipError_t staged_copy(void *dst, const void *src, size_t bytes, bool h2d, hipStream_t s) {
-    std::lock_guard<std::mutex> lk(g_stage_mu);
-    if (bytes < 2 * kStageChunk || !stage_ready()) {
+    std::unique_lock<std::mutex> lk(g_stage_mu, std::defer_lock);
+    if (bytes >= kStageMin) lk.lock();
+    int dev = 0;
+    if (bytes < kStageMin || hipGetDevice(&dev) != hipSuccess || !stage_ready(dev)) {
         hipError_t e = hipMemcpyAsync(dst, src, bytes, h2d ? hipMemcpyHostToDevice : hipMemcpyDeviceToHost, s);
         return e != hipSuccess ? e : hipStreamSynchronize(s);
     }
-    const size_t nch = (bytes + kStageChunk - 1) / kStageChunk;
-    auto len_of = [&](size_t i) { return std::min(kStageChunk, bytes - i * kStageChunk); };
-    hipError_t e;
-    if (h2d) {
-        for (size_t i = 0; i < nch; ++i) {
-            const int b = (int)(i % 2);
-            if (i >= 2 && (e = hipEventSynchronize(g_stage_ev[b])) != hipSuccess) return e;
-            parallel_memcpy(g_stage[b], static_cast<const char *>(src) + i * kStageChunk, len_of(i));
-            if ((e = hipMemcpyAsync(static_cast<char *>(dst) + i * kStageChunk, g_stage[b], len_of(i),
-                                    hipMemcpyHostToDevice, s)) != hipSuccess ||
-                (e = hipEventRecord(g_stage_ev[b], s)) != hipSuccess)
-                return e;
-        }
-        return hipStreamSynchronize(s);
+    // device -> host: the threads start when there is something to move
+    if (!h2d) {
+        const hipError_t e = hipStreamSynchronize(s);
+        if (e != hipSuccess) return e;
     }
-    auto enqueue = [&](size_t i) -> hipError_t {
-        const int b = (int)(i % 2);
-        hipError_t r = hipMemcpyAsync(g_stage[b], static_cast<const char *>(src) + i * kStageChunk, len_of(i),
-                                      hipMemcpyDeviceToHost, s);
-        return r != hipSuccess ? r : hipEventRecord(g_stage_ev[b], s);
+    const size_t npiece = (bytes + kStagePiece - 1) / kStagePiece, nunit = (bytes + kStageUnit - 1) / kStageUnit;
+    const int nt = (int)std::min<size_t>(kStageThreads, npiece);
+    std::atomic<size_t> next{0};  // the next piece to take
+    std::atomic<int> err{(int)hipSuccess};
+    auto check = [&](hipError_t e) {
+        if (e != hipSuccess) err.store((int)e);
+        return e == hipSuccess;
     };
-    for (size_t i = 0; i < std::min<size_t>(2, nch); ++i)
-        if ((e = enqueue(i)) != hipSuccess) return e;
-    for (size_t i = 0; i < nch; ++i) {
-        const int b = (int)(i % 2);
-        if ((e = hipEventSynchronize(g_stage_ev[b])) != hipSuccess) return e;
-        parallel_memcpy(static_cast<char *>(dst) + i * kStageChunk, g_stage[b], len_of(i));
-        if (i + 2 < nch && (e = enqueue(i + 2)) != hipSuccess) return e;
+    auto piece_len = [&](size_t i) { return std::min(kStagePiece, bytes - i * kStagePiece); };
+    auto unit_len = [&](size_t u) { return std::min(kStageUnit, bytes - u * kStageUnit); };
+    auto pin_of = [&](size_t u) { return g_stage + u % kStageSlots * kStageUnit; };
+    auto wait_for = [&](const std::atomic<size_t> &count, size_t want) {
+        while (count.load() < want) {
+            if (err.load() != (int)hipSuccess) return false;
+            std::this_thread::yield();
+        }
+        return true;
+    };
+    std::atomic<size_t> moved[kStageSlots], issued[kStageSlots];  // over all uses of a slot (of a half of them)
+    for (int i = 0; i < kStageSlots; ++i) {
+        moved[i].store(0);
+        issued[i].store(0);
     }
-    return hipSuccess;
+    // The threads take pieces in order until none is left, so any number of
+    // threads completes the copy.
+    //
+    // Host -> device: who fills a unit's last piece issues its copy.  An event
+    // between two copies costs 75 us on the stream, so there is one for each
+    // half of the slots, recorded after the half's last copy; who fills a slot
+    // of the half again waits for it.  (It is recorded again only after that.)
+    constexpr size_t kHalf = kStageSlots / 2;
+    auto upload = [&] {
+        size_t i;
+        while (err.load() == (int)hipSuccess && (i = next.fetch_add(1)) < npiece) {
+            const size_t u = i / kStagePieces, slot = u % kStageSlots, use = u / kStageSlots, h = slot / kHalf;
+            if (use > 0 &&
+                (!wait_for(issued[h], use * (kHalf + 1)) || !check(hipEventSynchronize(g_stage_ev[h]))))
+                return;
+            std::memcpy(pin_of(u) + i % kStagePieces * kStagePiece, static_cast<const char *>(src) + i * kStagePiece,
+                        piece_len(i));
+            const size_t full = use * kStagePieces + (unit_len(u) + kStagePiece - 1) / kStagePiece;
+            if (moved[slot].fetch_add(1) + 1 < full) continue;
+            if (!check(hipMemcpyAsync(static_cast<char *>(dst) + u * kStageUnit, pin_of(u), unit_len(u),
+                                      hipMemcpyHostToDevice, s)))
+                return;
+            // the recording counts as one more, after the half's copies
+            if (issued[h].fetch_add(1) + 1 == use * (kHalf + 1) + kHalf) {
+                if (!check(hipEventRecord(g_stage_ev[h], s))) return;
+                issued[h].fetch_add(1);
+            }
+        }
+    };
+    // Device -> host: the first units' copies are issued at once, each with its
+    // slot's event; who drains a unit's last piece issues the copy that takes
+    // its slot next.
+    auto fetch = [&](size_t u) {
+        const size_t slot = u % kStageSlots;
+        const bool ok = check(hipMemcpyAsync(pin_of(u), static_cast<const char *>(src) + u * kStageUnit, unit_len(u),
+                                             hipMemcpyDeviceToHost, s)) &&
+                        check(hipEventRecord(g_stage_ev[slot], s));
+        if (ok) issued[slot].fetch_add(1);
+        return ok;
+    };
+    auto download = [&] {
+        size_t i;
+        while (err.load() == (int)hipSuccess && (i = next.fetch_add(1)) < npiece) {
+            const size_t u = i / kStagePieces, slot = u % kStageSlots, use = u / kStageSlots;
+            if (!wait_for(issued[slot], use + 1) || !check(hipEventSynchronize(g_stage_ev[slot]))) return;
+            std::memcpy(static_cast<char *>(dst) + i * kStagePiece, pin_of(u) + i % kStagePieces * kStagePiece,
+                        piece_len(i));
+            if (moved[slot].fetch_add(1) + 1 == (use + 1) * kStagePieces && u + kStageSlots < nunit &&
+                !fetch(u + kStageSlots))
+                return;
+        }
+    };
+    if (!h2d)
+        for (size_t u = 0; u < std::min<size_t>(kStageSlots, nunit) && fetch(u);) ++u;
+    auto work = [&](int w) {
+        if (w > 0 && !check(hipSetDevice(dev))) return;
+        if (h2d) upload();
+        else download();
+    };
+    std::thread th[kStageThreads];
+    for (int w = 1; w < nt; ++w) {
+        try {
+            th[w] = std::thread(work, w);
+        } catch (const std::system_error &) {
+            break;  // the threads that run take its chunks
+        }
+    }
+    work(0);
+    for (int w = 1; w < nt; ++w)
+        if (th[w].joinable()) th[w].join();
+    const hipError_t e = hipStreamSynchronize(s);
+    return err.load() != (int)hipSuccess ? (hipError_t)err.load() : e;
 }
 
 // Device memory the drivers may plan with: 92 % of what is free, less
@@ -760,19 +835,21 @@ static int in_memory(const uint8_t *mask, int64_t nz, int64_t ny, int64_t nx, co
     }
     Stream st;
     MXB_HIP(hipStreamCreateWithFlags(&st.s, hipStreamNonBlocking));
-    DevBuf dm, d0, d1, dq, df;
-    MXB_HIP(dm.alloc(n));
-    MXB_HIP(d0.alloc(sb));
-    MXB_HIP(d1.alloc(sb));
-    if (out_u16) MXB_HIP(dq.alloc(n * 2));
-    if (out_f32) MXB_HIP(df.alloc(n * 4));
+    // one allocation for the mask, the two states and the outputs: a hipMalloc
+    // and hipFree pair costs 0.1 to 0.5 ms, five of them 1.1 of 256^3's 4.3 ms
+    auto part = [](int64_t bytes) { return (bytes + 4095) / 4096 * 4096; };
+    const int64_t o0 = part(n), o1 = o0 + part(sb), oq = o1 + part(sb), of = oq + (out_u16 ? part(2 * n) : 0);
+    DevBuf all;
+    MXB_HIP(all.alloc(of + (out_f32 ? part(4 * n) : 0)));
+    char *const base = static_cast<char *>(all.p);
+    uint16_t *const dq = out_u16 ? reinterpret_cast<uint16_t *>(base + oq) : nullptr;
+    float *const df = out_f32 ? reinterpret_cast<float *>(base + of) : nullptr;
     log_v(verbose, 1, "Converting uint8 to float");
-    MXB_HIP(staged_copy(dm.p, mask, n, true, st.s));
-    rc = run_steps((const uint8_t *)dm.p, nz, ny, nx, k, K, reps, precision, d0.p, d1.p,
-                   (uint16_t *)dq.p, (float *)df.p, st.s);
+    MXB_HIP(staged_copy(base, mask, n, true, st.s));
+    rc = run_steps((const uint8_t *)base, nz, ny, nx, k, K, reps, precision, base + o0, base + o1, dq, df, st.s);
     if (rc != OK) return rc;
-    if (out_u16) MXB_HIP(staged_copy(out_u16, dq.p, n * 2, false, st.s));
-    if (out_f32) MXB_HIP(staged_copy(out_f32, df.p, n * 4, false, st.s));
+    if (out_u16) MXB_HIP(staged_copy(out_u16, dq, n * 2, false, st.s));
+    if (out_f32) MXB_HIP(staged_copy(out_f32, df, n * 4, false, st.s));
     MXB_HIP(hipStreamSynchronize(st.s));
     log_v(verbose, 1, "Diffusion is complete!");
     return OK;

@@ -72,3 +72,25 @@ def test_fused_pass_edges(gpu, prec, bar, shape):
         assert np.abs(u - ref).max() <= bar and np.all(u[m > 0] == 1.0)
         assert np.array_equal(q, capi.diffusion(m, k, 3, precision=prec, u16=True, f32=False)[0])
         assert np.array_equal(u, capi.diffusion(m, k, 3, precision=prec, u16=False, f32=True)[1])
+
+
+@pytest.mark.parametrize("n", [(4 << 20) - 1, 4 << 20, (4 << 20) + 1, (8 << 20) + 1, (33 << 20) + 5, (70 << 20) + 3])
+def test_host_copies(gpu, n):
+    """Volumes in host memory about the sizes where the staged copies start,
+    end in a part of a piece, and use their ring again; from two threads at
+    once.  No repetition: the outputs are the mask's own values."""
+    import threading
+
+    print("host copies", n, flush=True)
+    m = (np.random.default_rng(n).integers(0, 256, n, dtype=np.uint8) > 100).astype(np.uint8).reshape(1, 1, n)
+    out = [None, None]
+
+    def run(i):
+        out[i] = capi.diffusion(m, np.ones(1, np.float32), 0, precision="fp32", u16=True, f32=True)
+
+    ts = [threading.Thread(target=run, args=(i,)) for i in range(2)]
+    [t.start() for t in ts]
+    [t.join() for t in ts]
+    for q, u in out:
+        assert np.array_equal(u, m.astype(np.float32))
+        assert np.array_equal(q, np.where(m, np.uint16(65535), np.uint16(0)))
