@@ -186,10 +186,21 @@ static int run_steps_f32(const uint8_t *d_mask, const MaskBits &bits, int64_t nz
         return OK;
     }
     const LineGeom gz = geom_z(nz, ny, nx), gy = geom_y(nz, ny, nx), gx = geom_x(nz, ny, nx);
+    const bool fused = arith == Arith::MFMA && xy_fusion_enabled() && yx_f32_supported(tmp, bits, nz, ny, nx, R);
     for (int64_t t = 0; t < reps; ++t) {
         const bool last = t == reps - 1;
         const Epilogue ez{nullptr, tmp, nullptr, MaskBits{}};
         MXB_HIP(timed(MXB_K_ZPASS, s, [&] { return launch_line_pass_f32(cur, gz, ez, k, R, arith, s); }));
+        if (fused) {
+            // y then x in one pass, back into cur (or into the outputs), illuminating
+            const bool unread = last && out_u16 != nullptr && final_state == nullptr;
+            float *dst = last && out_f32 != nullptr ? out_f32 : (unread ? nullptr : cur);
+            MXB_HIP(timed(MXB_K_XYPASS, s, [&] {
+                return launch_yx_f32(tmp, dst, last ? out_u16 : nullptr, bits, nz, ny, nx, k, R, s);
+            }));
+            if (last && final_state) *final_state = dst;
+            continue;
+        }
         const Epilogue ey{nullptr, cur, nullptr, MaskBits{}};
         MXB_HIP(timed(MXB_K_YPASS, s, [&] { return launch_line_pass_f32(tmp, gy, ey, k, R, arith, s); }));
         // the last x-pass writes the float state only where someone reads it

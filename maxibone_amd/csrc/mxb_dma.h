@@ -127,6 +127,35 @@ __device__ __forceinline__ void dma4(uint32_t lds_wave_base, const void *src) {
 #pragma clang diagnostic pop
 }
 
+// Buffer over [p, p + bytes): raw 32-bit byte offsets, those at or beyond
+// `bytes` read zeros and store nothing.  Uniform.
+__device__ __forceinline__ v4u32 raw_buffer(const void *p, uint32_t bytes) {
+    const uint64_t a = reinterpret_cast<uint64_t>(p);
+    return v4u32{(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)a),
+               (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(a >> 32)) & 0xffffu,
+               (uint32_t)__builtin_amdgcn_readfirstlane((int)bytes), 0x00020000u};
+}
+
+// dma16 / dma4 from a buffer.
+__device__ __forceinline__ void dma16_buf(uint32_t lds_wave_base, v4u32 buf, uint32_t off) {
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"
+                 :
+                 : "s"(lds_wave_base), "v"(off), "s"(buf)
+                 : "memory", "m0");
+#pragma clang diagnostic pop
+}
+__device__ __forceinline__ void dma4_buf(uint32_t lds_wave_base, v4u32 buf, uint32_t off) {
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dword %1, %2, 0 offen lds"
+                 :
+                 : "s"(lds_wave_base), "v"(off), "s"(buf)
+                 : "memory", "m0");
+#pragma clang diagnostic pop
+}
+
 // s_waitcnt with vmcnt = N and no wait on the other counters.
 template <int N>
 __device__ __forceinline__ void vm_wait() {

@@ -683,36 +683,8 @@ struct XYPair {
     static constexpr bool FITS = RT <= HALO && HALO - RT + TX + 32 * C - 16 <= ROWH && BYTES <= 160 * 1024 - 512;
 };
 
-typedef uint32_t v4u __attribute__((ext_vector_type(4)));
+typedef v4u32 v4u;
 
-// Buffer over [p, p + bytes): raw 32-bit byte offsets, those at or beyond
-// `bytes` read zeros and store nothing.  Uniform.
-__device__ __forceinline__ v4u raw_buffer(const void *p, uint32_t bytes) {
-    const uint64_t a = reinterpret_cast<uint64_t>(p);
-    return v4u{(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)a),
-               (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(a >> 32)) & 0xffffu,
-               (uint32_t)__builtin_amdgcn_readfirstlane((int)bytes), 0x00020000u};
-}
-
-// dma16 / dma4 from a buffer.
-__device__ __forceinline__ void dma16_buf(uint32_t lds_wave_base, v4u buf, uint32_t off) {
-#pragma clang diagnostic push
-#pragma clang diagnostic ignored "-Winline-asm"
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"
-                 :
-                 : "s"(lds_wave_base), "v"(off), "s"(buf)
-                 : "memory", "m0");
-#pragma clang diagnostic pop
-}
-__device__ __forceinline__ void dma4_buf(uint32_t lds_wave_base, v4u buf, uint32_t off) {
-#pragma clang diagnostic push
-#pragma clang diagnostic ignored "-Winline-asm"
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dword %1, %2, 0 offen lds"
-                 :
-                 : "s"(lds_wave_base), "v"(off), "s"(buf)
-                 : "memory", "m0");
-#pragma clang diagnostic pop
-}
 __device__ __forceinline__ void store16_buf(void *plane, uint32_t bytes, uint32_t off, v4u v) {
     __builtin_amdgcn_raw_buffer_store_b128(v, __builtin_amdgcn_make_buffer_rsrc(plane, 0, (int)bytes, 0x00020000),
                                            (int)off, 0, 0);

@@ -101,6 +101,13 @@ bool lds_pass_supported(const float *in, const LineGeom &g, const Epilogue &e, i
 hipError_t launch_line_pass_f32_lds(const float *in, const LineGeom &g, const Epilogue &e,
                                     const float *taps, int R, hipStream_t s);
 
+// Fused y -> x pass of the FP32 form (mxb_f32_yx.hip): the z-pass output `in`
+// -> out_f32 and / or out_u16 in (z, y, x) order, illuminating from the mask
+// bits; the values of the two separate passes bit for bit.
+bool yx_f32_supported(const float *in, const MaskBits &bits, int64_t nz, int64_t ny, int64_t nx, int R);
+hipError_t launch_yx_f32(const float *in, float *out_f32, uint16_t *out_u16, const MaskBits &bits, int64_t nz,
+                         int64_t ny, int64_t nx, const float *taps, int R, hipStream_t s);
+
 // Reduced-precision passes (mxb_kernels_lowp.hip): 16-bit state in and out,
 // `bf` selects BF16 (else FP16).  `mask` non-null illuminates.
 hipError_t launch_line_pass_lowp(const uint16_t *in, uint16_t *out, const uint8_t *mask,

@@ -94,3 +94,26 @@ def test_host_copies(gpu, n):
     for q, u in out:
         assert np.array_equal(u, m.astype(np.float32))
         assert np.array_equal(q, np.where(m, np.uint16(65535), np.uint16(0)))
+
+
+YX_SHAPES = [(1, 1, 4), (2, 63, 32), (3, 64, 36), (1, 65, 96), (2, 130, 128), (1, 200, 613), (30, 20, 31),
+             (1, 3, 1), (5, 129, 1000), (260, 300, 70)]
+
+
+@pytest.mark.parametrize("sigma", [1.0, 2.0, 3.0, 4.0, 5.0, 6.0, 8.0, 10.0, 12.0, 14.0, 16.0])
+def test_fused_fp32_y_and_x(gpu, monkeypatch, sigma):
+    """The FP32 form's fused y -> x pass against the register-ring passes, bit
+    for bit, one radius of each compiled size: tiles of 64 rows and pairs of 32
+    columns exactly, one more and one less, rows of 4-byte and of 16-byte
+    pieces, one and several segments, each set of outputs."""
+    k = gauss_kernel(sigma).astype(np.float32)
+    for i, shape in enumerate(YX_SHAPES):
+        print("fused y and x", shape, sigma, flush=True)
+        m = (np.random.default_rng(500 + i).random(shape) > 0.96).astype(np.uint8)
+        for out in ({"u16": True, "f32": True}, {"u16": True, "f32": False}, {"u16": False, "f32": True}):
+            monkeypatch.delenv("MXB_PASS_KERNEL", raising=False)
+            got = capi.diffusion(m, k, 2, precision="fp32", **out)
+            monkeypatch.setenv("MXB_PASS_KERNEL", "ring")
+            want = capi.diffusion(m, k, 2, precision="fp32", **out)
+            for a, b in zip(got, want):
+                assert (a is None) == (b is None) and (a is None or np.array_equal(a, b))
