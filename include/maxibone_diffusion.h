@@ -216,8 +216,8 @@ int mxb_device_diffusion_noalloc(const uint8_t *dev_mask, int64_t nz, int64_t ny
 
 /* ---- per-kernel timing (HIP events on the launch stream) ------------------ */
 
-/* Kernel classes reported by mxb_kernel_times (MXB_K_XYPASS: the fused
- * x -> y pass of the 16-bit and split forms). */
+/* Kernel classes reported by mxb_kernel_times (MXB_K_XYPASS: the fused pass
+ * over x and y, x -> y in the 16-bit and split forms, y -> x in FP32). */
 typedef enum {
     MXB_K_ZPASS = 0,
     MXB_K_YPASS = 1,

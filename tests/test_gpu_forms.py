@@ -117,3 +117,24 @@ def test_fused_fp32_y_and_x(gpu, monkeypatch, sigma):
             want = capi.diffusion(m, k, 2, precision="fp32", **out)
             for a, b in zip(got, want):
                 assert (a is None) == (b is None) and (a is None or np.array_equal(a, b))
+
+
+@pytest.mark.parametrize("prec", ["fp32", "bf16"])
+def test_fused_fp32_y_and_x_in_batches(gpu, monkeypatch, prec):
+    """The batched form's fused y -> x pass against its separate passes and the
+    single-volume form, bit for bit: rows whose last 16-byte piece holds pads,
+    rows of one pad less and more than a line, each radius size up to 40."""
+    shapes = [(3, 5, 7), (20, 64, 32), (9, 65, 33), (30, 63, 97), (4, 130, 126), (17, 31, 161), (2, 200, 62)]
+    sigmas = [2.0, 3.0, 4.0, 5.0, 6.0, 8.0, 10.0]
+    rng = np.random.default_rng(9)
+    ms = [(rng.random(s) > 0.95).astype(np.uint8) for s in shapes]
+    ks = [gauss_kernel(s).astype(np.float32) for s in sigmas]
+    print("fused batch", prec, flush=True)
+    got = capi.diffusion_batched(ms, ks, 3, precision=prec, u16=True, f32=True)
+    monkeypatch.setenv("MXB_XY_FUSED", "0")
+    want = capi.diffusion_batched(ms, ks, 3, precision=prec, u16=True, f32=True)
+    for i in range(len(ms)):
+        assert np.array_equal(got[0][i], want[0][i]) and np.array_equal(got[1][i], want[1][i])
+        if prec == "fp32":
+            one = capi.diffusion(ms[i], ks[i], 3, precision=prec, u16=True, f32=True)
+            assert np.array_equal(got[0][i], one[0]) and np.array_equal(got[1][i], one[1])
