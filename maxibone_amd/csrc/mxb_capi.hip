@@ -293,11 +293,12 @@ static int run_lowp_core(const uint8_t *d_mask, const MaskBits &bits, int64_t nz
 // the last in FP32.
 static int run_steps_lowp(const uint8_t *d_mask, const MaskBits &bits, int64_t nz, int64_t ny,
                           int64_t nx, const float *k, int64_t K, int64_t reps, bool bf, void *s0,
-                          void *s1, uint16_t *out_u16, float *out_f32, bool fused, hipStream_t s) {
+                          void *s1, uint16_t *out_u16, float *out_f32, bool fused, bool init_from_mask,
+                          hipStream_t s) {
     if (reps <= 1)
         return run_steps_f32(d_mask, bits, nz, ny, nx, k, K, reps, Arith::MFMA, (float *)s0,
-                             (float *)s1, true, out_u16, out_f32, nullptr, s);
-    return run_lowp_core(d_mask, bits, nz, ny, nx, k, K, reps - 1, true, bf, true, s0, s1, out_u16,
+                             (float *)s1, init_from_mask, out_u16, out_f32, nullptr, s);
+    return run_lowp_core(d_mask, bits, nz, ny, nx, k, K, reps - 1, true, bf, init_from_mask, s0, s1, out_u16,
                          out_f32, nullptr, nullptr, fused, s);
 }
 
@@ -327,8 +328,18 @@ static int split_serves(int64_t nz, int64_t ny, int64_t nx, int R, const void *s
                : 0;
 }
 
+// From the mask, the 0/1 state is exact in FP16: the first z-pass reads it as
+// the high plane alone (its low plane would be zeros).
+static SplitIO split_io_from_f16(int64_t lo) {
+    SplitIO io;
+    io.out_lo = lo;
+    io.widen = MXB_FP16;
+    return io;
+}
+
 // Split form: reps repetitions on FP16 hi + lo planes, starting from the mask
-// (from_f32 false) or from the FP32 state in s0 (split into s1 first).  Per
+// (from_f32 false), from the FP32 state in s0 (split into s1 first) or from
+// u0 as the FP16 plane in s0 (from_f16).  Per
 // repetition the z-pass writes the other buffer; then either the fused
 // x -> y pass writes back (form 2) or the y-pass (in (z, x, y) order) and the
 // x-pass do, swapping the buffers (form 1).  The last pass writes out_u16 /
@@ -336,7 +347,8 @@ static int split_serves(int64_t nz, int64_t ny, int64_t nx, int R, const void *s
 // state into the buffer its input is not in and reports it.
 static int run_steps_split(const uint8_t *d_mask, const MaskBits &bits, int64_t nz, int64_t ny, int64_t nx,
                            const float *k, int64_t K, int64_t reps, void *s0, void *s1, bool from_f32,
-                           uint16_t *out_u16, float *out_f32, float **final_state, int form, hipStream_t s) {
+                           uint16_t *out_u16, float *out_f32, float **final_state, int form, hipStream_t s,
+                           bool from_f16 = false) {
     const int64_t n = nz * ny * nx;
     const int R = (int)(K / 2);
     if (n == 0) return OK;
@@ -348,17 +360,13 @@ static int run_steps_split(const uint8_t *d_mask, const MaskBits &bits, int64_t 
     const LineGeom gz = geom_z(nz, ny, nx), gy = geom_y(nz, ny, nx), gx = geom_x(nz, ny, nx);
     SplitIO io;
     io.in_lo = io.out_lo = lo;
-    // From the mask, the 0/1 state is exact in FP16: the first z-pass reads
-    // it as the high plane alone (its low plane would be zeros).
-    SplitIO iz0 = io;
-    iz0.in_lo = 0;
-    iz0.widen = MXB_FP16;
+    const SplitIO iz0 = split_io_from_f16(lo);
     const bool widen0 = !from_f32 && split_pass_supported(cur, tmp, nullptr, bits, gz, R, iz0);
     if (from_f32) {
         MXB_HIP(timed(MXB_K_OTHER, s, [&] { return launch_split_state((const float *)s0, tmp, lo, n, s); }));
         std::swap(cur, tmp);
     } else if (widen0) {
-        MXB_HIP(timed(MXB_K_OTHER, s, [&] { return launch_init_lowp(d_mask, cur, n, false, s); }));
+        if (!from_f16) MXB_HIP(timed(MXB_K_OTHER, s, [&] { return launch_init_lowp(d_mask, cur, n, false, s); }));
     } else {
         MXB_HIP(timed(MXB_K_OTHER, s, [&] { return launch_init_split(d_mask, cur, lo, n, s); }));
     }
@@ -392,27 +400,42 @@ static int run_steps_split(const uint8_t *d_mask, const MaskBits &bits, int64_t 
 static int run_steps(const uint8_t *d_mask, int64_t nz, int64_t ny, int64_t nx, const float *k,
                      int64_t K, int64_t reps, int precision, void *s0, void *s1,
                      uint16_t *out_u16, float *out_f32, hipStream_t s, bool fused = true) {
+    const int64_t n = nz * ny * nx;
+    const bool lowp = is_lowp(precision);
+    if (lowp && K / 2 > kMaxRadiusLowp) {
+        set_error("BF16/FP16 forms support kernel radius <= " + std::to_string(kMaxRadiusLowp));
+        return EINVAL_;
+    }
     MaskBits bits;
-    if (reps > 0 && nz * ny * nx > 0) {
-        uint32_t *w = reinterpret_cast<uint32_t *>(static_cast<char *>(s0) + state_f32_bytes(nz * ny * nx));
-        MXB_HIP(timed(MXB_K_OTHER, s, [&] { return pack_bits(d_mask, nz, ny, nx, w, bits, s); }));
+    uint32_t *const w = reinterpret_cast<uint32_t *>(static_cast<char *>(s0) + state_f32_bytes(n));
+    if (reps > 0 && n > 0) bits = MaskBits{w, 1, mask_words_per_row(nx) * ny, ny};
+    const int form = precision == MXB_FP32_SPLIT && n > 0
+                         ? split_serves(nz, ny, nx, (int)(K / 2), s0, s1, bits, out_u16, out_f32, fused)
+                         : 0;
+    // the state's form at the start: 16-bit for runs that keep 16-bit state and
+    // for split runs whose first z-pass widens u0, else FP32
+    int start = lowp && reps > 1 ? precision : MXB_FP32;
+    bool inited = false;
+    if (reps > 0 && n > 0) {
+        const bool planes = form != 0 && !split_pass_supported((const uint16_t *)s0, (const uint16_t *)s1, nullptr, bits,
+                                                               geom_z(nz, ny, nx), (int)(K / 2),
+                                                               split_io_from_f16(split_lo_off(n)));
+        if (form != 0) start = MXB_FP16;
+        hipError_t e = hipErrorNotSupported;
+        if (!planes)
+            e = timed(MXB_K_OTHER, s, [&] { return launch_init_and_pack(d_mask, nz, ny, nx, s0, start, w, s); });
+        inited = e != hipErrorNotSupported;
+        if (!inited) e = timed(MXB_K_OTHER, s, [&] { return pack_bits(d_mask, nz, ny, nx, w, bits, s); });
+        MXB_HIP(e);
     }
-    if (is_lowp(precision)) {
-        if (K / 2 > kMaxRadiusLowp) {
-            set_error("BF16/FP16 forms support kernel radius <= " + std::to_string(kMaxRadiusLowp));
-            return EINVAL_;
-        }
+    if (lowp)
         return run_steps_lowp(d_mask, bits, nz, ny, nx, k, K, reps, precision == MXB_BF16, s0, s1,
-                              out_u16, out_f32, fused, s);
-    }
-    if (precision == MXB_FP32_SPLIT) {
-        const int form = split_serves(nz, ny, nx, (int)(K / 2), s0, s1, bits, out_u16, out_f32, fused);
-        if (form != 0)
-            return run_steps_split(d_mask, bits, nz, ny, nx, k, K, reps, s0, s1, false, out_u16, out_f32,
-                                   nullptr, form, s);
-    }
+                              out_u16, out_f32, fused, !inited, s);
+    if (form != 0)
+        return run_steps_split(d_mask, bits, nz, ny, nx, k, K, reps, s0, s1, false, out_u16, out_f32,
+                               nullptr, form, s, inited);
     return run_steps_f32(d_mask, bits, nz, ny, nx, k, K, reps, arith_of(precision), (float *)s0,
-                         (float *)s1, true, out_u16, out_f32, nullptr, s);
+                         (float *)s1, !inited, out_u16, out_f32, nullptr, s);
 }
 
 // RAII device buffer.

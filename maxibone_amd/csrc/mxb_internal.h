@@ -62,6 +62,12 @@ inline int64_t mask_bits_bytes(int64_t nz, int64_t ny, int64_t nx) {
 hipError_t launch_pack_mask_bits(const uint8_t *mask, int64_t nz, int64_t ny, int64_t nx, int64_t mask_row,
                                  int64_t mask_plane, uint32_t *bits, hipStream_t s);
 
+// Both of an unpadded mask's uses at the start of a diffusion, its bits and the
+// state u0 = (mask > 0) in `state`: BF16 or FP16 for those precisions, else
+// FP32.  hipErrorNotSupported: use the separate launches.
+hipError_t launch_init_and_pack(const uint8_t *mask, int64_t nz, int64_t ny, int64_t nx, void *state, int precision,
+                                uint32_t *bits, hipStream_t s);
+
 // Epilogue of the last pass of a step: illuminate from the mask, write the
 // float state and/or its uint16 quantisation.
 struct Epilogue {

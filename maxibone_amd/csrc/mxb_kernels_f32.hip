@@ -24,6 +24,7 @@
 // reference's skipped taps exactly.  The compiled tap capacity RT may exceed
 // the runtime radius R: the taps are centred and padded with zeros, which
 // again only adds exact zeros.
+#include "maxibone_diffusion.h"
 #include "mxb_internal.h"
 
 namespace mxb {
@@ -433,6 +434,85 @@ hipError_t launch_pack_mask_bits(const uint8_t *mask, int64_t nz, int64_t ny, in
     if (wpr > 65535) return hipErrorInvalidValue;
     const dim3 grid((unsigned)((ny + 255) / 256), (unsigned)wpr, (unsigned)(nz < 4096 ? nz : 4096));
     hipLaunchKernelGGL(k_pack_mask_bits, grid, dim3(256), 0, s, mask, nz, ny, nx, mask_row, mask_plane, bits);
+    return hipGetLastError();
+}
+
+// The start of a diffusion in one pass over the mask: its bits and the state
+// u0 = (mask > 0), `one` where it is set (T: the bits of a float, or of a
+// BF16 / FP16 value).  Block = 32 rows x 128 columns of a plane: a thread takes
+// the columns of one 16-byte store, at any alignment, and the rows' bits go
+// through LDS so that words leave in runs of 32 rows.
+// Bound by the stores: 1024^3 FP32 1.02 ms, 5.3 TB/s (1.40 + 0.32 as two
+// kernels); 512^3 split, a whole repetition 526 -> 454 us.
+template <typename T>
+__global__ __launch_bounds__(256) void k_init_and_pack(const uint8_t *__restrict__ m, int64_t nz, int64_t ny, int64_t nx,
+                                                       T *__restrict__ u, T one, uint32_t *__restrict__ bits) {
+    constexpr int E = 16 / sizeof(T), TPR = 128 / E, RPS = 256 / TPR;  // columns a thread, threads a row, rows a step
+    __shared__ __attribute__((aligned(4))) uint8_t sb[32][20];         // 20: rows in distinct banks
+    const int tid = threadIdx.x, c = tid % TPR;
+    const int64_t wpr = (nx + 31) / 32;
+    const int64_t x = 128 * (int64_t)blockIdx.x + E * c, y0 = 32 * (int64_t)blockIdx.y;
+    for (int64_t z = blockIdx.z; z < nz; z += gridDim.z) {
+#pragma unroll
+        for (int k = 0; k < 32 / RPS; ++k) {
+            const int r = RPS * k + tid / TPR;
+            const int64_t y = y0 + r;
+            uint32_t b = 0;
+            if (y < ny && x < nx) {
+                const int64_t at = (z * ny + y) * nx + x;
+                if (x + E <= nx) {
+                    uint32_t v[E / 4], w[4];
+                    __builtin_memcpy(v, m + at, E);
+#pragma unroll
+                    for (int e = 0; e < E / 4; ++e) b |= nonzero_bytes4(v[e]) << (4 * e);
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        if constexpr (E == 4)
+                            w[e] = (b >> e) & 1u ? one : 0u;
+                        else
+                            w[e] = ((b >> (2 * e)) & 1u ? (uint32_t)one : 0u) | ((b >> (2 * e + 1)) & 1u ? (uint32_t)one << 16 : 0u);
+                    }
+                    __builtin_memcpy(u + at, w, 16);
+                } else {
+                    for (int e = 0; e < (int)(nx - x); ++e) {
+                        const bool set = m[at + e] != 0;
+                        b |= (set ? 1u : 0u) << e;
+                        u[at + e] = set ? one : (T)0;
+                    }
+                }
+            }
+            if constexpr (E == 4) {
+                const uint32_t hi = __shfl_down(b, 1);
+                if ((c & 1) == 0) sb[r][c >> 1] = (uint8_t)(b | (hi << 4));
+            } else {
+                sb[r][c] = (uint8_t)b;
+            }
+        }
+        __syncthreads();
+        const int64_t w = 4 * (int64_t)blockIdx.x + (tid >> 5), y = y0 + (tid & 31);
+        if (tid < 128 && w < wpr && y < ny)
+            bits[(z * wpr + w) * ny + y] = *reinterpret_cast<const uint32_t *>(&sb[tid & 31][4 * (tid >> 5)]);
+        __syncthreads();
+    }
+}
+
+hipError_t launch_init_and_pack(const uint8_t *mask, int64_t nz, int64_t ny, int64_t nx, void *state, int precision,
+                                uint32_t *bits, hipStream_t s) {
+    if (nz * ny * nx == 0) return hipSuccess;
+    if ((nx + 31) / 32 > 65535) return hipErrorInvalidValue;  // as the packing alone
+    // Rows much shorter than a tile leave most of its threads idle (301x4001x5
+    // BF16 343 -> 391 us), which only small volumes, a launch's time, do not
+    // feel (24x40x72 25.6 -> 24.4).
+    if (nx < 96 && nz * ny * nx > (int64_t(1) << 18)) return hipErrorNotSupported;
+    const int64_t ty = (ny + 31) / 32;
+    if (ty > 65535) return hipErrorNotSupported;
+    const dim3 grid((unsigned)((nx + 127) / 128), (unsigned)ty, (unsigned)(nz < 4096 ? nz : 4096)), block(256);
+    if (precision == MXB_BF16 || precision == MXB_FP16)
+        hipLaunchKernelGGL(k_init_and_pack<uint16_t>, grid, block, 0, s, mask, nz, ny, nx, (uint16_t *)state,
+                           (uint16_t)(precision == MXB_BF16 ? 0x3f80 : 0x3c00), bits);
+    else
+        hipLaunchKernelGGL(k_init_and_pack<uint32_t>, grid, block, 0, s, mask, nz, ny, nx, (uint32_t *)state,
+                           0x3f800000u, bits);
     return hipGetLastError();
 }
 

@@ -138,3 +138,20 @@ def test_fused_fp32_y_and_x_in_batches(gpu, monkeypatch, prec):
         if prec == "fp32":
             one = capi.diffusion(ms[i], ks[i], 3, precision=prec, u16=True, f32=True)
             assert np.array_equal(got[0][i], one[0]) and np.array_equal(got[1][i], one[1])
+
+
+@pytest.mark.parametrize("prec", ["fp32", "fp32_exact", "bf16", "fp16", "fp32_split"])
+def test_start_from_the_mask(gpu, prec):
+    """The start of a diffusion (state and mask bits in one kernel, or two for
+    short rows of larger volumes): with a single tap of 1 the result is
+    (mask > 0) exactly, for any byte that is not zero, at the edges of a tile of
+    32 rows and 128 columns."""
+    shapes = [(2, 33, nx) for nx in (1, 7, 31, 32, 33, 95, 96, 127, 128, 129, 300)] + [(70, 80, 95), (5, 1, 640)]
+    for i, shape in enumerate(shapes):
+        print("start", prec, shape, flush=True)
+        rng = np.random.default_rng(40 + i)
+        m = (rng.integers(0, 256, shape) * (rng.random(shape) > 0.5)).astype(np.uint8)
+        for reps in (1, 3):
+            q, u = capi.diffusion(m, np.ones(1, np.float32), reps, precision=prec, u16=True, f32=True)
+            assert np.array_equal(u, (m > 0).astype(np.float32)), shape
+            assert np.array_equal(q, np.where(m > 0, np.uint16(65535), np.uint16(0))), shape
