@@ -122,6 +122,14 @@ hipError_t launch_line_pass_lowp(const uint16_t *in, uint16_t *out, const uint8_
 hipError_t launch_init_lowp(const uint8_t *mask, uint16_t *u, int64_t n, bool bf, hipStream_t s);
 hipError_t launch_lowp_to_f32(const uint16_t *u, float *f, int64_t n, bool bf, hipStream_t s);
 constexpr int kMaxRadiusLowp = 64;
+// 16-bit state in planes of py rows of px elements, the extents rounded up to
+// 8: u0, the mask and its bits in that pitch, pads zero, beside the dense bits;
+// and the true extents of a state widened, dense.
+hipError_t launch_init_and_pack_pitched(const uint8_t *mask, int64_t nz, int64_t ny, int64_t nx, int64_t py, int64_t px,
+                                        uint16_t *state, bool bf, uint32_t *bits, uint8_t *pmask, uint32_t *pbits,
+                                        hipStream_t s);
+hipError_t launch_unpitch_to_f32(const uint16_t *u, int64_t nz, int64_t ny, int64_t nx, int64_t py, int64_t px,
+                                 float *f, bool bf, hipStream_t s);
 
 // Extra operands of the split (FP32-class) form.  Its state travels as two
 // FP16 planes, u = hi + lo with hi = f16(u) and lo = f16(u - hi): the low

@@ -444,42 +444,58 @@ hipError_t launch_pack_mask_bits(const uint8_t *mask, int64_t nz, int64_t ny, in
 // through LDS so that words leave in runs of 32 rows.
 // Bound by the stores: 1024^3 FP32 1.02 ms, 5.3 TB/s (1.40 + 0.32 as two
 // kernels); 512^3 split, a whole repetition 526 -> 454 us.
-template <typename T>
+//
+// PITCH (16-bit): state in planes of py rows of px elements, multiples of 8,
+// with the mask (pm) and its bits (pbits) in the same pitch, pads zero.
+template <typename T, bool PITCH>
 __global__ __launch_bounds__(256) void k_init_and_pack(const uint8_t *__restrict__ m, int64_t nz, int64_t ny, int64_t nx,
-                                                       T *__restrict__ u, T one, uint32_t *__restrict__ bits) {
+                                                       T *__restrict__ u, T one, uint32_t *__restrict__ bits, int64_t py,
+                                                       int64_t px, uint8_t *__restrict__ pm,
+                                                       uint32_t *__restrict__ pbits) {
     constexpr int E = 16 / sizeof(T), TPR = 128 / E, RPS = 256 / TPR;  // columns a thread, threads a row, rows a step
+    static_assert(!PITCH || E == 8, "the pitched form is the 16-bit one");
     __shared__ __attribute__((aligned(4))) uint8_t sb[32][20];         // 20: rows in distinct banks
     const int tid = threadIdx.x, c = tid % TPR;
     const int64_t wpr = (nx + 31) / 32;
     const int64_t x = 128 * (int64_t)blockIdx.x + E * c, y0 = 32 * (int64_t)blockIdx.y;
+    if (!PITCH) {
+        py = ny;
+        px = nx;
+    }
     for (int64_t z = blockIdx.z; z < nz; z += gridDim.z) {
 #pragma unroll
         for (int k = 0; k < 32 / RPS; ++k) {
             const int r = RPS * k + tid / TPR;
             const int64_t y = y0 + r;
             uint32_t b = 0;
-            if (y < ny && x < nx) {
-                const int64_t at = (z * ny + y) * nx + x;
-                if (x + E <= nx) {
-                    uint32_t v[E / 4], w[4];
-                    __builtin_memcpy(v, m + at, E);
+            if (y < py && x < px) {
+                uint32_t v[E / 4] = {}, w[4];
+                if (y < ny) {
+                    const uint8_t *const src = m + (z * ny + y) * nx + x;
+                    if (x + E <= nx) {
+                        __builtin_memcpy(v, src, E);
+                    } else {
 #pragma unroll
-                    for (int e = 0; e < E / 4; ++e) b |= nonzero_bytes4(v[e]) << (4 * e);
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        if constexpr (E == 4)
-                            w[e] = (b >> e) & 1u ? one : 0u;
-                        else
-                            w[e] = ((b >> (2 * e)) & 1u ? (uint32_t)one : 0u) | ((b >> (2 * e + 1)) & 1u ? (uint32_t)one << 16 : 0u);
-                    }
-                    __builtin_memcpy(u + at, w, 16);
-                } else {
-                    for (int e = 0; e < (int)(nx - x); ++e) {
-                        const bool set = m[at + e] != 0;
-                        b |= (set ? 1u : 0u) << e;
-                        u[at + e] = set ? one : (T)0;
+                        for (int e = 0; e < E; ++e)
+                            if (x + e < nx) v[e / 4] |= (uint32_t)src[e] << (8 * (e & 3));
                     }
                 }
+#pragma unroll
+                for (int e = 0; e < E / 4; ++e) b |= nonzero_bytes4(v[e]) << (4 * e);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    if constexpr (E == 4)
+                        w[e] = (b >> e) & 1u ? one : 0u;
+                    else
+                        w[e] = ((b >> (2 * e)) & 1u ? (uint32_t)one : 0u) | ((b >> (2 * e + 1)) & 1u ? (uint32_t)one << 16 : 0u);
+                }
+                const int64_t at = (z * py + y) * px + x;
+                if (x + E <= px) {
+                    __builtin_memcpy(u + at, w, 16);
+                } else {
+                    for (int e = 0; e < (int)(px - x); ++e) u[at + e] = (b >> e) & 1u ? one : (T)0;
+                }
+                if constexpr (PITCH) *reinterpret_cast<uint2 *>(pm + at) = make_uint2(v[0], v[1]);
             }
             if constexpr (E == 4) {
                 const uint32_t hi = __shfl_down(b, 1);
@@ -490,8 +506,11 @@ __global__ __launch_bounds__(256) void k_init_and_pack(const uint8_t *__restrict
         }
         __syncthreads();
         const int64_t w = 4 * (int64_t)blockIdx.x + (tid >> 5), y = y0 + (tid & 31);
-        if (tid < 128 && w < wpr && y < ny)
-            bits[(z * wpr + w) * ny + y] = *reinterpret_cast<const uint32_t *>(&sb[tid & 31][4 * (tid >> 5)]);
+        if (tid < 128 && w < wpr) {
+            const uint32_t word = *reinterpret_cast<const uint32_t *>(&sb[tid & 31][4 * (tid >> 5)]);
+            if (y < ny) bits[(z * wpr + w) * ny + y] = word;
+            if (PITCH && y < py) pbits[(z * wpr + w) * py + y] = word;
+        }
         __syncthreads();
     }
 }
@@ -508,11 +527,20 @@ hipError_t launch_init_and_pack(const uint8_t *mask, int64_t nz, int64_t ny, int
     if (ty > 65535) return hipErrorNotSupported;
     const dim3 grid((unsigned)((nx + 127) / 128), (unsigned)ty, (unsigned)(nz < 4096 ? nz : 4096)), block(256);
     if (precision == MXB_BF16 || precision == MXB_FP16)
-        hipLaunchKernelGGL(k_init_and_pack<uint16_t>, grid, block, 0, s, mask, nz, ny, nx, (uint16_t *)state,
-                           (uint16_t)(precision == MXB_BF16 ? 0x3f80 : 0x3c00), bits);
+        hipLaunchKernelGGL((k_init_and_pack<uint16_t, false>), grid, block, 0, s, mask, nz, ny, nx, (uint16_t *)state,
+                           (uint16_t)(precision == MXB_BF16 ? 0x3f80 : 0x3c00), bits, ny, nx, nullptr, nullptr);
     else
-        hipLaunchKernelGGL(k_init_and_pack<uint32_t>, grid, block, 0, s, mask, nz, ny, nx, (uint32_t *)state,
-                           0x3f800000u, bits);
+        hipLaunchKernelGGL((k_init_and_pack<uint32_t, false>), grid, block, 0, s, mask, nz, ny, nx, (uint32_t *)state,
+                           0x3f800000u, bits, ny, nx, nullptr, nullptr);
+    return hipGetLastError();
+}
+
+hipError_t launch_init_and_pack_pitched(const uint8_t *mask, int64_t nz, int64_t ny, int64_t nx, int64_t py, int64_t px,
+                                        uint16_t *state, bool bf, uint32_t *bits, uint8_t *pmask, uint32_t *pbits,
+                                        hipStream_t s) {
+    const dim3 grid((unsigned)((px + 127) / 128), (unsigned)((py + 31) / 32), (unsigned)(nz < 4096 ? nz : 4096));
+    hipLaunchKernelGGL((k_init_and_pack<uint16_t, true>), grid, dim3(256), 0, s, mask, nz, ny, nx, state,
+                       (uint16_t)(bf ? 0x3f80 : 0x3c00), bits, py, px, pmask, pbits);
     return hipGetLastError();
 }
 

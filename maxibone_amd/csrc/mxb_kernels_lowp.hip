@@ -237,6 +237,37 @@ __global__ __launch_bounds__(256) void k_split_state(const float *__restrict__ u
     }
 }
 
+// Pitched 16-bit state (planes of py rows of px elements): FP32 values of the
+// true extents, dense.
+template <bool BF>
+__global__ __launch_bounds__(256) void k_unpitch_to_f32(const uint16_t *__restrict__ u, int64_t nz, int64_t ny,
+                                                        int64_t nx, int64_t py, int64_t px, float *__restrict__ f) {
+    const int64_t x = 4 * ((int64_t)blockIdx.x * 64 + (threadIdx.x & 63));
+    const int64_t row0 = (int64_t)blockIdx.y * 4 + (threadIdx.x >> 6);
+    if (x >= nx) return;
+    for (int64_t row = row0; row < nz * ny; row += 4 * (int64_t)gridDim.y) {
+        const int64_t z = row / ny, y = row % ny;
+        const uint2 v = *reinterpret_cast<const uint2 *>(u + (z * py + y) * px + x);  // px is a multiple of 8
+        const float r[4] = {Lowp<BF>::to_f32((uint16_t)(v.x & 0xffffu)), Lowp<BF>::to_f32((uint16_t)(v.x >> 16)),
+                            Lowp<BF>::to_f32((uint16_t)(v.y & 0xffffu)), Lowp<BF>::to_f32((uint16_t)(v.y >> 16))};
+        float *const dst = f + row * nx + x;
+        if (x + 4 <= nx) {
+            __builtin_memcpy(dst, r, 16);
+        } else {
+            for (int e = 0; e < (int)(nx - x); ++e) dst[e] = r[e];
+        }
+    }
+}
+
+hipError_t launch_unpitch_to_f32(const uint16_t *u, int64_t nz, int64_t ny, int64_t nx, int64_t py, int64_t px,
+                                 float *f, bool bf, hipStream_t s) {
+    const int64_t rows = (nz * ny + 3) / 4;
+    const dim3 grid((unsigned)((nx + 255) / 256), (unsigned)(rows < 65535 ? rows : 65535)), block(256);
+    if (bf) hipLaunchKernelGGL(k_unpitch_to_f32<true>, grid, block, 0, s, u, nz, ny, nx, py, px, f);
+    else hipLaunchKernelGGL(k_unpitch_to_f32<false>, grid, block, 0, s, u, nz, ny, nx, py, px, f);
+    return hipGetLastError();
+}
+
 // ---------------------------------------------------------------- host side
 static void plan_segments_lowp(LineGeom &g) {
     const int64_t threads = ((g.n_lane + 63) / 64) * 16 * g.n_outer;  // one wave per 16 lines

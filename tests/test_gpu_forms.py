@@ -155,3 +155,24 @@ def test_start_from_the_mask(gpu, prec):
             q, u = capi.diffusion(m, np.ones(1, np.float32), reps, precision=prec, u16=True, f32=True)
             assert np.array_equal(u, (m > 0).astype(np.float32)), shape
             assert np.array_equal(q, np.where(m > 0, np.uint16(65535), np.uint16(0))), shape
+
+
+@pytest.mark.parametrize("prec", ["bf16", "fp16"])
+@pytest.mark.parametrize("sigma", [1.0, 3.0, 10.0, 15.0])
+def test_pitched_16_bit_rows(gpu, monkeypatch, prec, sigma):
+    """16-bit repetitions on rows that are not whole 16-byte pieces run in a
+    pitched copy of the state: bit for bit the register-ring passes, at extents
+    one from a multiple of 8, of 32 and of 64, with odd and even repetitions
+    (either buffer last), and where the pitch does not fit the buffers."""
+    k = gauss_kernel(sigma).astype(np.float32)
+    for i, shape in enumerate([(20, 33, 65), (9, 64, 63), (65, 31, 127), (3, 129, 130), (40, 100, 33), (7, 9, 9),
+                               (2, 3, 1001), (30, 5, 3), (1, 257, 259)]):
+        rng = np.random.default_rng(90 + i)
+        m = (rng.integers(0, 256, shape) * (rng.random(shape) > 0.95)).astype(np.uint8)
+        for reps in (2, 3, 4):
+            print("pitched", prec, sigma, shape, reps, flush=True)
+            monkeypatch.delenv("MXB_PASS_KERNEL", raising=False)
+            got = capi.diffusion(m, k, reps, precision=prec, u16=True, f32=True)
+            monkeypatch.setenv("MXB_PASS_KERNEL", "ring")
+            want = capi.diffusion(m, k, reps, precision=prec, u16=True, f32=True)
+            assert np.array_equal(got[0], want[0]) and np.array_equal(got[1], want[1])
