@@ -424,7 +424,7 @@ def bench_edt(args):
                    "shape": list(shape), "implant_voxels": int(implant.sum(dtype=np.int64))},
         "roofline": {"bound": "hbm", "achieved": round(gbps, 1), "peak": PEAK_HBM_GBS, "unit": "GB/s",
                      "frac": round(gbps / PEAK_HBM_GBS, 4), "traffic": None,
-                     "kernel": "k_edt_pass (3 passes) + k_edt_to_u16"},
+                     "kernel": "k_edt_rows + k_edt_lines (y, z) + k_edt_to_u16"},
     }
     for b in (d_m, d_c, d_out, ws):
         b.free()
@@ -475,12 +475,14 @@ def bench_chunked(args, w, reps):
     print(json.dumps(rec), flush=True)
 
 
-def load_traffic(workload_name, precision, kernel):
+def load_traffic(workload_name, precision, kernel, form=""):
+    """Counted HBM bytes per launch; form "steps of 32 rows/": the 16-bit and
+    split forms' fused pass as it runs at radii up to 48."""
     path = os.path.join(ROOT, "profiles", "traffic.json")
     if not os.path.exists(path):
         return None
     try:
-        d = json.load(open(path)).get(f"{workload_name}/{precision}/{kernel}")
+        d = json.load(open(path)).get(f"{form}{workload_name}/{precision}/{kernel}")
         return None if d is None else d["bytes_per_launch"]
     except (ValueError, OSError):
         return None
@@ -643,7 +645,10 @@ def device_run(args, w, mask_h, k, reps, precision):
     frac_hbm = d["GBps"] / PEAK_HBM_GBS
     frac_cmp = d["TFLOPs"] / compute_peak
     # the committed counter readings are for the workload's own shape and sigma
-    traffic = None if args.shape or args.sigma else load_traffic(args.workload, precision, dom)
+    traffic = None
+    if not (args.shape or args.sigma):
+        traffic = (load_traffic(args.workload, precision, dom, "steps of 32 rows/")
+                   or load_traffic(args.workload, precision, dom))
     if frac_cmp >= frac_hbm:
         roof = {"bound": "mfma", "achieved": round(d["TFLOPs"], 3), "peak": compute_peak,
                 "unit": "TFLOP/s", "frac": round(frac_cmp, 4), "traffic": traffic}
