@@ -262,18 +262,33 @@ static void split_taps_into(const float *k, int R, int RT, bool bf, uint16_t *hi
     }
 }
 
-// Pitched-layout initialisation and final unpadding.
+// Final unpadding: 4 columns of a row per thread (a pitched row holds whole
+// pieces), stored at any alignment.  16 volumes of 64 to 384 a side: 26 -> 16 us
+// a volume, against one element and three 64-bit divisions per thread.
 __global__ __launch_bounds__(256) void k_unpad_out(const float *__restrict__ st, int64_t nz,
                                                    int64_t ny, int64_t nx, int64_t py, int64_t px,
                                                    uint16_t *__restrict__ q, float *__restrict__ f) {
-    const int64_t n = nz * ny * nx;
-    const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) {
-        const int64_t x = i % nx, zy = i / nx;
-        const int64_t y = zy % ny, z = zy / ny;
-        const float v = st[(z * py + y) * px + x];
-        if (q != nullptr) q[i] = quantise_u16_l(v);
-        if (f != nullptr) f[i] = v;
+    const int64_t x = 4 * ((int64_t)blockIdx.x * 64 + (threadIdx.x & 63));
+    if (x >= nx) return;
+    for (int64_t row = (int64_t)blockIdx.y * 4 + (threadIdx.x >> 6); row < nz * ny; row += 4 * (int64_t)gridDim.y) {
+        const int64_t z = row / ny, y = row % ny;
+        const v4f v = *reinterpret_cast<const v4f *>(st + (z * py + y) * px + x);
+        const int64_t at = row * nx + x;
+        if (x + 4 <= nx) {
+            if (q != nullptr) {
+                const uint32_t w[2] = {(uint32_t)quantise_u16_l(v[0]) | ((uint32_t)quantise_u16_l(v[1]) << 16),
+                                       (uint32_t)quantise_u16_l(v[2]) | ((uint32_t)quantise_u16_l(v[3]) << 16)};
+                __builtin_memcpy(q + at, w, 8);
+            }
+            if (f != nullptr) __builtin_memcpy(f + at, &v, 16);
+        } else {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                if (x + e >= nx) break;
+                if (q != nullptr) q[at + e] = quantise_u16_l(v[e]);
+                if (f != nullptr) f[at + e] = v[e];
+            }
+        }
     }
 }
 
@@ -290,13 +305,6 @@ __global__ __launch_bounds__(256) void k_pitch_mask(const uint8_t *__restrict__ 
     }
 }
 
-__global__ __launch_bounds__(256) void k_init_pitched(const uint8_t *__restrict__ m, float *__restrict__ u,
-                                                      int64_t n) {
-    const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride)
-        u[i] = m[i] > 0 ? 1.0f : 0.0f;
-}
-
 static unsigned blocks_for(int64_t n) {
     int64_t b = (n + 255) / 256;
     return (unsigned)(b < 1 ? 1 : (b > 16384 ? 16384 : b));
@@ -311,6 +319,13 @@ struct VolLayout {
     int R, bucket;
     int lbucket;       // 16-bit radius bucket
 };
+
+static hipError_t launch_unpad_out(const float *st, const VolLayout &L, const mxb_device_volume &V, hipStream_t s) {
+    const int64_t rows = (L.nz * L.ny + 3) / 4;
+    const dim3 grid((unsigned)((L.nx + 255) / 256), (unsigned)(rows < 65535 ? rows : 65535));
+    hipLaunchKernelGGL(k_unpad_out, grid, dim3(256), 0, s, st, L.nz, L.ny, L.nx, L.py, L.px, V.dev_out_u16, V.dev_out_f32);
+    return hipGetLastError();
+}
 
 struct TuneChoice {
     int grid = 0;
@@ -614,30 +629,19 @@ static int enqueue_persistent(mxb_batch_plan *P) {
         MXB_BHIP(launch_rep_f32(P, parity, P->tune.grid, &parity));
         for (int v = 0; v < P->n; ++v) {
             const VolLayout &L = P->lay[v];
-            const mxb_device_volume &V = P->vols[v];
-            const int64_t n = L.nz * L.ny * L.nx;
-            hipLaunchKernelGGL(k_unpad_out, dim3(blocks_for(n)), dim3(256), 0, P->stream, P->st[parity] + L.st_off,
-                               L.nz, L.ny, L.nx, L.py, L.px, V.dev_out_u16, V.dev_out_f32);
-            MXB_BHIP(hipGetLastError());
+            MXB_BHIP(launch_unpad_out(P->st[parity] + L.st_off, L, P->vols[v], P->stream));
         }
         return OK;
     }
     for (int v = 0; v < P->n; ++v) {
         const VolLayout &L = P->lay[v];
-        const int64_t n = L.nz * L.py * L.px;
-        hipLaunchKernelGGL(k_init_pitched, dim3(blocks_for(n)), dim3(256), 0, P->stream, P->masks + L.mask_off,
-                           P->st[0] + L.st_off, n);
-        MXB_BHIP(hipGetLastError());
+        MXB_BHIP(launch_init_state(P->masks + L.mask_off, P->st[0] + L.st_off, L.nz * L.py * L.px, P->stream));
     }
     int parity = 0;
     for (int64_t t = 0; t < P->reps; ++t) MXB_BHIP(launch_rep_f32(P, parity, P->tune.grid, &parity));
     for (int v = 0; v < P->n; ++v) {
         const VolLayout &L = P->lay[v];
-        const mxb_device_volume &V = P->vols[v];
-        const int64_t n = L.nz * L.ny * L.nx;
-        hipLaunchKernelGGL(k_unpad_out, dim3(blocks_for(n)), dim3(256), 0, P->stream, P->st[parity] + L.st_off,
-                           L.nz, L.ny, L.nx, L.py, L.px, V.dev_out_u16, V.dev_out_f32);
-        MXB_BHIP(hipGetLastError());
+        MXB_BHIP(launch_unpad_out(P->st[parity] + L.st_off, L, P->vols[v], P->stream));
     }
     return OK;
 }
@@ -686,9 +690,7 @@ static int autotune(mxb_batch_plan *P, int cus) {
             MXB_BHIP(launch_init_lowp(P->masks + L.mask_off, reinterpret_cast<uint16_t *>(P->st[0] + L.st_off), n,
                                       P->precision == MXB_BF16, P->stream));
         } else {
-            hipLaunchKernelGGL(k_init_pitched, dim3(blocks_for(n)), dim3(256), 0, P->stream,
-                               P->masks + L.mask_off, P->st[0] + L.st_off, n);
-            MXB_BHIP(hipGetLastError());
+            MXB_BHIP(launch_init_state(P->masks + L.mask_off, P->st[0] + L.st_off, n, P->stream));
         }
     }
     TuneChoice best;
