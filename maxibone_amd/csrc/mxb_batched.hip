@@ -918,8 +918,8 @@ int mxb_batch_run(mxb_batch_plan *P, int mode) {
         MXB_BHIP(hipGraphLaunch(P->exec, P->stream));
         return OK;
     }
-    // per-volume launches (also the form used for the other precisions), with
-    // the persistent passes' three-pass structure
+    // per-volume launches (also the form used for the other precisions), the
+    // 16-bit repetitions in the persistent passes' three-pass structure
     for (int v = 0; v < P->n; ++v) {
         const mxb_device_volume &V = P->vols[v];
         const VolLayout &L = P->lay[v];

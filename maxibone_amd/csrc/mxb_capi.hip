@@ -167,7 +167,8 @@ static hipError_t pack_bits(const uint8_t *d_mask, int64_t nz, int64_t ny, int64
 // Runs `reps` repetitions on device buffers.  If init_from_mask, state0 is
 // first set to (mask > 0); otherwise state0 already holds the FP32 state.
 // FP32 step: z: s0 -> s1, y: s1 -> s0 ((z, x, y) order), x: s0 -> s1 with
-// illumination; then the buffers swap roles.  The final x-pass writes
+// illumination; then the buffers swap roles.  Where the fused pass serves: z:
+// s0 -> s1, y and x: s1 -> s0 with illumination.  The final x-pass writes
 // out_f32 / out_u16 (when non-null); when out_f32 is null the final FP32
 // state is left in the buffer returned through *final_state (may be null).
 static int run_steps_f32(const uint8_t *d_mask, const MaskBits &bits, int64_t nz, int64_t ny,
