@@ -303,10 +303,6 @@ static int device_combine(const uint16_t *g, const uint16_t *e, int64_t nz, int6
     return OK;
 }
 
-static int64_t field_ws_bytes(int64_t nZ, int64_t nY, int64_t nX) {
-    return kFieldHistWorkspace + (nZ + nY + nX) * 4 + 256;
-}
-
 static int device_field_histogram(const uint16_t *vox, int64_t nZ, int64_t nY, int64_t nX,
                                   const uint16_t *field, int64_t nz, int64_t ny, int64_t nx,
                                   uint64_t *bins, int64_t fb, int64_t vb, double vmin, double vmax,
@@ -408,7 +404,7 @@ int mxb_combine_fields(const uint16_t *gauss, const uint16_t *edt, int64_t nz, i
 
 int64_t mxb_histogram_workspace_bytes(int64_t nZ, int64_t nY, int64_t nX) {
     if (nZ < 0 || nY < 0 || nX < 0) return -1;
-    return field_ws_bytes(nZ, nY, nX);
+    return field_workspace_bytes(nZ, nY, nX);
 }
 
 int mxb_device_field_histogram(const uint16_t *dev_voxels, int64_t nZ, int64_t nY, int64_t nX,
@@ -439,7 +435,7 @@ int mxb_field_histogram(const uint16_t *voxels, int64_t nZ, int64_t nY, int64_t 
     FBuf v, f, b, ws;
     int rc;
     if ((rc = v.alloc(n * 2)) || (rc = f.alloc(nf * 2)) || (rc = b.alloc(nb * 8)) ||
-        (rc = ws.alloc(field_ws_bytes(nZ, nY, nX))))
+        (rc = ws.alloc(field_workspace_bytes(nZ, nY, nX))))
         return rc;
     MXB_FHIP(staged_copy(v.p, voxels, n * 2, true, nullptr));
     MXB_FHIP(staged_copy(f.p, field, nf * 2, true, nullptr));

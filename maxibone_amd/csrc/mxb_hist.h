@@ -8,6 +8,8 @@
 #include <cstdint>
 #include <vector>
 
+#include "mxb_field_plan.h"
+
 namespace mxb {
 
 // bin(v) = floor(c * ((v - lo) / d)) in float64 (cpu/histograms.cc:62, :279,
@@ -80,9 +82,6 @@ __device__ __forceinline__ void load_chunk(const uint16_t *__restrict__ base, in
         for (int k = 0; k < 8; ++k) q[k] = e0 + k >= b && e0 + k < e ? base[e0 + k] : (uint16_t)0;
     }
 }
-
-// Bytes of a field histogram's workspace beside 4 per voxel coordinate of each axis.
-constexpr int64_t kFieldHistWorkspace = 2 * 65536 * 4;
 
 // Field histogram, enqueued on `s`.  `words` receives the host tables that are
 // copied to the start of `ws`: they must outlive the copy.

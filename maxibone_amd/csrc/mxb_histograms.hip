@@ -509,12 +509,8 @@ hipError_t launch_axis_histograms(const uint16_t *vox, int64_t nz, int64_t ny, i
 namespace {
 
 constexpr int kGroupThreads = 1024, kGroupWaves = kGroupThreads / 64;
-constexpr int64_t kGroupCells = 32768;   // 32-bit counters of a block's table (128 KB)
-constexpr int64_t kMaxGroups = 2048;
-constexpr int64_t kMaxBricks = 49152;    // 192 KB of ranges in the workspace
 constexpr int kQueue = 368;              // field values queued per wave
 constexpr int kList = kGroupThreads * 3 / 2; // bricks a block lists at a time
-constexpr int64_t kMaxBox = 512;         // voxels per field value
 constexpr int kGroupBlocks = 1024;       // blocks wanted at most (one fits a CU at a time; 256 leave a long tail)
 constexpr int64_t kBlockVoxels = 2048;   // and one per so many voxels: each clears and flushes its table
 
@@ -1004,36 +1000,6 @@ uint32_t least_value(const BinMap &m, int64_t b) {
 
 }  // namespace
 
-// Axis tables: the field coordinate of every voxel coordinate (z, y, x axis
-// after axis), then the first voxel coordinate of every segment, and the
-// extent.  A segment is a run of voxel coordinates with one field coordinate.
-struct AxisTables {
-    int64_t ns[3] = {0, 0, 0}, width[3] = {0, 0, 0};  // segments, the widest
-};
-
-static AxisTables axis_tables(const int64_t n[3], const int64_t nf[3], std::vector<int32_t> &words) {
-    AxisTables t;
-    words.clear();
-    for (int k = 0; k < 3; ++k) {
-        const double d = (double)nf[k] / (double)n[k];  // histograms.cc:246-249, :284-287
-        for (int64_t i = 0; i < n[k]; ++i)
-            words.push_back((int32_t)std::min<int64_t>(nf[k] - 1, (int64_t)std::floor((double)i * d)));
-    }
-    int64_t at = 0;
-    for (int k = 0; k < 3; ++k) {
-        int64_t first = 0;
-        for (int64_t i = 0; i <= n[k]; ++i) {
-            if (i != 0 && i != n[k] && words[at + i] == words[at + i - 1]) continue;
-            if (i != 0) t.width[k] = std::max(t.width[k], i - first);
-            if (i != n[k]) ++t.ns[k];
-            first = i;
-            words.push_back((int32_t)i);
-        }
-        at += n[k];
-    }
-    return t;
-}
-
 hipError_t launch_field_histogram(const uint16_t *vox, int64_t nZ, int64_t nY, int64_t nX, const uint16_t *field,
                                   int64_t nz, int64_t ny, int64_t nx, uint64_t *bins, int64_t fb, int64_t vb,
                                   double vmin, double vmax, double fmin, double fmax, void *ws,
@@ -1041,55 +1007,38 @@ hipError_t launch_field_histogram(const uint16_t *vox, int64_t nZ, int64_t nY, i
     const BinMap vm = make_bin_map(vmin, vmax, vb, true), fm = make_bin_map(fmin, fmax, fb, false);
     if (vm.vlo > vm.vhi) return hipSuccess;  // no voxel is counted
     const int64_t n[3] = {nZ, nY, nX}, nf[3] = {nz, ny, nx}, nmaps = nZ + nY + nX;
-    const AxisTables t = axis_tables(n, nf, words);
+    FieldPlan p;
+    make_field_plan(n, nf, fb, vb, vm.fast && fm.fast, p);
+    if (4 * p.table_words() > field_workspace_bytes(nZ, nY, nX)) return hipErrorInvalidValue;
+    words = std::move(p.words);
     int32_t *const d = static_cast<int32_t *>(ws);
     unsigned long long *const dst = reinterpret_cast<unsigned long long *>(bins);
-
-    // The grouped form: every field coordinate is sampled (the segments are the
-    // field's coordinates), the tables fit the workspace, a group holds at least one row
-    // of bins, and bins are monotone in the value.
+    const bool grouped = p.grouped;
+    const int64_t box = p.width[0] * p.width[1] * p.width[2], bricks = p.bricks;
     FieldGeom g{};
-    g.G = (int32_t)std::min<int64_t>(2047, std::min(fb, kGroupCells / vb));
-    const int64_t box = t.width[0] * t.width[1] * t.width[2];
-    bool grouped = g.G >= 1 && (fb + g.G - 1) / g.G <= kMaxGroups && box <= kMaxBox && vm.fast && fm.fast &&
-                   nmaps <= 40000;
-    for (int k = 0; k < 3; ++k) grouped = grouped && t.ns[k] == nf[k] && nf[k] <= 8192;  // brick numbers of 11, 10 and 11 bits
-    // bricks: 16 x 8 x 8 field values, doubled along the shortest edge (in
-    // voxels) until the table of ranges fits
-    g.lb[0] = 3; g.lb[1] = 3; g.lb[2] = 4;
-    int64_t bricks = 0;
-    while (grouped) {
-        bricks = 1;
-        for (int k = 0; k < 3; ++k) {
-            g.nb[k] = (int32_t)((nf[k] + (int64_t(1) << g.lb[k]) - 1) >> g.lb[k]);
-            bricks *= g.nb[k];
-        }
-        if (bricks <= kMaxBricks) break;
-        int best = 0;
-        for (int k = 1; k < 3; ++k)
-            if ((t.width[k] << g.lb[k]) < (t.width[best] << g.lb[best])) best = k;
-        if (++g.lb[best] > 7) grouped = false;
-    }
     if (grouped) {
+        g.G = (int32_t)p.G;
         g.bricks = (int32_t)bricks;
         g.fb = fb;
         g.vb = vb;
-        g.ng = (int32_t)((fb + g.G - 1) / g.G);
+        g.ng = (int32_t)p.ng;
         const int32_t *st = d + nmaps;
         bool even = true;
         for (int k = 0; k < 3; ++k) {
             g.n[k] = n[k];
             g.nf[k] = nf[k];
-            g.width[k] = (int32_t)t.width[k];
-            even = even && t.width[k] * nf[k] == n[k];
+            g.nb[k] = (int32_t)p.nb[k];
+            g.lb[k] = p.lb[k];
+            g.width[k] = (int32_t)p.width[k];
+            even = even && p.width[k] * nf[k] == n[k];
             g.starts[k] = st;
-            st += t.ns[k] + 1;
+            st += p.ns[k] + 1;
         }
         auto magic = [](int64_t v) { return v <= 1 ? 0u : (uint32_t)(((uint64_t(1) << 32) + v - 1) / v); };
         g.box = (uint32_t)box;
         g.m_box = magic(box);
-        g.m_xy = magic(t.width[1] * t.width[2]);
-        g.m_x = magic(t.width[2]);
+        g.m_xy = magic(p.width[1] * p.width[2]);
+        g.m_x = magic(p.width[2]);
         // testing a field value costs about 1/64 of hashing a voxel (0.7 against
         // 50 ps at 1024^3), and a value stands for `box` voxels
         g.visits_max = (uint32_t)std::min<int64_t>(0x7fffffff, 64 * box * bricks);
@@ -1101,7 +1050,7 @@ hipError_t launch_field_histogram(const uint16_t *vox, int64_t nZ, int64_t nY, i
         g.blocks_wanted = (int32_t)std::max<int64_t>(1, std::min<int64_t>(kGroupBlocks, nZ * nY * nX / kBlockVoxels));
         g.pairs = box <= 8 ? 4 : 1;
         // 32-bit offsets within a unit
-        even = even && box <= 64 && (box & (box - 1)) == 0 && 8 * t.width[0] * nY * nX < (int64_t(1) << 31);
+        even = even && box <= 64 && (box & (box - 1)) == 0 && 8 * p.width[0] * nY * nX < (int64_t(1) << 31);
         g.lbox = -1;
         for (int k = 0; even && k <= 6; ++k)
             if (box == int64_t(1) << k) g.lbox = k;

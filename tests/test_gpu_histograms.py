@@ -131,3 +131,29 @@ def test_combine_at_edges(gpu, case):
     capi.check(L.mxb_device_combine_fields(dg.ptr + shift, de.ptr + shift, *shape, None if dc is None else dc.ptr,
                                            out.ptr, ws.ptr, None))
     assert np.array_equal(out.to_array(np.uint16, shape), want)
+
+
+LONG = [  # voxel shape, field shape: tables of more words than the workspace's fixed part
+    ((1, 1, 140000), (1, 1, 140000)), ((2, 3, 200000), (2, 3, 200000)), ((150000, 2, 3), (75000, 1, 2)),
+    ((3, 131200, 1), (3, 43733, 1)),
+]
+
+
+@pytest.mark.parametrize("case", range(len(LONG)))
+def test_field_histogram_of_long_axes_stays_in_its_workspace(gpu, case):
+    vshape, fshape = LONG[case]
+    print("field histogram, long axis", LONG[case], flush=True)
+    rng = np.random.default_rng(990 + case)
+    vox = rng.integers(0, 65536, vshape, dtype=np.uint16)
+    fld = rng.integers(0, 65536, fshape, dtype=np.uint16)
+    nbins, vrange, frange = (64, 128), (1.0, 65535.0), (1.0, 65535.0)
+    want = F.field_histogram(vox, fld, np.zeros(nbins, np.uint64), vrange, frange)
+    L = capi.lib()
+    size, guard = L.mxb_histogram_workspace_bytes(*vshape), 1 << 20
+    ws = hip.DeviceBuffer.from_array(np.full(size + guard, 0xA5, np.uint8))
+    dv, df = hip.DeviceBuffer.from_array(vox), hip.DeviceBuffer.from_array(fld)
+    db = hip.DeviceBuffer.from_array(np.zeros(nbins, np.uint64))
+    capi.check(L.mxb_device_field_histogram(dv.ptr, *vshape, df.ptr, *fshape, db.ptr, *nbins, *vrange, *frange,
+                                            ws.ptr, None))
+    assert np.array_equal(db.to_array(np.uint64, nbins), want)
+    assert np.all(ws.to_array(np.uint8, (size + guard,))[size:] == 0xA5)
