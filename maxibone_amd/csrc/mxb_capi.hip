@@ -164,6 +164,12 @@ static hipError_t pack_bits(const uint8_t *d_mask, int64_t nz, int64_t ny, int64
 }
 
 // ---------------------------------------------------------------- driver
+// Whether [a, a + an) and [b, b + bn) share a byte; a null a holds none.
+static bool overlap(const void *a, int64_t an, const void *b, int64_t bn) {
+    const uintptr_t x = reinterpret_cast<uintptr_t>(a), y = reinterpret_cast<uintptr_t>(b);
+    return a != nullptr && x < y + (uintptr_t)bn && y < x + (uintptr_t)an;
+}
+
 // Runs `reps` repetitions on device buffers.  If init_from_mask, state0 is
 // first set to (mask > 0); otherwise state0 already holds the FP32 state.
 // FP32 step: z: s0 -> s1, y: s1 -> s0 ((z, x, y) order), x: s0 -> s1 with
@@ -171,6 +177,8 @@ static hipError_t pack_bits(const uint8_t *d_mask, int64_t nz, int64_t ny, int64
 // s0 -> s1, y and x: s1 -> s0 with illumination.  The final x-pass writes
 // out_f32 / out_u16 (when non-null); when out_f32 is null the final FP32
 // state is left in the buffer returned through *final_state (may be null).
+// An output may lie in the buffer that the last x-pass does not read: where
+// that is the fused pass's input, the last repetition runs its passes apart.
 static int run_steps_f32(const uint8_t *d_mask, const MaskBits &bits, int64_t nz, int64_t ny,
                          int64_t nx, const float *k, int64_t K, int64_t reps, Arith arith, float *s0,
                          float *s1, bool init_from_mask, uint16_t *out_u16, float *out_f32,
@@ -188,11 +196,12 @@ static int run_steps_f32(const uint8_t *d_mask, const MaskBits &bits, int64_t nz
     }
     const LineGeom gz = geom_z(nz, ny, nx), gy = geom_y(nz, ny, nx), gx = geom_x(nz, ny, nx);
     const bool fused = arith == Arith::MFMA && xy_fusion_enabled() && yx_f32_supported(tmp, bits, nz, ny, nx, R);
+    const bool onto_tmp = overlap(out_f32, 4 * n, tmp, 4 * n) || overlap(out_u16, 2 * n, tmp, 4 * n);
     for (int64_t t = 0; t < reps; ++t) {
         const bool last = t == reps - 1;
         const Epilogue ez{nullptr, tmp, nullptr, MaskBits{}};
         MXB_HIP(timed(MXB_K_ZPASS, s, [&] { return launch_line_pass_f32(cur, gz, ez, k, R, arith, s); }));
-        if (fused) {
+        if (fused && !(last && onto_tmp)) {
             // y then x in one pass, back into cur (or into the outputs), illuminating
             const bool unread = last && out_u16 != nullptr && final_state == nullptr;
             float *dst = last && out_f32 != nullptr ? out_f32 : (unread ? nullptr : cur);

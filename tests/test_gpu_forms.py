@@ -6,7 +6,7 @@ import numpy as np
 import pytest
 
 import oracle
-from maxibone_amd import capi
+from maxibone_amd import capi, hip
 from maxibone_amd.helpers import gauss_kernel
 
 pytestmark = pytest.mark.gpu
@@ -176,3 +176,27 @@ def test_pitched_16_bit_rows(gpu, monkeypatch, prec, sigma):
             monkeypatch.setenv("MXB_PASS_KERNEL", "ring")
             want = capi.diffusion(m, k, reps, precision=prec, u16=True, f32=True)
             assert np.array_equal(got[0], want[0]) and np.array_equal(got[1], want[1])
+
+
+@pytest.mark.parametrize("prec, shape, sigma", [("fp32", (20, 70, 64), 3.0), ("fp32", (9, 65, 67), 10.0),
+                                                ("fp32", (40, 33, 30), 15.0), ("bf16", (20, 33, 65), 3.0)])
+def test_output_in_a_state_buffer(gpu, prec, shape, sigma):
+    """The float output in the state buffer that the separate passes' last
+    x-pass does not read (the buffers swap roles each repetition, and once
+    more before the 16-bit forms' FP32 repetition) is the output of a buffer
+    of its own."""
+    n = int(np.prod(shape))
+    m = (np.random.default_rng(61).random(shape) > 0.97).astype(np.uint8)
+    k = gauss_kernel(sigma).astype(np.float32)
+    L = capi.lib()
+    dm = hip.DeviceBuffer.from_array(m)
+    size = L.mxb_state_bytes(capi.PRECISION[prec], *shape)
+    for reps in (1, 2, 3, 4):
+        print("output in a state buffer", prec, shape, sigma, reps, flush=True)
+        st, own = [hip.DeviceBuffer(size) for _ in range(2)], hip.DeviceBuffer(4 * n)
+        free = st[reps % 2] if prec == "fp32" or reps == 1 else st[1 - reps % 2]
+        for out in (own, free):
+            capi.check(L.mxb_device_diffusion(dm.ptr, *shape, k.ctypes.data, k.size, reps, capi.PRECISION[prec],
+                                              st[0].ptr, st[1].ptr, None, out.ptr, None))
+            hip.synchronize()
+        assert np.array_equal(free.to_array(np.float32, shape), own.to_array(np.float32, shape))
