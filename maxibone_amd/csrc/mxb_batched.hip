@@ -646,7 +646,7 @@ static int enqueue_persistent(mxb_batch_plan *P) {
     return OK;
 }
 
-// Time one repetition (three passes) with the current tables.
+// Time one repetition with the current tables.
 static int time_one_rep(mxb_batch_plan *P, int grid, double *ms) {
     hipEvent_t a, b;
     MXB_BHIP(hipEventCreate(&a));
@@ -810,6 +810,14 @@ int mxb_batch_create(const mxb_device_volume *vols, int n, int64_t repetitions, 
         key += "_" + std::to_string(V.nz) + "x" + std::to_string(V.ny) + "x" + std::to_string(V.nx) + "r" +
                std::to_string(L.R);
     }
+    P->fused = P->persistent && xy_fusion_enabled();
+    for (auto &L : P->lay)
+        P->fused = P->fused && L.bucket < kFusedBuckets && (L.py + 512) * L.px < (int64_t(1) << 28);
+    // A choice is timed with the passes that its plan runs: one made with the y-
+    // and x-passes apart (another setting, or a file saved before they could be
+    // one) is no choice for the fused pass, whose segments cost a halo each.
+    // 16-bit plans time their 16-bit passes, which are the same either way.
+    if (P->fused && !P->lowp) key += "_yx";
     P->key = key;
     if (n == 0) {
         *plan_out = P;
@@ -882,9 +890,6 @@ int mxb_batch_create(const mxb_device_volume *vols, int n, int64_t repetitions, 
         }
     }
     if (P->persistent) {
-        P->fused = xy_fusion_enabled();
-        for (auto &L : P->lay)
-            P->fused = P->fused && L.bucket < kFusedBuckets && (L.py + 512) * L.px < (int64_t(1) << 28);
         for (auto &L : P->lay) {
             if (P->fused) P->yx_smem_bytes = std::max(P->yx_smem_bytes, yx_smem_bytes_of(L.bucket));
             P->smem_bytes[0] = std::max(P->smem_bytes[0], smem_bytes_of<0>(L.bucket));

@@ -200,3 +200,24 @@ def test_output_in_a_state_buffer(gpu, prec, shape, sigma):
                                               st[0].ptr, st[1].ptr, None, out.ptr, None))
             hip.synchronize()
         assert np.array_equal(free.to_array(np.float32, shape), own.to_array(np.float32, shape))
+
+
+def test_batch_choice_belongs_to_its_passes(gpu, monkeypatch, tmp_path):
+    """A plan with the y- and x-passes apart does not take the grid and segment
+    that were timed for the fused pass: the file of choices holds one for each,
+    and a second plan of one kind takes the first one's."""
+    choices = tmp_path / "choices"
+    monkeypatch.setenv("MXB_TUNE_FILE", str(choices))
+    shape, k = (21, 75, 99), gauss_kernel(2.0).astype(np.float32)
+    m = hip.DeviceBuffer.from_array((np.random.default_rng(3).random(shape) > 0.9).astype(np.uint8))
+    q = hip.DeviceBuffer(2 * int(np.prod(shape)))
+    info = []
+    for fused in ("1", "0", "1", "0"):
+        monkeypatch.setenv("MXB_XY_FUSED", fused)
+        plan = capi.BatchPlan([m.ptr], [shape], [k], 2, outs_u16=[q.ptr])
+        info.append(plan.info())
+        plan.close()
+    keys = [line.split()[0] for line in choices.read_text().splitlines() if "_21x75x99r" in line]
+    print(info, keys, flush=True)
+    assert len(set(keys)) == 2
+    assert info[0] == info[2] and info[1] == info[3]
