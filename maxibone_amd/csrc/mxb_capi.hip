@@ -781,15 +781,29 @@ bool stage_ready(int dev) {
     g_stage_dev = dev;
     return true;
 }
+
+// Whether the runtime knows the memory at both ends of [p, p + bytes).
+bool known_memory(const void *p, size_t bytes) {
+    for (const char *c : {static_cast<const char *>(p), static_cast<const char *>(p) + bytes - 1}) {
+        hipPointerAttribute_t a;
+        if (hipPointerGetAttributes(&a, c) != hipSuccess) {
+            (void)hipGetLastError();
+            return false;
+        }
+        if (a.type == hipMemoryTypeUnregistered) return false;
+    }
+    return true;
+}
 }  // namespace
 
 // Host -> device (h2d) or device -> host copy of `bytes`, ordered on `s`
 // after the work already queued there; returns with the copy complete.
 hipError_t staged_copy(void *dst, const void *src, size_t bytes, bool h2d, hipStream_t s) {
     std::unique_lock<std::mutex> lk(g_stage_mu, std::defer_lock);
-    if (bytes >= kStageMin) lk.lock();
+    const bool plain = bytes < kStageMin || known_memory(h2d ? src : dst, bytes);
+    if (!plain) lk.lock();
     int dev = 0;
-    if (bytes < kStageMin || hipGetDevice(&dev) != hipSuccess || !stage_ready(dev)) {
+    if (plain || hipGetDevice(&dev) != hipSuccess || !stage_ready(dev)) {
         hipError_t e = hipMemcpyAsync(dst, src, bytes, h2d ? hipMemcpyHostToDevice : hipMemcpyDeviceToHost, s);
         return e != hipSuccess ? e : hipStreamSynchronize(s);
     }

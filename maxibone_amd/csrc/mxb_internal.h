@@ -34,7 +34,8 @@ struct LineGeom {
 };
 
 // Host <-> device copy of `bytes`, ordered on `s` after its queued work and
-// complete on return; copies of 8 MB and more go through a ring of pinned
+// complete on return; copies of 8 MB and more between the device and pageable
+// memory go through a ring of pinned
 // memory that host threads fill or drain.
 hipError_t staged_copy(void *dst, const void *src, size_t bytes, bool h2d, hipStream_t s);
 

@@ -221,3 +221,38 @@ def test_batch_choice_belongs_to_its_passes(gpu, monkeypatch, tmp_path):
     print(info, keys, flush=True)
     assert len(set(keys)) == 2
     assert info[0] == info[2] and info[1] == info[3]
+
+
+@pytest.mark.parametrize("pinned", [(True, True), (True, False), (False, True)])
+def test_host_copies_of_pinned_memory(gpu, pinned):
+    """Masks and outputs in pinned memory, from an address within the
+    allocation, and beside pageable ones: the mask's own values, as from
+    pageable memory."""
+    import ctypes
+
+    n = (33 << 20) + 5
+    H = hip.rt()
+    H.hipHostMalloc.argtypes = [ctypes.POINTER(ctypes.c_void_p), ctypes.c_size_t, ctypes.c_uint]
+    H.hipHostFree.argtypes = [ctypes.c_void_p]
+    held = []
+
+    def array(pin, dtype):
+        if not pin:
+            return np.zeros(n, dtype)
+        p, size = ctypes.c_void_p(), n * np.dtype(dtype).itemsize
+        hip.check(H.hipHostMalloc(ctypes.byref(p), size + 64, 0))
+        held.append(p)
+        a = np.frombuffer((ctypes.c_char * size).from_address(p.value + 64), dtype)
+        a[:] = 0
+        return a
+
+    print("pinned", pinned, flush=True)
+    m, q, u = array(pinned[0], np.uint8), array(pinned[1], np.uint16), array(pinned[1], np.float32)
+    m[:] = np.random.default_rng(4).random(n) > 0.5
+    k = np.ones(1, np.float32)
+    capi.check(capi.lib().mxb_diffusion_ex(m.ctypes.data, 1, 1, n, k.ctypes.data, 1, 0, 0, q.ctypes.data, u.ctypes.data, 0))
+    assert np.array_equal(u, m.astype(np.float32))
+    assert np.array_equal(q, np.where(m, np.uint16(65535), np.uint16(0)))
+    del m, q, u
+    for p in held:
+        hip.check(H.hipHostFree(p))
