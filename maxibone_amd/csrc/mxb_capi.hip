@@ -746,8 +746,11 @@ static int chunked_host(const uint8_t *mask, int64_t nz, int64_t ny, int64_t nx,
 // 640^3, staged in 64 MB chunks before, 12.6 -> 10.5 and 20.1 -> 19.2.
 // The pinned ring (64 MB) is allocated at the first large copy and kept until
 // the process ends; one staged copy runs at a time (a mutex).  Copies of fewer
-// than kStageMin bytes, where starting the threads costs more than it saves,
-// or a failed pinned allocation, take the plain path.
+// than kStageMin bytes, where starting the threads costs more than it saves, and
+// a failed pinned allocation take the plain path, and so does host memory that
+// the runtime knows: the DMA engine reads pinned memory itself, and the ring
+// would only add a memcpy (one repetition of 256^3 between pinned arrays 1.90 ->
+// 1.41 ms, of 512^3 9.8 -> 8.5; the distance transform of 256^3 3.07 -> 2.49).
 namespace {
 constexpr size_t kStagePiece = size_t(2) << 20, kStagePieces = 4;  // a thread's share; pieces per unit
 constexpr size_t kStageUnit = kStagePiece * kStagePieces;

@@ -34,9 +34,8 @@ struct LineGeom {
 };
 
 // Host <-> device copy of `bytes`, ordered on `s` after its queued work and
-// complete on return; copies of 8 MB and more between the device and pageable
-// memory go through a ring of pinned
-// memory that host threads fill or drain.
+// complete on return; copies of 8 MB and more to or from pageable memory go
+// through a ring of pinned memory that host threads fill or drain.
 hipError_t staged_copy(void *dst, const void *src, size_t bytes, bool h2d, hipStream_t s);
 
 // Axis histograms (mxb_histograms.hip), enqueued on `s`: vb <= 8192, every
