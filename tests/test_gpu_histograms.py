@@ -157,3 +157,30 @@ def test_field_histogram_of_long_axes_stays_in_its_workspace(gpu, case):
                                             ws.ptr, None))
     assert np.array_equal(db.to_array(np.uint64, nbins), want)
     assert np.all(ws.to_array(np.uint8, (size + guard,))[size:] == 0xA5)
+
+
+SLABS = [  # shape, Nr, bins, centre: slabs a few rows or columns thick, also seen from afar
+    ((3000, 1, 300), 200, 16, (0, 150)), ((9000, 2, 70), 80, 5, (1, 3)), ((700, 3, 2000), 2000, 64, (1, 1000)),
+    ((5000, 90, 1), 60, 9, (45, 0)), ((2500, 2, 2), 500, 7, (-300, 40)), ((40, 1, 3000), 4000, 300, (900, 10)),
+    ((66000, 1, 9), 12, 3, (0, 4)), ((300, 1300, 2), 700, 33, (650, 1)),
+]
+
+
+@pytest.mark.parametrize("case", range(len(SLABS)))
+def test_axis_histograms_of_thin_slabs(gpu, case):
+    """Equal voxels, so that every counter of a ring takes all of its pixels in
+    all of a block's layers, and voxels of two values."""
+    shape, Nr, vb, centre = SLABS[case]
+    for top in (1, 2):
+        print("thin slab", SLABS[case], top, flush=True)
+        vox = (np.random.default_rng(70 + case).integers(0, top, shape) * 20000 + 30000).astype(np.uint16)
+        sizes = (shape[2], shape[1], shape[0], Nr)
+        want = F.axis_histograms(vox, 0, *[np.zeros((n, vb), np.uint64) for n in sizes], centre, (1.0, 65535.0))
+        L = capi.lib()
+        dv = hip.DeviceBuffer.from_array(vox)
+        db = [hip.DeviceBuffer.from_array(np.zeros((n, vb), np.uint64)) for n in sizes]
+        ws = hip.DeviceBuffer(L.mxb_histogram_workspace_bytes(*shape))
+        capi.check(L.mxb_device_axis_histograms(dv.ptr, *shape, 0, *(b.ptr for b in db), shape[0], Nr, vb,
+                                                centre[0] % 2**64, centre[1] % 2**64, 1.0, 65535.0, ws.ptr, None))
+        for b, w, n in zip(db, want, sizes):
+            assert np.array_equal(b.to_array(np.uint64, (n, vb)), w)
