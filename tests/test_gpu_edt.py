@@ -176,3 +176,61 @@ def test_edt_many_lines(gpu, case, kind):
 
 def test_edt_many_lines_without_sites(gpu):
     assert np.all(edt.edt_sq(np.ones((260, 258, 256), bool)) == edt.EDT_NONE)
+
+
+# A lane per line along y (65536 lines) or along z (131072 lines).
+LANES = [(300, 37, 257), (9, 330, 410), (257, 9, 256)]
+
+
+@pytest.mark.parametrize("case", range(len(LANES)))
+@pytest.mark.parametrize("kind", ["noise", "some planes", "some lines", "late gap", "early gap", "just near", "columns"])
+def test_edt_of_near_sites(gpu, case, kind):
+    """Lines whose sites are near everywhere, up to the farthest distance that
+    still counts as near and one more; beside empty lines in one wave; and with
+    a gap late or early in the line.  Squares, distances and the field."""
+    shape = LANES[case]
+    nz, ny, nx = shape
+    rng = np.random.default_rng(1300 + case)
+    data = np.ones(shape, bool)
+    if kind == "noise":
+        data[rng.random(shape) < 0.4] = False
+    elif kind == "some planes":
+        data[rng.random(nz) < 0.4] = False
+    elif kind == "some lines":
+        data[np.broadcast_to(rng.random((nz, 1, nx)) < 0.3, shape)] = False
+    elif kind == "late gap":
+        data[rng.random(shape) < 0.5] = False
+        data[:, 3 * ny // 4:, nx // 3:] = True
+        data[4 * nz // 5:] = True
+    elif kind == "early gap":
+        data[rng.random(shape) < 0.5] = False
+        data[: nz // 3, : ny // 2, 5:] = True
+    elif kind == "just near":
+        data[3::9 if case % 2 else 11, ::10, ::3] = False
+    else:
+        data[:, ::9, ::2] = False
+    data.flat[rng.integers(data.size)] = False
+    _say("edt near sites", shape, kind)
+    want = E.edt_sq(data)
+    assert np.array_equal(edt.edt_sq(data).astype(np.uint64), want)
+    assert np.array_equal(edt.edt(data), E.edt(data))
+    cyl = generate_cylinder_mask(ny, nx)
+    assert np.array_equal(edt.generate_edt_field(~data, cyl), E.edt_field(~data, cyl))
+
+
+@pytest.mark.parametrize("kind", ["sparse", "rod", "planes"])
+def test_edt_lanes_along_z_distances_and_field(gpu, kind):
+    """The lane-per-line pass along z writing distances and the field."""
+    for shape in [(9, 330, 410), (33, 300, 451)]:
+        rng = np.random.default_rng(1400)
+        if kind == "rod":
+            implant = _rod_implant(shape, rng)
+        else:
+            implant = rng.random(shape) < 1e-4
+            if kind == "planes":
+                implant[:, :, shape[2] // 3] = True
+        implant.flat[rng.integers(implant.size)] = True
+        _say("edt lanes along z", shape, kind)
+        cyl = generate_cylinder_mask(shape[1], shape[2])
+        assert np.array_equal(edt.edt(~implant), E.edt(~implant))
+        assert np.array_equal(edt.generate_edt_field(implant, cyl), E.edt_field(implant, cyl))
