@@ -234,3 +234,36 @@ def test_edt_lanes_along_z_distances_and_field(gpu, kind):
         cyl = generate_cylinder_mask(shape[1], shape[2])
         assert np.array_equal(edt.edt(~implant), E.edt(~implant))
         assert np.array_equal(edt.generate_edt_field(implant, cyl), E.edt_field(implant, cyl))
+
+
+# Short lines along z that look outward: about a run of 8 and of 16, the 16 or 32
+# positions looked at one by one, several turns of a block's waves, the longest.
+SCAN_DEPTHS = [1, 7, 16, 17, 33, 48, 65, 128, 129, 150, 257, 496, 512]
+
+
+@pytest.mark.parametrize("n", SCAN_DEPTHS)
+def test_edt_scan_of_far_sites(gpu, n):
+    """Sites far from most of a line: one, a plane, two planes, a slanted
+    plane, a cone, a corner under a plane, sparse sites; ragged last block."""
+    ny, nx = 9, 71
+    z, y, x = np.ogrid[:n, :ny, :nx]
+    rng = np.random.default_rng(1500 + n)
+    masks = {
+        "one": (z == n // 3) & (y == 4) & (x == 50),
+        "plane": (z == n // 2) & (y >= 0) & (x >= 0),
+        "ends": ((z == 0) | (z == n - 1)) & (y >= 0) & (x > 30),
+        "slanted": (np.abs(x * 1.0 - z * nx / n) < 1) & (y >= 0),
+        "cone": (y - 4) ** 2 + (x - 35) ** 2 <= (0.4 * nx * z / n) ** 2,
+        "corner": ((z == 0) & (y >= 0) & (x >= 0)) | ((y == 0) & (x == 0) & (z >= 0)),
+        "sparse": rng.random((n, ny, nx)) < 2e-4,
+        "late": (z >= n - 2) & (x % 5 == 0) & (y >= 0),
+    }
+    for kind, implant in masks.items():
+        implant = np.array(np.broadcast_to(implant, (n, ny, nx)))
+        implant.flat[rng.integers(implant.size)] |= kind == "sparse"
+        _say("edt scan", n, kind)
+        assert np.array_equal(edt.edt_sq(~implant).astype(np.uint64), E.edt_sq(~implant)), kind
+        if kind in ("one", "cone", "sparse"):
+            cyl = generate_cylinder_mask(ny, nx)
+            assert np.array_equal(edt.edt(~implant), E.edt(~implant)), kind
+            assert np.array_equal(edt.generate_edt_field(implant, cyl), E.edt_field(implant, cyl)), kind
