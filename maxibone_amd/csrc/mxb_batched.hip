@@ -12,11 +12,11 @@
 // line counts (px or py lines); pad lines only ever feed pad outputs (each
 // line is independent and no pass reads positions beyond the true extent),
 // so the valid region does not depend on what the pads hold.  The mask is
-// copied into the same pitch (zero pads), and a final per-volume kernel
-// writes the caller's unpadded outputs.  FP32 repetitions run the y- and the
-// x-pass as one where every volume's radius allows it (the fused body leaves
-// the columns that a row's pads would feed at zero): 16 volumes of 64 to 384 a
-// side, sigma 2 to 10, 20 repetitions 19.3 -> 15.9 ms.
+// copied into the same pitch (zero pads), and a final kernel writes the
+// caller's unpadded outputs.  FP32 repetitions run the y- and the x-pass as one
+// where every volume's radius allows it (the fused body leaves the columns that
+// a row's pads would feed at zero): 16 volumes of 64 to 384 a side, sigma 2 to
+// 10, 20 repetitions 19.3 -> 15.2 ms.
 // The whole repetition loop is captured once in a HIP graph; replays launch it.
 //
 // The grid size and the segment length are chosen by timing candidates on
@@ -262,31 +262,67 @@ static void split_taps_into(const float *k, int R, int RT, bool bf, uint16_t *hi
     }
 }
 
+// What the first and the last launch of an FP32 run need of a volume.
+struct BatchVol {
+    const uint8_t *mask;       // pitched
+    int64_t mask_bytes;        // whole rows of 32
+    int64_t st_off;            // floats
+    int64_t nz, ny, nx, py, px;
+    uint16_t *q;
+    float *f;
+    int32_t lanes;             // 2^lanes threads unpad a row, 4 columns each
+};
+
+// Both take all volumes in one launch (blockIdx.y): 64 volumes of 40x41x42, one
+// repetition, 400 -> 92 us against a launch for each, of 2 to 4 us.
+
+// The state u0 = (mask > 0), 8 elements per thread.
+__global__ __launch_bounds__(256) void k_batched_init(const BatchVol *__restrict__ vols, int n, float *__restrict__ st) {
+    for (int v = blockIdx.y; v < n; v += gridDim.y) {
+        const BatchVol V = vols[v];
+        for (int64_t g = (int64_t)blockIdx.x * 256 + threadIdx.x; g < V.mask_bytes / 8; g += (int64_t)gridDim.x * 256) {
+            const uint2 m = *reinterpret_cast<const uint2 *>(V.mask + 8 * g);
+            v4f r[2];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) r[e >> 2][e & 3] = (((e < 4 ? m.x : m.y) >> (8 * (e & 3))) & 0xffu) ? 1.0f : 0.0f;
+            v4f *const dst = reinterpret_cast<v4f *>(st + V.st_off + 8 * g);
+            dst[0] = r[0];
+            dst[1] = r[1];
+        }
+    }
+}
+
 // Final unpadding: 4 columns of a row per thread (a pitched row holds whole
 // pieces), stored at any alignment.  16 volumes of 64 to 384 a side: 26 -> 16 us
 // a volume, against one element and three 64-bit divisions per thread.
-__global__ __launch_bounds__(256) void k_unpad_out(const float *__restrict__ st, int64_t nz,
-                                                   int64_t ny, int64_t nx, int64_t py, int64_t px,
-                                                   uint16_t *__restrict__ q, float *__restrict__ f) {
-    const int64_t x = 4 * ((int64_t)blockIdx.x * 64 + (threadIdx.x & 63));
-    if (x >= nx) return;
-    for (int64_t row = (int64_t)blockIdx.y * 4 + (threadIdx.x >> 6); row < nz * ny; row += 4 * (int64_t)gridDim.y) {
-        const int64_t z = row / ny, y = row % ny;
-        const v4f v = *reinterpret_cast<const v4f *>(st + (z * py + y) * px + x);
-        const int64_t at = row * nx + x;
-        if (x + 4 <= nx) {
-            if (q != nullptr) {
-                const uint32_t w[2] = {(uint32_t)quantise_u16_l(v[0]) | ((uint32_t)quantise_u16_l(v[1]) << 16),
-                                       (uint32_t)quantise_u16_l(v[2]) | ((uint32_t)quantise_u16_l(v[3]) << 16)};
-                __builtin_memcpy(q + at, w, 8);
-            }
-            if (f != nullptr) __builtin_memcpy(f + at, &v, 16);
-        } else {
+__global__ __launch_bounds__(256) void k_batched_unpad(const BatchVol *__restrict__ vols, int n,
+                                                       const float *__restrict__ st) {
+    for (int v = blockIdx.y; v < n; v += gridDim.y) {
+        const BatchVol V = vols[v];
+        const uint32_t rows = (uint32_t)(V.nz * V.ny);  // a row takes 128 bytes: fewer than 2^32
+        const uint32_t ny = (uint32_t)V.ny, step = gridDim.x << (8 - V.lanes);
+        for (uint32_t row = (blockIdx.x << (8 - V.lanes)) + (threadIdx.x >> V.lanes); row < rows; row += step) {
+            const uint32_t z = row / ny, y = row - z * ny;
+            const float *const src = st + V.st_off + (z * V.py + y) * V.px;
+            const int64_t to = row * V.nx;
+            for (int64_t x = 4 * (int64_t)(threadIdx.x & ((1 << V.lanes) - 1)); x < V.nx; x += int64_t(4) << V.lanes) {
+                const v4f u = *reinterpret_cast<const v4f *>(src + x);
+                const int64_t at = to + x;
+                if (x + 4 <= V.nx) {
+                    if (V.q != nullptr) {
+                        const uint32_t w[2] = {(uint32_t)quantise_u16_l(u[0]) | ((uint32_t)quantise_u16_l(u[1]) << 16),
+                                               (uint32_t)quantise_u16_l(u[2]) | ((uint32_t)quantise_u16_l(u[3]) << 16)};
+                        __builtin_memcpy(V.q + at, w, 8);
+                    }
+                    if (V.f != nullptr) __builtin_memcpy(V.f + at, &u, 16);
+                } else {
 #pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                if (x + e >= nx) break;
-                if (q != nullptr) q[at + e] = quantise_u16_l(v[e]);
-                if (f != nullptr) f[at + e] = v[e];
+                    for (int e = 0; e < 4; ++e) {
+                        if (x + e >= V.nx) break;
+                        if (V.q != nullptr) V.q[at + e] = quantise_u16_l(u[e]);
+                        if (V.f != nullptr) V.f[at + e] = u[e];
+                    }
+                }
             }
         }
     }
@@ -319,13 +355,6 @@ struct VolLayout {
     int R, bucket;
     int lbucket;       // 16-bit radius bucket
 };
-
-static hipError_t launch_unpad_out(const float *st, const VolLayout &L, const mxb_device_volume &V, hipStream_t s) {
-    const int64_t rows = (L.nz * L.ny + 3) / 4;
-    const dim3 grid((unsigned)((L.nx + 255) / 256), (unsigned)(rows < 65535 ? rows : 65535));
-    hipLaunchKernelGGL(k_unpad_out, grid, dim3(256), 0, s, st, L.nz, L.ny, L.nx, L.py, L.px, V.dev_out_u16, V.dev_out_f32);
-    return hipGetLastError();
-}
 
 struct TuneChoice {
     int grid = 0;
@@ -375,6 +404,8 @@ struct mxb_batch_plan {
     uint32_t *bits = nullptr;
     float *st[2] = {nullptr, nullptr};
     float *taps = nullptr;
+    mxb::BatchVol *bvols = nullptr;       // [n]
+    unsigned init_blocks = 1, unpad_blocks = 1;  // those of the largest volume
     mxb::BatchPassDesc *descs = nullptr;  // [6][n]: (parity, pass)
     mxb::BatchLowpDesc *ldescs = nullptr; // [6][n]: (parity, pass), 16-bit plans
     uint16_t *ltaps = nullptr;            // 16-bit tap table
@@ -604,6 +635,37 @@ static hipError_t launch_rep_f32(mxb_batch_plan *P, int parity, int grid, int *a
     return hipSuccess;
 }
 
+// One row of blocks per volume.
+static dim3 vol_grid(const mxb_batch_plan *P, unsigned blocks) { return dim3(blocks, (unsigned)std::min(P->n, 65535)); }
+
+static int launch_unpad(mxb_batch_plan *P, int parity) {
+    hipLaunchKernelGGL(k_batched_unpad, vol_grid(P, P->unpad_blocks), dim3(256), 0, P->stream, P->bvols, P->n,
+                       P->st[parity]);
+    MXB_BHIP(hipGetLastError());
+    return OK;
+}
+
+// The volumes' table for the first and the last launch.
+static int build_volumes(mxb_batch_plan *P) {
+    std::vector<BatchVol> t;
+    int64_t init = 1, unpad = 1;
+    for (int v = 0; v < P->n; ++v) {
+        const VolLayout &L = P->lay[v];
+        int lanes = 0;
+        while (lanes < 6 && (int64_t(4) << lanes) < L.nx) ++lanes;
+        const int64_t n = L.nz * L.py * L.px;
+        t.push_back(BatchVol{P->masks + L.mask_off, n, L.st_off, L.nz, L.ny, L.nx, L.py, L.px, P->vols[v].dev_out_u16,
+                             P->vols[v].dev_out_f32, lanes});
+        init = std::max(init, (n / 8 + 255) / 256);
+        unpad = std::max(unpad, (L.nz * L.ny + (256 >> lanes) - 1) >> (8 - lanes));
+    }
+    P->init_blocks = (unsigned)std::min<int64_t>(init, 65536);
+    P->unpad_blocks = (unsigned)std::min<int64_t>(unpad, 65536);
+    MXB_BHIP(hipMemcpyAsync(P->bvols, t.data(), t.size() * sizeof(BatchVol), hipMemcpyHostToDevice, P->stream));
+    MXB_BHIP(hipStreamSynchronize(P->stream));
+    return OK;
+}
+
 // Enqueue the whole persistent-form diffusion on P->stream.
 static int enqueue_persistent(mxb_batch_plan *P) {
     if (P->lowp && P->reps > 1) {
@@ -627,23 +689,13 @@ static int enqueue_persistent(mxb_batch_plan *P) {
         }
         parity ^= 1;
         MXB_BHIP(launch_rep_f32(P, parity, P->tune.grid, &parity));
-        for (int v = 0; v < P->n; ++v) {
-            const VolLayout &L = P->lay[v];
-            MXB_BHIP(launch_unpad_out(P->st[parity] + L.st_off, L, P->vols[v], P->stream));
-        }
-        return OK;
+        return launch_unpad(P, parity);
     }
-    for (int v = 0; v < P->n; ++v) {
-        const VolLayout &L = P->lay[v];
-        MXB_BHIP(launch_init_state(P->masks + L.mask_off, P->st[0] + L.st_off, L.nz * L.py * L.px, P->stream));
-    }
+    hipLaunchKernelGGL(k_batched_init, vol_grid(P, P->init_blocks), dim3(256), 0, P->stream, P->bvols, P->n, P->st[0]);
+    MXB_BHIP(hipGetLastError());
     int parity = 0;
     for (int64_t t = 0; t < P->reps; ++t) MXB_BHIP(launch_rep_f32(P, parity, P->tune.grid, &parity));
-    for (int v = 0; v < P->n; ++v) {
-        const VolLayout &L = P->lay[v];
-        MXB_BHIP(launch_unpad_out(P->st[parity] + L.st_off, L, P->vols[v], P->stream));
-    }
-    return OK;
+    return launch_unpad(P, parity);
 }
 
 // Time one repetition with the current tables.
@@ -843,6 +895,7 @@ int mxb_batch_create(const mxb_device_volume *vols, int n, int64_t repetitions, 
     const size_t o_s0 = carve((size_t)st_total * 4);
     const size_t o_s1 = carve((size_t)st_total * 4);
     const size_t o_taps = carve((size_t)taps_cap * 4);
+    const size_t o_vols = carve((size_t)n * sizeof(BatchVol));
     const size_t o_desc = carve(6 * (size_t)n * sizeof(BatchPassDesc));
     const size_t o_ldesc = carve(P->lowp ? 6 * (size_t)n * sizeof(BatchLowpDesc) : 0);
     const size_t o_ltaps = carve(P->lowp ? (size_t)(4 * 65 * (int64_t)n + 16) * sizeof(uint16_t) : 0);
@@ -859,6 +912,7 @@ int mxb_batch_create(const mxb_device_volume *vols, int n, int64_t repetitions, 
     P->st[0] = (float *)(base + o_s0);
     P->st[1] = (float *)(base + o_s1);
     P->taps = (float *)(base + o_taps);
+    P->bvols = (BatchVol *)(base + o_vols);
     P->descs = (BatchPassDesc *)(base + o_desc);
     if (P->lowp) {
         P->ldescs = (BatchLowpDesc *)(base + o_ldesc);
@@ -906,6 +960,7 @@ int mxb_batch_create(const mxb_device_volume *vols, int n, int64_t repetitions, 
             hipDeviceProp_t prop;
             if (hipGetDeviceProperties(&prop, dev) == hipSuccess) cus = prop.multiProcessorCount;
         }
+        if ((rc = build_volumes(P)) != OK) return fail(rc);
         if ((rc = autotune(P, cus)) != OK) return fail(rc);
         if ((rc = capture_graph(P)) != OK) return fail(rc);
     }
