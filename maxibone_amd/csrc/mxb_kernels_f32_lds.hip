@@ -118,7 +118,12 @@ static hipError_t launch_lds_rt(const float *in, LineGeom g, const Epilogue &e, 
     const TapsF<2 * RT + 1> t = centred_taps_l<RT>(k, R);
     if (!force_vgpr_staging()) {
         if (const int form = f32_dma_form(in, g, e, false)) return launch_f32_dma_rt<RT, false>(form, in, g, e, t, s);
-        if (const int form = f32_dma_form(in, g, e, true)) return launch_f32_dma_rt<RT, true>(form, in, g, e, t, s);
+        // lines too short for the loads to matter take the VGPR-staged form where
+        // their rows allow it (y-pass of 1000x4x600 sigma 16 122 -> 73 us, ten
+        // passes of 400x44x404 2 to 8 % faster; 400x76x404 2 to 14 % slower)
+        const bool staged = rows_aligned(in, g) && g.n_ax < 64;
+        if (const int form = staged ? 0 : f32_dma_form(in, g, e, true))
+            return launch_f32_dma_rt<RT, true>(form, in, g, e, t, s);
     }
     if (!rows_aligned(in, g)) return hipErrorNotSupported;
     hipLaunchKernelGGL((k_line_mfma_lds<RT>), dim3((unsigned)blocks), dim3(256), 0, s, in, g, e, t);

@@ -256,3 +256,27 @@ def test_host_copies_of_pinned_memory(gpu, pinned):
     del m, q, u
     for p in held:
         hip.check(H.hipHostFree(p))
+
+
+THIN = [(130, 4, 60), (60, 12, 100), (33, 20, 64), (20, 60, 36), (9, 76, 68), (100, 24, 40), (300, 4, 96)]
+
+
+@pytest.mark.parametrize("fused", ["1", "0"])
+@pytest.mark.parametrize("sigma", [1.0, 4.0, 12.0, 16.0])
+def test_thin_volumes_and_separate_passes(gpu, monkeypatch, fused, sigma):
+    """Rows of whole 16-byte pieces in thin volumes, whose y lines are shorter or
+    longer than 64 positions and leave tiles of 64 rows and rounds of blocks
+    part empty, and rows of any alignment, with the y- and x-passes fused and
+    apart: bit for bit the register-ring passes, each set of outputs."""
+    k = gauss_kernel(sigma).astype(np.float32)
+    for i, shape in enumerate(THIN + SHAPES):
+        print("thin", shape, sigma, fused, flush=True)
+        m = (np.random.default_rng(700 + i).random(shape) > 0.97).astype(np.uint8)
+        for out in ({"u16": True, "f32": True}, {"u16": True, "f32": False}, {"u16": False, "f32": True}):
+            monkeypatch.delenv("MXB_PASS_KERNEL", raising=False)
+            monkeypatch.setenv("MXB_XY_FUSED", fused)
+            got = capi.diffusion(m, k, 2, precision="fp32", **out)
+            monkeypatch.setenv("MXB_PASS_KERNEL", "ring")
+            want = capi.diffusion(m, k, 2, precision="fp32", **out)
+            for a, b in zip(got, want):
+                assert (a is None) == (b is None) and (a is None or np.array_equal(a, b))
