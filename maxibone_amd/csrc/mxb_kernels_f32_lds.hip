@@ -1,5 +1,7 @@
 // FP32 line pass, LDS-staged forms: single-volume kernels and launcher (the
 // per-block bodies live in mxb_lds_body.h and mxb_f32_dma_body.h).
+#include <algorithm>
+
 #include "mxb_f32_dma_body.h"
 
 namespace mxb {
@@ -94,12 +96,17 @@ static hipError_t launch_lds_rt(const float *in, LineGeom g, const Epilogue &e, 
     int64_t nseg = groups > 0 ? (target + groups - 1) / groups : 1;
     const int64_t q = e.mask != nullptr ? 32 : 16;  // the illuminating pass: whole mask-bit words
     // Segments of at least 64 positions, whose halo costs little; where single
-    // tiles leave fewer than four blocks a CU a pass is its blocks' own
-    // latency, and the shortest segments win (64^3, sigma 3 / 10, ten
-    // repetitions: 140 -> 125 / 176 -> 130 us, 96^3 sigma 3 186 -> 176; at
-    // 128^3, four blocks a CU, 244 -> 246).
-    const int64_t max_tiles = (g.n_ax + q - 1) / q;
-    const int64_t max_seg = groups * max_tiles < 256 * 4 ? max_tiles : (g.n_ax + 63) / 64;
+    // tiles leave fewer than four blocks a CU, and no more than its LDS holds at
+    // once, a pass is its blocks' own latency, and the shortest segments win
+    // (64^3, sigma 3 / 10, ten repetitions: 140 -> 125 / 176 -> 130 us, 96^3
+    // sigma 3 186 -> 176; at 128^3, four blocks a CU, 244 -> 246; 100x24x300
+    // sigma 16, four blocks a CU of which two fit, 195 -> 237).
+    constexpr int D = MXB_F32_DMA_DEPTH;
+    const int bytes = e.mask != nullptr ? F32DmaForm<RT, D, true, false>::BYTES
+                      : g.out_lane == 1 ? F32DmaForm<RT, D, false, true>::BYTES
+                                        : F32DmaForm<RT, D, false, false>::BYTES;
+    const int64_t max_tiles = (g.n_ax + q - 1) / q, at_once = 256 * std::min(4, 160 * 1024 / bytes);
+    const int64_t max_seg = groups * max_tiles < at_once ? max_tiles : (g.n_ax + 63) / 64;
     if (nseg > max_seg) nseg = max_seg;
     if (nseg < 1) nseg = 1;
     int64_t seg = (g.n_ax + nseg - 1) / nseg;
