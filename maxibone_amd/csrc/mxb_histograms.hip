@@ -516,7 +516,10 @@ hipError_t launch_axis_histograms(const uint16_t *vox, int64_t nz, int64_t ny, i
 //                   G x vb table, which reaches the bins once.
 // 1024^3 voxels, 512^3 field, 2048 x 4096 bins: 52.5 -> 4.8 ms; with a 1024^3
 // field 53.5 -> 15.7 (tests of field values against about ten groups each);
-// 240^3 with a 60^3 field 0.71 -> 0.15.  Bound by the latency of the scattered
+// 240^3 with a 60^3 field 0.71 -> 0.15.  Extents that do not divide (boxes of
+// two or three voxels a side): 301x257x263 and half, smooth field 0.43, noise 1.10
+// (the hash form 1.37); with a place of the widest box per lane, and bricks
+// weighed by it, 0.87 and 2.65.  Bound by the latency of the scattered
 // reads (cache lines of a steep field are fetched by several groups' blocks)
 // with 16 waves per CU, which the table allows.
 // A field that is not smooth (noise) makes every brick meet every group; then,
@@ -538,7 +541,8 @@ struct FieldGeom {
     int32_t blocks_wanted;
     int32_t pairs;         // layer pairs per unit of work: 4, or 1 where a value stands for many voxels
     int64_t fb, vb;
-    uint32_t box, m_box, m_xy, m_x;  // voxels per value and magic reciprocals
+    uint32_t box, mean;              // voxels per value, at most and on average
+    uint32_t m_y, m_xy, m_x;         // magic reciprocals of widths
     const int32_t *starts[3];        // first voxel coordinate of every segment, and the extent
     uint32_t *ranges;                // per brick: least << 16 | greatest nonzero value
     uint32_t *start;                 // per group: first block; [ng]: blocks, [ng + 1]: brick visits
@@ -614,7 +618,7 @@ __global__ __launch_bounds__(kGroupThreads) void k_field_plan(FieldGeom g) {
         int a = last_at(lo), b = last_at(hi);
         a = a < 0 ? 0 : a;
         // a visit tests all of the brick's values and counts its share of their voxels
-        const int cost = 4 + 12 * (int)g.box / (b - a + 1);
+        const int cost = 4 + 12 * (int)g.mean / (b - a + 1);
         atomicAdd(&diff[a], cost);
         atomicAdd(&diff[b + 1], -cost);
         met += b - a + 1;
@@ -738,33 +742,46 @@ __global__ __launch_bounds__(kGroupThreads) void k_field_groups(const uint16_t *
             return;
         }
         wave_lds_sync();
-        const uint32_t items = (uint32_t)n * g.box;
-        constexpr int kU = 4;
+        // a lane takes one row of a value's box, neighbouring values' rows first
+        const uint32_t un = (uint32_t)n, m_n = un == 1 ? 0 : 0xffffffffu / un + 1;  // magic reciprocal of n
+        const uint32_t items = un * (uint32_t)(g.width[0] * g.width[1]);
+        constexpr int kU = 2, kX = 4;
         for (uint32_t i0 = lane; i0 < items; i0 += 64 * kU) {
-            uint32_t v[kU], row[kU];
+            uint32_t row[kU];
+            const uint16_t *p[kU];
+            int len[kU], longest = 0;
 #pragma unroll
             for (int u = 0; u < kU; ++u) {
                 const uint32_t i = i0 + 64 * u;
-                v[u] = 0;
                 row[u] = 0;
+                p[u] = vox;
+                len[u] = 0;
                 if (i < items) {
-                    const uint32_t e = div_magic(i, g.m_box), w = i - e * g.box;
-                    const uint32_t dz = div_magic(w, g.m_xy), w2 = w - dz * (uint32_t)(g.width[1] * g.width[2]);
-                    const uint32_t dy = div_magic(w2, g.m_x), dx = w2 - dy * (uint32_t)g.width[2];
-                    const uint32_t q = queue[e];
+                    const uint32_t w = div_magic(i, m_n), q = queue[i - w * un];
+                    const uint32_t dz = div_magic(w, g.m_y), dy = w - dz * (uint32_t)g.width[1];
                     const int sz = (int)(q >> 7 & 7), sy = (int)(q >> 4 & 7), sx = (int)(q & 15);
-                    const int z = starts[26 + sz] + (int)dz, y = starts[17 + sy] + (int)dy, x = starts[sx] + (int)dx;
-                    const bool in = z < starts[27 + sz] && y < starts[18 + sy] && x < starts[sx + 1];
-                    if (in) {
-                        v[u] = vox[((int64_t)z * g.n[1] + y) * g.n[2] + x];
+                    const int z = starts[26 + sz] + (int)dz, y = starts[17 + sy] + (int)dy, x = starts[sx];
+                    if (z < starts[27 + sz] && y < starts[18 + sy]) {
+                        p[u] = vox + ((int64_t)z * g.n[1] + y) * g.n[2] + x;
+                        len[u] = starts[sx + 1] - x;
                         row[u] = (q >> 10) * (uint32_t)g.vb;
                     }
                 }
+                longest = max(longest, len[u]);
             }
+            for (int x = 0; x < longest; x += kX) {
+                uint32_t v[kU][kX];
 #pragma unroll
-            for (int u = 0; u < kU; ++u) {
-                const int bin = bin_of<true>(v[u], vm);  // 0 has no bin
-                if (bin >= 0) atomicAdd(&tab[row[u] + (uint32_t)bin], 1u);
+                for (int u = 0; u < kU; ++u)
+#pragma unroll
+                    for (int k = 0; k < kX; ++k) v[u][k] = x + k < len[u] ? p[u][x + k] : 0u;
+#pragma unroll
+                for (int u = 0; u < kU; ++u)
+#pragma unroll
+                    for (int k = 0; k < kX; ++k) {
+                        const int bin = bin_of<true>(v[u][k], vm);  // 0 has no bin
+                        if (bin >= 0) atomicAdd(&tab[row[u] + (uint32_t)bin], 1u);
+                    }
             }
         }
         wave_lds_sync();
@@ -1051,19 +1068,21 @@ hipError_t launch_field_histogram(const uint16_t *vox, int64_t nZ, int64_t nY, i
         }
         auto magic = [](int64_t v) { return v <= 1 ? 0u : (uint32_t)(((uint64_t(1) << 32) + v - 1) / v); };
         g.box = (uint32_t)box;
-        g.m_box = magic(box);
+        const int64_t values = nz * ny * nx, mean = std::max<int64_t>(1, (nZ * nY * nX + values / 2) / values);
+        g.mean = (uint32_t)mean;
+        g.m_y = magic(p.width[1]);
         g.m_xy = magic(p.width[1] * p.width[2]);
         g.m_x = magic(p.width[2]);
         // testing a field value costs about 1/64 of hashing a voxel (0.7 against
-        // 50 ps at 1024^3), and a value stands for `box` voxels
-        g.visits_max = (uint32_t)std::min<int64_t>(0x7fffffff, 64 * box * bricks);
+        // 50 ps at 1024^3), and a value stands for `mean` voxels
+        g.visits_max = (uint32_t)std::min<int64_t>(0x7fffffff, 64 * mean * bricks);
         g.bound = reinterpret_cast<const uint32_t *>(d) + words.size();
         for (int i = 0; i <= g.ng; ++i)
             words.push_back((int32_t)least_value(fm, i < g.ng ? (int64_t)i * g.G : fb));
         g.start = reinterpret_cast<uint32_t *>(d) + words.size();
         g.ranges = g.start + g.ng + 2;
         g.blocks_wanted = (int32_t)std::max<int64_t>(1, std::min<int64_t>(kGroupBlocks, nZ * nY * nX / kBlockVoxels));
-        g.pairs = box <= 8 ? 4 : 1;
+        g.pairs = mean <= 8 ? 4 : 1;
         // 32-bit offsets within a unit
         even = even && box <= 64 && (box & (box - 1)) == 0 && 8 * p.width[0] * nY * nX < (int64_t(1) << 31);
         g.lbox = -1;

@@ -184,3 +184,31 @@ def test_axis_histograms_of_thin_slabs(gpu, case):
                                                 centre[0] % 2**64, centre[1] % 2**64, 1.0, 65535.0, ws.ptr, None))
         for b, w, n in zip(db, want, sizes):
             assert np.array_equal(b.to_array(np.uint64, (n, vb)), w)
+
+
+MANY = [  # voxel shape, field shape, bins, noisy field
+    ((150, 150, 130), (150, 150, 130), (2048, 4096), False),  # several thousand bricks
+    ((232, 232, 240), (232, 232, 240), (400, 4096), True),    # a block's list of bricks fills more than once
+    ((8000, 400, 1), (8000, 400, 1), (300, 512), False),      # bricks enlarged to fit their table
+    ((40, 45, 70), (9, 11, 8), (64, 4096), False),            # uneven boxes of up to 5 x 5 x 9
+    ((61, 77, 83), (30, 38, 41), (2048, 4096), True),         # of 2 or 3 a side
+    ((61, 77, 83), (20, 51, 82), (2048, 256), False),         # of 3 or 4, 1 or 2, and 1 or 2
+]
+
+
+@pytest.mark.parametrize("case", range(len(MANY)))
+def test_field_histogram_of_many_bricks_and_uneven_boxes(gpu, case):
+    vshape, fshape, nbins, noisy = MANY[case]
+    print("field histogram", MANY[case], flush=True)
+    rng = np.random.default_rng(1050 + case)
+    vox = np.clip(rng.normal(30000, 9000, vshape), 0, 65535).astype(np.uint16)
+    fld = rng.integers(0, 65536, fshape, dtype=np.uint16) if noisy else _smooth(fshape)
+    vrange = frange = (1.0, 65535.0)
+    want = F.field_histogram(vox, fld, np.zeros(nbins, np.uint64), vrange, frange)
+    L = capi.lib()
+    dv, df = hip.DeviceBuffer.from_array(vox), hip.DeviceBuffer.from_array(fld)
+    db = hip.DeviceBuffer.from_array(np.zeros(nbins, np.uint64))
+    ws = hip.DeviceBuffer(L.mxb_histogram_workspace_bytes(*vshape))
+    capi.check(L.mxb_device_field_histogram(dv.ptr, *vshape, df.ptr, *fshape, db.ptr, *nbins, *vrange, *frange,
+                                            ws.ptr, None))
+    assert np.array_equal(db.to_array(np.uint64, nbins), want)
