@@ -32,9 +32,11 @@ struct BinMap {
 // otherwise every nonzero value with a bin in range is (the field axis).
 BinMap make_bin_map(double lo, double hi, int64_t nbins, bool mask_range);
 
-// The bin of v, or -1.
+// The bin of v, or kNoBin (bin counts multiply to less than 2^32 - 1, so a bin
+// may be 2^31 or more).
+constexpr uint32_t kNoBin = 0xffffffffu;
 template <bool FAST>
-__device__ __forceinline__ int bin_of(uint32_t v, const BinMap &m) {
+__device__ __forceinline__ uint32_t bin_of(uint32_t v, const BinMap &m) {
 #pragma clang fp contract(off)
     const double x = (double)v - m.lo;
     double q;
@@ -47,7 +49,7 @@ __device__ __forceinline__ int bin_of(uint32_t v, const BinMap &m) {
     const double t = m.c * q;
     // t < c + 1 and t >= 0 exactly when floor(t) is a bin (false for NaN)
     const bool ok = v - m.vlo <= m.vhi - m.vlo && t >= 0.0 && t < m.c + 1.0;
-    return ok ? (int)t : -1;
+    return ok ? (uint32_t)t : kNoBin;
 }
 
 // Float32 division of many values by one: the correctly rounded quotient from

@@ -110,8 +110,8 @@ __global__ __launch_bounds__(kLineThreads) void k_axis_lines(Vol v, LineSet s, B
             load_chunk(v.base, c, b, e, q);
 #pragma unroll
             for (int k = 0; k < 8; ++k) {
-                const int bin = bin_of<FAST>(q[k], m);
-                if (bin >= 0) atomicAdd(&hist[bin], 1u);
+                const uint32_t bin = bin_of<FAST>(q[k], m);
+                if (bin != kNoBin) atomicAdd(&hist[bin], 1u);
             }
         }
     }
@@ -201,8 +201,8 @@ __global__ __launch_bounds__(kTableThreads) void k_axis_cols(const uint16_t *__r
                 const uint32_t w[4] = {w4.x, w4.y, w4.z, w4.w};
 #pragma unroll
                 for (int j = 0; j < 8; ++j) {
-                    const int bin = bin_of<FAST>((w[j >> 1] >> (16 * (j & 1))) & 0xffffu, m);
-                    if (bin >= 0) count_in<WIDE>(tab, (uint32_t)((col + j) * vb + bin));
+                    const uint32_t bin = bin_of<FAST>((w[j >> 1] >> (16 * (j & 1))) & 0xffffu, m);
+                    if (bin != kNoBin) count_in<WIDE>(tab, (uint32_t)((col + j) * vb + bin));
                 }
             };
             for (; q + 3 * step < q1; q += 4 * step) {
@@ -225,8 +225,8 @@ __global__ __launch_bounds__(kTableThreads) void k_axis_cols(const uint16_t *__r
                 for (int u = 0; u < 8; ++u) w[u] = q + u * step < q1 ? p[(q + u * step) * s.nx] : (uint16_t)0;
 #pragma unroll
                 for (int u = 0; u < 8; ++u) {
-                    const int bin = bin_of<FAST>(w[u], m);  // 0 has no bin
-                    if (bin >= 0) count_in<WIDE>(tab, (uint32_t)(col * vb + bin));
+                    const uint32_t bin = bin_of<FAST>(w[u], m);  // 0 has no bin
+                    if (bin != kNoBin) count_in<WIDE>(tab, (uint32_t)(col * vb + bin));
                 }
             }
         }
@@ -332,8 +332,8 @@ __global__ __launch_bounds__(kTableThreads) void k_axis_rings(const uint16_t *__
                 for (int u = 0; u < kU; ++u) w[u] = z + u < nzb ? px[(z + u) * plane] : (uint16_t)0;
 #pragma unroll
                 for (int u = 0; u < kU; ++u) {
-                    const int bin = bin_of<FAST>(w[u], m);  // 0 has no bin
-                    if (bin >= 0) count_in<WIDE>(tab, row + (uint32_t)bin);
+                    const uint32_t bin = bin_of<FAST>(w[u], m);  // 0 has no bin
+                    if (bin != kNoBin) count_in<WIDE>(tab, row + (uint32_t)bin);
                 }
             }
         };
@@ -726,7 +726,7 @@ __global__ __launch_bounds__(kGroupThreads) void k_field_groups(const uint16_t *
             }
 #pragma unroll
             for (int u = 0; u < kU; ++u) {
-                const int bin = bin_of<true>(v[u], vm);  // 0 has no bin
+                const int bin = (int)bin_of<true>(v[u], vm);  // at most 32768 of them; 0 has none
                 if (bin >= 0) atomicAdd(&tab[row[u] + (uint32_t)bin], 1u);
             }
         };
@@ -779,7 +779,7 @@ __global__ __launch_bounds__(kGroupThreads) void k_field_groups(const uint16_t *
                 for (int u = 0; u < kU; ++u)
 #pragma unroll
                     for (int k = 0; k < kX; ++k) {
-                        const int bin = bin_of<true>(v[u][k], vm);  // 0 has no bin
+                        const int bin = (int)bin_of<true>(v[u][k], vm);  // at most 32768 of them; 0 has none
                         if (bin >= 0) atomicAdd(&tab[row[u] + (uint32_t)bin], 1u);
                     }
             }
@@ -854,7 +854,7 @@ __global__ __launch_bounds__(kGroupThreads) void k_field_groups(const uint16_t *
 #pragma unroll
                 for (int k = 0; k < 4; ++k)
                     if (h >> (4 * u + k) & 1) {
-                        const int fi = bin_of<true>(f[k], fm) - f0;
+                        const int fi = (int)bin_of<true>(f[k], fm) - f0;
                         queue[at[u]++] = (uint32_t)fi << 10 | (uint32_t)(lz + 2 * u) << 7 | (uint32_t)ly << 4 | (uint32_t)(lx + k);
                     }
             }
@@ -981,11 +981,11 @@ __global__ __launch_bounds__(kHashThreads) void k_field_hash(const uint16_t *__r
 #pragma unroll
                 for (int k = 0; k < 8; ++k) {
                     if (x0 + k >= a.nX) break;
-                    const int32_t vi = bin_of<FAST>(v[k], vm);
-                    if (vi < 0) continue;
-                    const int32_t fi = bin_of<FAST>(frow[a.xmap[x0 + k]], fm);
-                    if (fi < 0) continue;
-                    const uint32_t key = (uint32_t)fi * (uint32_t)a.vb + (uint32_t)vi;
+                    const uint32_t vi = bin_of<FAST>(v[k], vm);
+                    if (vi == kNoBin) continue;
+                    const uint32_t fi = bin_of<FAST>(frow[a.xmap[x0 + k]], fm);
+                    if (fi == kNoBin) continue;
+                    const uint32_t key = fi * (uint32_t)a.vb + vi;
                     uint32_t slot = (key * 2654435761u) >> kHashShift;
                     while (true) {
                         const uint32_t prev = atomicCAS(&keys[slot], kEmpty, key);

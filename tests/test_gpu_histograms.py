@@ -212,3 +212,31 @@ def test_field_histogram_of_many_bricks_and_uneven_boxes(gpu, case):
     capi.check(L.mxb_device_field_histogram(dv.ptr, *vshape, df.ptr, *fshape, db.ptr, *nbins, *vrange, *frange,
                                             ws.ptr, None))
     assert np.array_equal(db.to_array(np.uint64, nbins), want)
+
+
+def test_field_histogram_of_more_than_2_31_bins(gpu):
+    """Voxel bins from 2^31 on count where they lie (17 GB of bins, of which
+    the few that count are read back)."""
+    vb, vox = (1 << 31) + 64, np.array([[[1, 65535, 32768, 65534, 65535]]], np.uint16)
+    fld = np.full((1, 1, 5), 7, np.uint16)
+    L = capi.lib()
+    db = hip.DeviceBuffer(8 * vb)
+    db.fill_bytes(0)
+    dv, df = hip.DeviceBuffer.from_array(vox), hip.DeviceBuffer.from_array(fld)
+    ws = hip.DeviceBuffer(L.mxb_histogram_workspace_bytes(*vox.shape))
+    print("field histogram of", vb, "bins", flush=True)
+    capi.check(L.mxb_device_field_histogram(dv.ptr, *vox.shape, df.ptr, *fld.shape, db.ptr, 1, vb, 1.0, 65535.0, 1.0,
+                                            65535.0, ws.ptr, None))
+
+    def count(i):
+        one = np.empty(1, np.uint64)
+        hip.check(hip.rt().hipMemcpy(one.ctypes.data, db.ptr + 8 * i, 8, hip.D2H))
+        return int(one[0])
+
+    def bin_of(v):
+        return int(np.floor(np.float64(vb - 1) * ((np.float64(v) - 1.0) / 65534.0)))
+
+    assert bin_of(65535) == vb - 1
+    assert [count(bin_of(v)) for v in (1, 32768, 65534, 65535)] == [1, 1, 1, 2]
+    assert count((1 << 31) - 1) == 0
+    db.free()
