@@ -89,3 +89,46 @@ def test_rings_hold_at_most_seven_pixels_per_radius():
         r = np.floor(np.sqrt((x * x + y * y).astype(np.float64))).astype(np.int64)
         count += np.bincount(r[r <= R], minlength=R + 1) * (1 if y == 0 else 2)
     assert (count <= 7 * (np.arange(R + 1) + 1)).all()
+
+
+def _quick_quotient(x, d):
+    """x / d as the kernels divide by a shared divisor: the rounded reciprocal,
+    a product and one residual, each rounded to float32 (the fused products
+    formed in 64-bit significands)."""
+    r = np.float32(1.0) / d
+    q = x * r
+    e = (x.astype(np.float64) - q.astype(np.float64) * np.float64(d)).astype(np.float32)  # exact in FP64
+    return (e.astype(np.longdouble) * np.longdouble(r) + q.astype(np.longdouble)).astype(np.float32)
+
+
+def test_float32_division_by_a_shared_divisor():
+    """Every dividend significand against divisors about the ends of their
+    binade, fractions and maxima of fields; and whole numbers below 2^16 against
+    whole ones, as the field combination divides."""
+    x = np.arange(1 << 23, 1 << 24, dtype=np.uint32).astype(np.float32)
+    for d in (1.0, 3.0, 0.7, 65535.0, np.float32(2.0) - np.float32(2.0 ** -22), np.float32(1.0) + np.float32(2.0 ** -23)):
+        d = np.float32(d)
+        assert np.array_equal(_quick_quotient(x, d), x / d), d
+    whole = np.arange(0, 65536, dtype=np.float32)
+    rng = np.random.default_rng(5)
+    for d in np.concatenate([[1, 2, 3, 32767, 32768, 65534, 65535], rng.integers(4, 65534, 100)]):
+        assert np.array_equal(_quick_quotient(whole, np.float32(d)), whole / np.float32(d)), d
+
+
+def test_square_root_from_the_reciprocal_root():
+    """The distance transform's square root of a whole number (one residual on
+    x times the reciprocal square root) is the rounded one for reciprocal roots
+    anywhere within one unit in the last place, the instruction's bound: all
+    numbers up to 2^20, and samples up to the largest squared distance."""
+    rng = np.random.default_rng(6)
+    top = 3 * 4095 ** 2
+    n = np.concatenate([np.arange(1, 1 << 20), rng.integers(1 << 20, top, 1_500_000), np.arange(top - 1000, top + 1),
+                        np.arange(1, 4096) ** 2, np.arange(2, 4096) ** 2 - 1, np.arange(1, 4096) ** 2 + 1])
+    x = n.astype(np.float32)  # the kernel's conversion rounds above 2^24
+    want = np.sqrt(x)
+    mid = (1.0 / np.sqrt(x.astype(np.float64))).astype(np.float32)
+    for y in (mid, np.nextafter(mid, np.float32(0)), np.nextafter(mid, np.float32(2))):
+        g = x * y
+        r = (x.astype(np.float64) - g.astype(np.float64) ** 2).astype(np.float32)  # exact in FP64
+        got = (r.astype(np.longdouble) * (np.float32(0.5) * y).astype(np.longdouble) + g.astype(np.longdouble))
+        assert np.array_equal(got.astype(np.float32), want)
