@@ -71,8 +71,10 @@ __device__ __forceinline__ void fold_minmax(uint32_t lo, uint32_t hi, uint32_t *
 }
 
 // The correctly rounded square root of a whole number below 2^26 (as float32):
-// the reciprocal square root and one residual, equal to sqrtf for every such
-// value (all of them compared), in a third of its instructions.
+// the reciprocal square root and one residual, in a third of sqrtf's
+// instructions.  Equal to sqrtf for every such value if the instruction returns
+// the rounded reciprocal root; if it returns a neighbour, which is its bound, for
+// all but seven, and for those it does not.
 __device__ __forceinline__ float root(uint32_t d2) {
     const float x = (float)d2, y = __builtin_amdgcn_rsqf(x);
     const float g = x * y;

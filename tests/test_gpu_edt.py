@@ -267,3 +267,18 @@ def test_edt_scan_of_far_sites(gpu, n):
             cyl = generate_cylinder_mask(ny, nx)
             assert np.array_equal(edt.edt(~implant), E.edt(~implant)), kind
             assert np.array_equal(edt.generate_edt_field(implant, cyl), E.edt_field(implant, cyl)), kind
+
+
+# Offsets from a corner whose squared distance has a float32 root that depends on
+# the last bit of the reciprocal root: of all up to 2^24, those four.
+@pytest.mark.parametrize("far", [(12, 74, 2873), (1, 520, 3629), (1, 565, 3745), (1, 2508, 3057)])
+def test_edt_root_where_the_reciprocal_decides(gpu, far):
+    """8259749, 13440042, 14344251 and 15635314: distances to one corner site."""
+    _say("edt root", far)
+    data = np.ones(tuple(f + 1 for f in far), dtype=bool)
+    data[0, 0, 0] = False
+    z, y, x = np.ogrid[:data.shape[0], :data.shape[1], :data.shape[2]]
+    want = np.sqrt((z * z + y * y + x * x).astype(np.float32))
+    got = edt.edt(data)
+    assert got[far] == want[far]
+    assert np.array_equal(got, want)

@@ -6,7 +6,10 @@ one rounding of the exact a * scale - hi (an FMA) equals the two-step form
 fp16(fp32(a * scale) - hi); (2) a BF16 value widened to FP16 is exact from
 2^-14 (FP16's smallest normal number) up, and within 2^-25 below.
 """
+import subprocess
+
 import numpy as np
+import pytest
 
 
 def _split_two_step(a, scale):
@@ -118,7 +121,7 @@ def test_float32_division_by_a_shared_divisor():
 def test_square_root_from_the_reciprocal_root():
     """The distance transform's square root of a whole number (one residual on
     x times the reciprocal square root) is the rounded one for reciprocal roots
-    anywhere within one unit in the last place, the instruction's bound: all
+    one unit in the last place to either side, the instruction's bound: all
     numbers up to 2^20, and samples up to the largest squared distance."""
     rng = np.random.default_rng(6)
     top = 3 * 4095 ** 2
@@ -132,3 +135,52 @@ def test_square_root_from_the_reciprocal_root():
         r = (x.astype(np.float64) - g.astype(np.float64) ** 2).astype(np.float32)  # exact in FP64
         got = (r.astype(np.longdouble) * (np.float32(0.5) * y).astype(np.longdouble) + g.astype(np.longdouble))
         assert np.array_equal(got.astype(np.float32), want)
+
+
+EVERY_VALUE = r"""
+#include <cmath>
+#include <cstdio>
+int main() {
+    static float top[65536];
+    for (int i = 0; i < 65536; ++i) top[i] = (float)i;
+    long long bad = 0;
+    for (int i = 1; i < 65536; ++i) {  // combine: x / d of 16-bit whole numbers
+        const float d = (float)i, r = 1.0f / d;
+        int wrong = 0;
+        for (int j = 0; j < 65536; ++j) {
+            const float x = top[j], q = x * r;
+            wrong += __builtin_fmaf(__builtin_fmaf(-q, d, x), r, q) != x / d;
+        }
+        bad += wrong;
+    }
+    std::printf("%lld\n", bad);
+    for (int n = 1; n <= 3 * 4095 * 4095; ++n) {  // the distance transform's root
+        const float x = (float)n, mid = (float)(1.0 / std::sqrt((double)x)), want = std::sqrt(x);
+        for (int ulp = -1; ulp <= 1; ++ulp) {
+            const float y = ulp == 0 ? mid : std::nextafter(mid, ulp < 0 ? 0.0f : 2.0f), g = x * y;
+            if (__builtin_fmaf(__builtin_fmaf(-g, g, x), 0.5f * y, g) != want) std::printf("%d:%d\n", n, ulp);
+        }
+    }
+}
+"""
+
+
+DECIDED_BY_SEED = {8259749: [1], 13440042: [-1], 14344251: [-1], 15635314: [-1, 1], 33038995: [1], 33038996: [1],
+                   33038997: [1]}
+
+
+def test_every_whole_quotient_and_root(tmp_path):
+    """All quotients of 16-bit whole numbers, and all roots up to the largest
+    squared distance.  With the rounded reciprocal root every root is the rounded
+    one; with a neighbour of it, as the instruction may return, all but those of
+    DECIDED_BY_SEED, which the GPU tests compare (the last three are 4 times the
+    first and its neighbours that round to the same float32)."""
+    with open("/proc/cpuinfo") as f:
+        if " fma " not in f.read():
+            pytest.skip("no fused multiply-add on this CPU: too slow in software")
+    src, exe = tmp_path / "every.cpp", tmp_path / "every"
+    src.write_text(EVERY_VALUE)
+    subprocess.run(["g++", "-std=c++17", "-O3", "-mavx2", "-mfma", "-ffp-contract=off", "-fno-math-errno", str(src),
+                    "-o", str(exe)], check=True)
+    out = subprocess.run([str(exe)], stdout=subprocess.PIPE, text=True, check=True).stdout.split()
+    assert out == ["0"] + [f"{n}:{ulp}" for n, ulps in DECIDED_BY_SEED.items() for ulp in ulps]
