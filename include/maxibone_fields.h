@@ -65,10 +65,11 @@ int mxb_axis_histograms(const uint16_t *voxels, int64_t nz, int64_t ny, int64_t 
                         uint64_t cx, double vmin, double vmax, int verbose);
 
 /* Device forms of the histograms: all pointers in HBM, enqueued on `stream`
- * (the bins are added to); each call returns after synchronising `stream`
- * (its lookup tables are staged from host memory).  The workspace holds the bin lookup tables and
- * coordinate maps; mxb_histogram_workspace_bytes gives its size for the
- * larger of the two uses with these extents. */
+ * (the bins are added to); each call returns after synchronising `stream`.
+ * mxb_histogram_workspace_bytes gives the workspace of the field form for
+ * these voxel extents: its coordinate maps, copied from host memory, and the
+ * tables its kernels divide the work by.  The axis form asks for a workspace
+ * that is not NULL, and does not use it. */
 int64_t mxb_histogram_workspace_bytes(int64_t nZ, int64_t nY, int64_t nX);
 int mxb_device_field_histogram(const uint16_t *dev_voxels, int64_t nZ, int64_t nY, int64_t nX,
                                const uint16_t *dev_field, int64_t nz, int64_t ny, int64_t nx,

@@ -16,7 +16,7 @@
 // caller's unpadded outputs.  FP32 repetitions run the y- and the x-pass as one
 // where every volume's radius allows it (the fused body leaves the columns that
 // a row's pads would feed at zero): 16 volumes of 64 to 384 a side, sigma 2 to
-// 10, 20 repetitions 19.3 -> 15.2 ms.
+// 10, 20 repetitions 19.3 -> 15.1 ms.
 // The whole repetition loop is captured once in a HIP graph; replays launch it.
 //
 // The grid size and the segment length are chosen by timing candidates on

@@ -307,8 +307,8 @@ static int run_lowp_core(const uint8_t *d_mask, const MaskBits &bits, int64_t nz
 // mask and its bits sit behind the second state's 16-bit half; where they do
 // not fit (extents of a few voxels, mostly pads) the unpitched passes run,
 // whose register-ring kernel moves 32-byte pieces of unaligned rows.  BF16,
-// sigma 4, ten repetitions: 257x331x403 2.90 -> 1.37 ms, 100x90x110 278 -> 205
-// us; 700x701x702 sigma 6, four repetitions 15.4 -> 5.6 ms.
+// sigma 4, ten repetitions: 257x331x403 2.90 -> 1.34 ms, 100x90x110 278 -> 204
+// us; 700x701x702 sigma 6, four repetitions 15.4 -> 5.3 ms.
 struct PitchedLowp {
     int64_t py, px, mask_at, bits_at, end;  // byte offsets in the second state
 };

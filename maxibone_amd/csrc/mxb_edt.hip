@@ -527,9 +527,11 @@ __global__ __launch_bounds__(256) void k_edt_rows(const uint8_t *__restrict__ da
 //   Z: input uint32 squared distances; entries hold position << gbits | value
 //      and are stored over the input (entry m <= positions read so far).
 // The turn test is done in float64, where products below 2^39 are exact.
-// 1024^3 implant field: y 10.1 -> 2.05 ms, z 14.8 -> 4.0 ms against one wave
+// 1024^3 implant field: y 10.1 -> 1.98 ms, z 14.8 -> 3.73 ms against one wave
 // per line (k_edt_pass: 7100 instructions per 1024-voxel line and one min/max
-// atomic per block); about 125 instructions per 64 voxels, half the VALU rate.
+// atomic per block).  z is bound by its vector instructions, 113 per 64 voxels
+// (93 % of the SIMDs' cycles); y, 35 per 64 voxels and 55 %, by its serial loads
+// beside them.
 struct EdtLines {
     const void *in;
     void *stack;
@@ -1131,11 +1133,12 @@ int device_edt_core(const uint8_t *data, int64_t nz, int64_t ny, int64_t nx, boo
     }
     // A lane per line needs lines enough for the device, and is bound by the
     // latency of its serial steps below that (129x300x257: along y, 33 K lines,
-    // 140 us against 95 for k_edt_pass; 400x333x417, 139 K lines along z, 920
-    // us for the whole field against 1458 scanning outward).  Along z, where
+    // 140 us against 95 for k_edt_pass; 400x333x417, 139 K lines along z, 793
+    // us for the whole field against 1044 scanning outward and 1316 for
+    // k_edt_pass).  Along z, where
     // after the y pass every plane with a site has values throughout, short
-    // lines that are not plenty scan outward (200^3: 95 us, k_edt_pass 240;
-    // 256^3: 349 us for the field, lanes 503; 500x250x250: 599, k_edt_pass 690);
+    // lines that are not plenty scan outward (whole field of 200^3: 211 us, k_edt_pass 391;
+    // 256^3: 302, lanes 454; 500x250x250: 599, k_edt_pass 733, lanes 780);
     // along y, where most values are none, scanning is no faster.
     constexpr int64_t kLinesWanted = 65536, kLinesPlenty = 131072;
     if (nz * nx >= kLinesWanted) {

@@ -30,8 +30,8 @@
 // 16-byte read serves four chunks of the x-pass; y ^ (x % 4) is stored in y's
 // place, so a y-pass result's writes fall in distinct banks.
 //
-// Bound: the FP32 matrix cores from R = 40 on (75 % busy at 512^3, R = 40: 0.52 ms
-// a launch), below that the chain of an iteration (barrier, operand reads,
+// Bound: the FP32 matrix cores from R = 40 on (busy 74 % of the cycles at 512^3, R =
+// 40: 0.52 ms a launch; 56 % at R = 12), below that the chain of an iteration (barrier, operand reads,
 // products, ring writes) beside 3.7 TB/s of memory traffic (512^3, R = 12: 0.28
 // ms).  Two blocks share a CU up to R = 40 and three up to R = 16, which hides
 // more than a second or third group in flight would (256^3, sigma 5: 805 us

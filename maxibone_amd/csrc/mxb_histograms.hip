@@ -81,8 +81,9 @@ struct LineSet {
 // One vb-entry table per block (32 KB at most, so the wave slots fill), 16
 // bytes per lane and load.  1024^3 with 4096 bins of noisy data: 0.57-0.6 ms
 // each for y and z (3.7 TB/s); both counted along rows, with a flush of the y
-// table after every row, took 10.7 ms.  Bound by the LDS atomics (a wave's 64
-// counts take several passes over the banks) and the read together.
+// table after every row, took 10.7 ms.  Bound by its vector instructions (the
+// float64 bin of each voxel): they fill 87 % of the SIMDs' cycles, the LDS 38 %
+// of its own.
 template <bool FAST>
 __global__ __launch_bounds__(kLineThreads) void k_axis_lines(Vol v, LineSet s, BinMap m, int64_t vb,
                                                              unsigned long long *__restrict__ bins) {
@@ -177,7 +178,8 @@ struct ColSet {
 // group read the same 128-byte lines, so they go to one XCD next to each
 // other (block b runs on XCD b % 8).  VEC: 16-byte loads of 8 columns
 // (aligned rows), else one voxel per lane, 2 NT contiguous bytes per row.
-// 1024^3, 4096 bins: 0.87 ms (2.5 TB/s).
+// 1024^3, 4096 bins: 0.87 ms (2.5 TB/s), 69 % of the SIMDs' cycles in vector
+// instructions.
 template <bool FAST, bool WIDE, bool VEC>
 __global__ __launch_bounds__(kTableThreads) void k_axis_cols(const uint16_t *__restrict__ vox, ColSet s, BinMap m,
                                                              int64_t vb, unsigned long long *__restrict__ bins) {
@@ -257,7 +259,10 @@ constexpr int kU = 4;  // layers whose loads a lane issues together (1024^3: 4 3
 // block.  A pixel's radius is so worked out once per block, no lane idles on
 // short runs, and the layers' loads are independent.  1024^3, 4096 bins: 1.9
 // ms; with x, one global atomic per voxel and lanes grouped by equal bins, it
-// took 36.5 ms.  Where an annulus has fewer pixels than half the threads,
+// took 36.5 ms.  Three times k_axis_lines, with as many LDS atomics: a lane
+// loads 2 bytes (eight times the loads) and each count takes 2.4 times the
+// vector instructions (58 % of the SIMDs' cycles), while a wave waits 62 % of
+// its time.  Where an annulus has fewer pixels than half the threads,
 // lanes share a pixel's layers (4096x1x4096, 4096 bins, the whole call: 567 ->
 // 211 us).
 template <bool FAST, bool WIDE>
@@ -514,14 +519,15 @@ hipError_t launch_axis_histograms(const uint16_t *vox, int64_t nz, int64_t ny, i
 //                   waves test the bricks' field values, queue the matches,
 //                   and count the queued values' voxels in the block's
 //                   G x vb table, which reaches the bins once.
-// 1024^3 voxels, 512^3 field, 2048 x 4096 bins: 52.5 -> 4.8 ms; with a 1024^3
-// field 53.5 -> 15.7 (tests of field values against about ten groups each);
+// 1024^3 voxels, 512^3 field, 2048 x 4096 bins, calls back to back: 52.5 ->
+// 4.8 ms (k_field_groups 4.5); with a 1024^3 field 53.5 -> 15.5 (tests of field values against about ten groups each);
 // 240^3 with a 60^3 field 0.71 -> 0.15.  Extents that do not divide (boxes of
 // two or three voxels a side): 301x257x263 and half, smooth field 0.43, noise 1.10
 // (the hash form 1.37); with a place of the widest box per lane, and bricks
-// weighed by it, 0.87 and 2.65.  Bound by the latency of the scattered
-// reads (cache lines of a steep field are fetched by several groups' blocks)
-// with 16 waves per CU, which the table allows.
+// weighed by it, 0.87 and 2.65.  Bound by vector
+// instructions (64 % of a busy SIMD's cycles: tests, bins, the queue), beside
+// scattered reads (a wave waits 47 % of its time) that only 16 waves per CU,
+// which the table allows, can hide.
 // A field that is not smooth (noise) makes every brick meet every group; then,
 // and for tables or axes beyond the limits below, k_field_hash counts.
 namespace {
