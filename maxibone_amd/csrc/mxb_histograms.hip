@@ -551,9 +551,10 @@ struct FieldGeom {
     uint32_t m_y, m_xy, m_x;         // magic reciprocals of widths
     const int32_t *starts[3];        // first voxel coordinate of every segment, and the extent
     uint32_t *ranges;                // per brick: least << 16 | greatest nonzero value
-    uint32_t *start;                 // per group: first block; [ng]: blocks, [ng + 1]: brick visits
+    uint32_t *start;                 // per group: first block; [ng]: blocks, [ng + 1]: brick visits, weighed
     const uint32_t *bound;           // per group: least field value, [ng]: end
     uint32_t visits_max;             // beyond, the hash form counts
+    uint32_t few_weight;             // of a visit, in 16ths, where voxels have one value or two
 };
 
 // i / d for i < 2^20, d <= 512 by m = ceil(2^32 / d); d = 1: m = 0
@@ -598,8 +599,20 @@ __global__ __launch_bounds__(256) void k_field_ranges(const uint16_t *__restrict
 }
 
 // Blocks per group, in proportion to its work; one block.
-__global__ __launch_bounds__(kGroupThreads) void k_field_plan(FieldGeom g) {
+//
+// It also weighs the visits against the hash form (visits_max).  Voxels of very
+// few values (a mask, a constant) stay as few pairs in a hash block's table: 11
+// ps a voxel for one value, 14 for two, 20 for four to sixteen, instead of 50, so
+// there a visit weighs more.  A sample of voxels tells how many values there
+// are; kFewPairs bounds the pairs with the field bins that a brick meets, beyond
+// which the table (8192 slots) overflows.  One value over noise, field of half
+// the extents: 512^3 4.70 -> 1.24 ms, 1024^3 37.9 -> 9.1; over a smooth field as
+// fine as the voxels, 1024^3 18.3 -> 11.2.  Four values there are faster grouped
+// (15.6 against 17.9), hence the lesser weight from three on.
+constexpr int64_t kFewPairs = 8192;
+__global__ __launch_bounds__(kGroupThreads) void k_field_plan(const uint16_t *__restrict__ vox, FieldGeom g, BinMap vm) {
     __shared__ uint32_t bound[kMaxGroups + 1];
+    __shared__ uint32_t seen[kGroupCells / 32];
     __shared__ int32_t diff[kMaxGroups + 1];
     __shared__ int32_t wsum[kGroupWaves];
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
@@ -607,7 +620,11 @@ __global__ __launch_bounds__(kGroupThreads) void k_field_plan(FieldGeom g) {
         bound[i] = g.bound[i];
         diff[i] = 0;
     }
+    for (int i = tid; i < kGroupCells / 32; i += kGroupThreads) seen[i] = 0;
     __syncthreads();
+    uint32_t sample = 0;
+    if (g.few_weight > 16)
+        sample = vox[__umul64hi((uint64_t)(tid + 1) * 0x9e3779b97f4a7c15u, (uint64_t)(g.n[0] * g.n[1] * g.n[2]))];
     auto last_at = [&](uint32_t f) {  // the last group that starts at or before f, or -1
         int lo = -1, hi = g.ng;
         while (hi - lo > 1) {
@@ -628,6 +645,10 @@ __global__ __launch_bounds__(kGroupThreads) void k_field_plan(FieldGeom g) {
         atomicAdd(&diff[a], cost);
         atomicAdd(&diff[b + 1], -cost);
         met += b - a + 1;
+    }
+    if (g.few_weight > 16) {
+        const uint32_t b = bin_of<true>(sample, vm);
+        if (b != kNoBin) atomicOr(&seen[b >> 5], 1u << (b & 31));
     }
     __syncthreads();
     // two groups per thread: inclusive scans of diff (work per group), then of
@@ -660,11 +681,15 @@ __global__ __launch_bounds__(kGroupThreads) void k_field_plan(FieldGeom g) {
     auto blocks = [&](int v) { return v == 0 ? 0 : (int)((v * want + work - 1) / work); };
     const int p0 = blocks(v0), p1 = blocks(v1);
     scan(p0, p1, before, total);
+    int values = 0, unused;
+    if (g.few_weight > 16) scan(__popc(seen[tid]), 0, unused, values);
     if (i0 < g.ng) g.start[i0] = (uint32_t)before;
     if (i1 < g.ng) g.start[i1] = (uint32_t)(before + p0);
     if (tid == 0) {
         g.start[g.ng] = (uint32_t)total;
-        g.start[g.ng + 1] = (uint32_t)visits;
+        const bool few = g.few_weight > 16 && (int64_t)values * g.G * visits <= kFewPairs * g.bricks;
+        const uint32_t w = values <= 2 ? g.few_weight : max(16u, g.few_weight * 6 / 16);
+        g.start[g.ng + 1] = few ? (uint32_t)min((uint64_t)visits * w >> 4, (uint64_t)0xffffffffu) : (uint32_t)visits;
     }
 }
 
@@ -1082,6 +1107,9 @@ hipError_t launch_field_histogram(const uint16_t *vox, int64_t nZ, int64_t nY, i
         // testing a field value costs about 1/64 of hashing a voxel (0.7 against
         // 50 ps at 1024^3), and a value stands for `mean` voxels
         g.visits_max = (uint32_t)std::min<int64_t>(0x7fffffff, 64 * mean * bricks);
+        // voxels of few values: 13 times that (k_field_plan), less in volumes that do
+        // not fill the device with hash blocks, 512 of 2^16 voxels
+        g.few_weight = (uint32_t)std::max<int64_t>(16, std::min<int64_t>(208, 208 * (nZ * nY * nX) >> 25));
         g.bound = reinterpret_cast<const uint32_t *>(d) + words.size();
         for (int i = 0; i <= g.ng; ++i)
             words.push_back((int32_t)least_value(fm, i < g.ng ? (int64_t)i * g.G : fb));
@@ -1101,7 +1129,7 @@ hipError_t launch_field_histogram(const uint16_t *vox, int64_t nZ, int64_t nY, i
         auto *fn = &k_field_groups;
         if ((e = allow_lds(fn, kGroupLds)) != hipSuccess) return e;
         hipLaunchKernelGGL(k_field_ranges, dim3((unsigned)((bricks + 3) / 4)), dim3(256), 0, s, field, g);
-        hipLaunchKernelGGL(k_field_plan, dim3(1), dim3(kGroupThreads), 0, s, g);
+        hipLaunchKernelGGL(k_field_plan, dim3(1), dim3(kGroupThreads), 0, s, vox, g, vm);
         hipLaunchKernelGGL(fn, dim3((unsigned)(g.blocks_wanted + g.ng + 7) / 8 * 8), dim3(kGroupThreads), kGroupLds, s, vox, field, g, vm, fm, dst);
     }
     HashArgs h{nZ, nY, nX, nz, ny, nx, vb, d, d + nZ, d + nZ + nY, grouped ? g.start + g.ng + 1 : nullptr, g.visits_max};

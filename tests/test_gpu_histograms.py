@@ -214,6 +214,33 @@ def test_field_histogram_of_many_bricks_and_uneven_boxes(gpu, case):
     assert np.array_equal(db.to_array(np.uint64, nbins), want)
 
 
+FEW = ["none", "one", "two", "four", "rare"]
+
+
+@pytest.mark.parametrize("noisy", [True, False])
+@pytest.mark.parametrize("kind", FEW)
+def test_field_histogram_of_voxels_of_few_values(gpu, kind, noisy):
+    """Voxels of so few values that they are hashed where others are grouped;
+    among them values in places that a sample may miss."""
+    vshape, fshape, nbins, vrange = (184, 180, 186), (92, 90, 93), (2048, 4096), (1.0, 40000.0)
+    print("field histogram of few values", kind, noisy, flush=True)
+    rng = np.random.default_rng(1070)
+    values = {"none": [0, 50000], "two": [900, 40000], "four": [0, 1, 900, 901]}.get(kind, [900])
+    vox = np.array(values, np.uint16)[rng.integers(0, len(values), vshape)]
+    if kind == "rare":
+        vox[90, 91:99] = rng.integers(0, 65536, (8, 186))
+        vox[0, 0, 0] = vox[-1, -1, -1] = 40000
+    fld = rng.integers(0, 65536, fshape, dtype=np.uint16) if noisy else _smooth(fshape)
+    want = F.field_histogram(vox, fld, np.zeros(nbins, np.uint64), vrange, (1.0, 65535.0))
+    L = capi.lib()
+    dv, df = hip.DeviceBuffer.from_array(vox), hip.DeviceBuffer.from_array(fld)
+    db = hip.DeviceBuffer.from_array(np.zeros(nbins, np.uint64))
+    ws = hip.DeviceBuffer(L.mxb_histogram_workspace_bytes(*vshape))
+    capi.check(L.mxb_device_field_histogram(dv.ptr, *vshape, df.ptr, *fshape, db.ptr, *nbins, *vrange, 1.0, 65535.0,
+                                            ws.ptr, None))
+    assert np.array_equal(db.to_array(np.uint64, nbins), want)
+
+
 def test_field_histogram_of_more_than_2_31_bins(gpu):
     """Voxel bins from 2^31 on count where they lie (17 GB of bins, of which
     the few that count are read back)."""
